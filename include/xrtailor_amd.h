@@ -129,12 +129,14 @@ typedef struct xrt_tuning {
   int32_t persistent_unroll; /* constraints per thread per round in the persistent substep:
                               * 0 default (2 stretch / 1 bend in LDS, 4 / 2 in global memory,
                               * 4 FEM), 1 light (1 / 1, 2 / 1, 2), 2 heavy (4 / 2, 8 / 4, 8) */
-  int32_t wide_per_thread;   /* stretch / bend elements per thread of the wide launches (the
-                              * batched substep with contacts): 1 (default) or 2 */
-  int32_t path;              /* 0 persistent substep, 1 wide substep (one launch per color of
-                              * every instance, each instance over as many blocks as the
-                              * color needs); contexts with contacts, particles or bindings
-                              * always take the wide substep */
+  int32_t wide_per_thread;   /* stretch / bend elements per thread of the wide substep's
+                              * constraint launches: 1 (default) or 2 (half the threads) */
+  int32_t path;              /* 0 persistent substep (one workgroup per instance), 1 wide
+                              * substep (each instance over as many workgroups as it needs;
+                              * the colors of an iteration in one launch).  xrt_start sets
+                              * the default from the instances' sizes; contexts with
+                              * contacts, particles or bindings always take the wide
+                              * substep */
   float best_ms;             /* set by xrt_autotune: ms per substep of the chosen shapes */
   float default_ms;          /* set by xrt_autotune: ms per substep of the defaults */
   int32_t candidates;        /* set by xrt_autotune: configurations timed */
@@ -388,8 +390,9 @@ int xrt_substep_plain(xrt_ctx* ctx, int32_t inst);
  * sequence) -- the plain path of the batched workload */
 int xrt_frames_plain(xrt_ctx* ctx, int32_t nframes);
 /* one substep of all instances: without contacts one persistent launch (CSR instance
- * table); with body or self contact every constraint color, LRA pass, contact phase and
- * LBVH operation of all instances in one launch each.  Results equal xrt_substep_plain's
+ * table) or the wide substep (xrt_tuning.path); with body or self contact the wide substep:
+ * the constraint colors of an iteration, each LRA pass, contact phase and LBVH operation of
+ * all instances in one launch each.  Results equal xrt_substep_plain's
  * bit for bit. */
 int xrt_substep_batched(xrt_ctx* ctx);
 /* `nframes` frames of all instances; the frame's substep launches are captured once in

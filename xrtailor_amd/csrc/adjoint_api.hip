@@ -31,7 +31,7 @@ WideArgs MakeWideArgs(xrt_ctx* c) {
   a.slam = c->slam.ptr;
   a.bidx = c->bidx.ptr;
   a.bpar = c->bpar.ptr;
-  a.x = c->x.ptr;
+  a.x = c->xcur;
   a.xw = c->x0.ptr;
   return a;
 }
@@ -263,7 +263,9 @@ int WideSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, AdjointData
   const WideConfig& W = c->wide;
   hipStream_t s = c->stream;
   const int N = W.n_total, n_inst = static_cast<int>(c->inst.size());
-  const WideArgs wa = MakeWideArgs(c);
+  c->xcur = c->x.ptr;
+  const bool sweep = c->patches.ready && !FemOn(c);
+  const bool sweep_ground = sweep && k.enable_ground && c->total_slots == 0;
   float4* T = (A && sub >= 0)
                   ? A->tape.ptr + (static_cast<size_t>(A->slot) * c->params.num_substeps + sub) *
                                       A->sub_stride
@@ -275,7 +277,7 @@ int WideSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, AdjointData
   if (T) XRT_CHECK_HIP(LaunchCopy4(s, T, c->x0.ptr, N));
   if (T && A->rep && sub == 0)  // a frame slot's response pool starts empty
     XRT_CHECK_HIP(hipMemsetAsync(A->rep_count.ptr + A->slot, 0, sizeof(unsigned long long), s));
-  XRT_CHECK_HIP(LaunchPredict(s, c->x0.ptr, c->v.ptr, c->x.ptr, N, k));
+  XRT_CHECK_HIP(LaunchPredict(s, c->x0.ptr, c->v.ptr, c->xcur, N, k));
   if ((rc = ParticleSubstepBegin(c, -1)) != XRT_OK) return rc;
   for (int it = 0; it < k.iterations; ++it) {
     float4* TI = T ? T + N + static_cast<size_t>(it) * A->it_stride : nullptr;
@@ -298,36 +300,45 @@ int WideSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, AdjointData
           return rc;
     if (FemOn(c)) {  // never taped: the adjoint refuses the FEM constraints
       if ((rc = FemIter(c, -1, it)) != XRT_OK) return rc;
+    } else if (sweep) {  // every color (and the ground plane, when it comes next) in one launch
+      if ((rc = PatchIter(c, k, bm, it, sweep_ground, TI ? TI + A->off_s : nullptr,
+                          TI ? TI + A->off_b : nullptr, TI ? TI + A->off_g : nullptr)) != XRT_OK)
+        return rc;
     } else {
+      const WideArgs wa = MakeWideArgs(c);
       for (int col = 0; col < static_cast<int>(W.s_max.size()); ++col)
         XRT_CHECK_HIP(LaunchWideStretch(s, wa, n_inst, col, W.s_max[col], k.inv_dt2, it,
                                         TI ? TI + A->off_s : nullptr, W.maps.ptr + W.s_map[col],
                                         W.s_blocks[col], c->tuning.wide_per_thread));
     }
-    if (k.solve_bending && !FemOn(c))
+    if (k.solve_bending && !FemOn(c) && !sweep) {
+      const WideArgs wa = MakeWideArgs(c);
       for (int col = 0; col < static_cast<int>(W.b_max.size()); ++col)
         XRT_CHECK_HIP(LaunchWideBend(s, wa, n_inst, col, W.b_max[col], k.inv_dt2, bm,
                                      TI ? TI + A->off_b : nullptr, W.maps.ptr + W.b_map[col],
                                      W.b_blocks[col], c->tuning.wide_per_thread));
+    }
     if (c->total_slots > 0) {
-      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_l, c->x.ptr, N));
-      XRT_CHECK_HIP(LaunchWideLra(s, c->desc.ptr, n_inst, c->max_slots, c->max_nv, c->x.ptr,
+      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_l, c->xcur, N));
+      XRT_CHECK_HIP(LaunchWideLra(s, c->desc.ptr, n_inst, c->max_slots, c->max_nv, c->xcur,
                                   c->slot_vert.ptr, c->slot_pos_all.ptr, c->lra_ptr.ptr,
                                   c->lra_slot.ptr, c->lra_rest.ptr, k.stretchiness));
     }
-    if (k.enable_ground) {
-      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_g, c->x.ptr, N));
-      XRT_CHECK_HIP(LaunchGround(s, c->x.ptr, c->x0.ptr, N, k.ground_y, k.friction));
+    if (k.enable_ground && !sweep_ground) {
+      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_g, c->xcur, N));
+      XRT_CHECK_HIP(LaunchGround(s, c->xcur, c->x0.ptr, N, k.ground_y, k.friction));
     }
     if (obs_contact) {
-      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_c, c->x.ptr, N));
+      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_c, c->xcur, N));
       if ((rc = MultiContactVfSolve(c)) != XRT_OK) return rc;
-      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_e, c->x.ptr, N));
+      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_e, c->xcur, N));
       if ((rc = MultiContactEeSolve(c)) != XRT_OK) return rc;
     }
     if ((rc = BindingIter(c, -1)) != XRT_OK) return rc;  // never taped: the adjoint refuses
   }
-  XRT_CHECK_HIP(LaunchFinalize(s, c->x0.ptr, c->v.ptr, c->x.ptr, N, k));
+  XRT_CHECK_HIP(LaunchFinalize(s, c->x0.ptr, c->v.ptr, c->xcur, N, k,
+                               c->xcur == c->x.ptr ? nullptr : c->x.ptr));
+  c->xcur = c->x.ptr;
   if ((rc = ParticleSubstepEnd(c, -1)) != XRT_OK) return rc;
   return MultiContactSubstepEnd(c);
 }
@@ -350,6 +361,7 @@ int ReverseSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, int sub)
   AdjointData& A = *c->adj;
   hipStream_t s = c->stream;
   const int N = A.n_total, n_inst = static_cast<int>(c->inst.size());
+  c->xcur = c->x.ptr;
   const WideArgs wa = MakeWideArgs(c);
   const float4* T =
       A.tape.ptr + (static_cast<size_t>(A.slot) * c->params.num_substeps + sub) * A.sub_stride;

@@ -358,6 +358,15 @@ int TimeCandidate(xrt_ctx* c, const SavedRun& r, int n, float* ms) {
   return RestoreRun(c, r);
 }
 
+// Default path (xrt_set_tuning and xrt_autotune replace it): the fused sweeps of the wide
+// substep where they spread an instance over several CUs; else the persistent kernel, which
+// is the same one workgroup per instance with one launch per substep (ms per frame,
+// persistent / sweeps: one cloth of 32 x 32 2.07 / 2.23, 64 x 64 4.08 / 2.29, 100 x 100
+// 8.16 / 2.33; 64 of 64 x 64 4.47 / 3.33; 256 of 64 x 64 4.66 / 5.64)
+int DefaultPath(const xrt_ctx* ctx) {
+  return ctx->patches.ready && ctx->patches.split && !FemOn(ctx) ? 1 : 0;
+}
+
 int CheckTuning(const xrt_tuning& t) {
   XRT_REQUIRE(t.persistent_block >= 64 && t.persistent_block <= 1024 && t.persistent_block % 64 == 0,
               XRT_ERR_INVALID_ARG, "persistent_block must be a multiple of 64 in [64, 1024]");
@@ -635,6 +644,7 @@ int xrt_set_stretch_compliance(xrt_ctx* ctx, int32_t inst, const float* complian
     XRT_CHECK_HIP(hipMemcpyAsync(ctx->sc.ptr + h.sbeg, sc.data(), sizeof(StretchC) * sc.size(),
                                  hipMemcpyHostToDevice, ctx->stream));
     XRT_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    return PatchRefreshCompliance(ctx);
   }
   return XRT_OK;
 }
@@ -827,8 +837,11 @@ int xrt_start(xrt_ctx* ctx, uint64_t seed) {
     XRT_CHECK_HIP(w.maps.Upload(maps, ctx->stream));
     XRT_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   }
-  int rc = ContactStart(ctx);
+  ctx->xcur = ctx->x.ptr;
+  int rc = PatchPrepare(ctx);
   if (rc != XRT_OK) return rc;
+  ctx->tuning.path = DefaultPath(ctx);
+  if ((rc = ContactStart(ctx)) != XRT_OK) return rc;
   if ((rc = ParticleStart(ctx)) != XRT_OK) return rc;
   if ((rc = BindingStart(ctx)) != XRT_OK) return rc;
   ctx->fem.seed = seed;
@@ -1083,6 +1096,7 @@ int xrt_autotune(xrt_ctx* ctx, int32_t substeps, xrt_tuning* out) {
   if ((rc = SaveRun(ctx, saved)) != XRT_OK) return rc;
   const bool wide = ContactsActive(ctx) || ParticlesOn(ctx) || BindingsOn(ctx);
   std::vector<xrt_tuning> cand;
+  const int default_path = wide || DefaultPath(ctx) == 1 ? 1 : 0;
   const xrt_tuning base{1024, 0, 1, wide ? 1 : 0, 0.0f, 0.0f, 0};
   if (wide) {
     for (int pt : {1, 2}) {
@@ -1113,7 +1127,9 @@ int xrt_autotune(xrt_ctx* ctx, int32_t substeps, xrt_tuning* out) {
     float ms = 0.0f;
     rc = TimeCandidate(ctx, saved, substeps, &ms);
     if (rc != XRT_OK) break;
-    if (j == 0) default_ms = ms;
+    if (cand[j].path == default_path && cand[j].persistent_block == base.persistent_block &&
+        cand[j].persistent_unroll == base.persistent_unroll && cand[j].wide_per_thread == 1)
+      default_ms = ms;
     if (j == 0 || ms < best_ms) {
       best_ms = ms;
       best = cand[j];

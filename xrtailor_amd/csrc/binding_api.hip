@@ -228,7 +228,8 @@ int BindingIter(xrt_ctx* ctx, int inst) {
   BindingData& B = ctx->binding;
   if (B.total == 0) return XRT_OK;
   const MapRef& r = inst < 0 ? B.all : B.one[inst];
-  XRT_CHECK_HIP(LaunchBindingSolve(ctx->stream, B.dev.ptr, B.items.ptr, Map(B.maps, r), ctx->x.ptr));
+  XRT_CHECK_HIP(LaunchBindingSolve(ctx->stream, B.dev.ptr, B.items.ptr, Map(B.maps, r),
+                                   inst < 0 ? ctx->xcur : ctx->x.ptr));
   return XRT_OK;
 }
 

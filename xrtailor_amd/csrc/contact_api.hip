@@ -562,18 +562,18 @@ int MultiContactIterPre(xrt_ctx* ctx, int it, bool* pass_ran, const RepTapeHook*
       if (c && c->obs_nf > 0) pass = c->pass_cnt;
     const float alpha = (static_cast<float>(pass) + 1.0f) / static_cast<float>(p.num_collision_passes);
     XRT_CHECK_HIP(MultiObstacleRefit(s, ctx->ic.ptr, ctx->maps, alpha, p.bvh_tolerance));
-    XRT_CHECK_HIP(MultiGenerate(s, ctx->ic.ptr, ctx->maps, ctx->x0.ptr, ctx->x.ptr));
+    XRT_CHECK_HIP(MultiGenerate(s, ctx->ic.ptr, ctx->maps, ctx->x0.ptr, ctx->xcur));
     for (auto& c : ctx->contact)
       if (c && c->obs_nf > 0) c->pass_cnt++;
     if (pass_ran) *pass_ran = true;
   }
   if (p.enable_self_contact) {
     if (it % interval == 0)
-      XRT_CHECK_HIP(MultiPairs(s, ctx->ic.ptr, ctx->maps, ctx->x.ptr, ctx->x0.ptr, kPairThickness));
+      XRT_CHECK_HIP(MultiPairs(s, ctx->ic.ptr, ctx->maps, ctx->xcur, ctx->x0.ptr, kPairThickness));
     if (rep_tape) {
-      XRT_CHECK_HIP(hipMemcpyAsync(rep_tape->x_out, ctx->x.ptr, sizeof(float4) * ctx->x.n,
+      XRT_CHECK_HIP(hipMemcpyAsync(rep_tape->x_out, ctx->xcur, sizeof(float4) * ctx->x.n,
                                    hipMemcpyDeviceToDevice, s));
-      XRT_CHECK_HIP(MultiRepRecord(s, ctx->ic.ptr, ctx->maps, ctx->x.ptr, ctx->x0.ptr,
+      XRT_CHECK_HIP(MultiRepRecord(s, ctx->ic.ptr, ctx->maps, ctx->xcur, ctx->x0.ptr,
                                    p.pbd_thickness, rep_tape->pool, rep_tape->count,
                                    rep_tape->cap, rep_tape->flags, rep_tape->marks,
                                    rep_tape->marks + 1));
@@ -584,7 +584,7 @@ int MultiContactIterPre(xrt_ctx* ctx, int it, bool* pass_ran, const RepTapeHook*
       e1 = ctx->rep_events[ctx->rep_next + 1];
       ctx->rep_next += 2;
     }
-    XRT_CHECK_HIP(MultiRepulsion(s, ctx->ic.ptr, ctx->maps, ctx->x.ptr, ctx->x0.ptr, p.pbd_thickness,
+    XRT_CHECK_HIP(MultiRepulsion(s, ctx->ic.ptr, ctx->maps, ctx->xcur, ctx->x0.ptr, p.pbd_thickness,
                                  p.repulsion_relaxation, e0, e1));
   }
   return XRT_OK;
@@ -592,7 +592,7 @@ int MultiContactIterPre(xrt_ctx* ctx, int it, bool* pass_ran, const RepTapeHook*
 
 int MultiContactVfSolve(xrt_ctx* ctx) {
   if (!ctx->params.enable_obstacle_contact) return XRT_OK;
-  XRT_CHECK_HIP(MultiVfSolve(ctx->stream, ctx->ic.ptr, ctx->maps, ctx->x.ptr, ctx->x0.ptr,
+  XRT_CHECK_HIP(MultiVfSolve(ctx->stream, ctx->ic.ptr, ctx->maps, ctx->xcur, ctx->x0.ptr,
                              ctx->params.contact_friction,
                              1.0f / static_cast<float>(ctx->params.num_substeps)));
   return XRT_OK;
@@ -600,7 +600,7 @@ int MultiContactVfSolve(xrt_ctx* ctx) {
 
 int MultiContactEeSolve(xrt_ctx* ctx) {
   if (!ctx->params.enable_obstacle_contact) return XRT_OK;
-  XRT_CHECK_HIP(MultiEeSolve(ctx->stream, ctx->ic.ptr, ctx->maps, ctx->x.ptr,
+  XRT_CHECK_HIP(MultiEeSolve(ctx->stream, ctx->ic.ptr, ctx->maps, ctx->xcur,
                              ctx->params.relaxation_factor));
   return XRT_OK;
 }

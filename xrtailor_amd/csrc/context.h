@@ -16,6 +16,7 @@
 #include "device.h"
 #include "fem.h"
 #include "particle.h"
+#include "patch.h"
 #include "topology.h"
 
 namespace xrt {
@@ -216,6 +217,19 @@ struct WideConfig {
   DevBuf<int32_t> maps;
 };
 
+// Fused constraint sweeps (patch.h) over every instance, built at xrt_start.
+struct PatchData {
+  bool ready = false;  // false: the colors run as launches of their own
+  bool split = false;  // some instance is cut into several patches
+  int n = 0, ns = 0, nb = 0, threads = 0;
+  size_t lds_bytes = 0;
+  DevBuf<PatchDev> patch;
+  DevBuf<int32_t> verts, off, bcon;
+  DevBuf<int4> srec, brec;
+  DevBuf<float> slam;
+  DevBuf<float4> alt;  // the second position buffer
+};
+
 // Adjoint (differentiable rollout) state: checkpoints, one frame of tape, adjoints.
 struct AdjointData {
   int n_frames = 0, ckpt_every = 1, n_passes = 0, frequency = 1;
@@ -309,6 +323,10 @@ struct xrt_ctx {
   xrt::MultiMaps maps;
   // wide (all instances per launch) launch sizes
   xrt::WideConfig wide;
+  // fused constraint sweeps; xcur holds the iterate between the launches of a substep of
+  // every instance (x, or the sweeps' second buffer; x again when the substep has ended)
+  xrt::PatchData patches;
+  float4* xcur = nullptr;
   // swift-mode particle self-collision
   xrt::ParticleData particles;
   // obstacle skinning and cloth-to-body bindings
@@ -400,6 +418,13 @@ bool FemOn(const xrt_ctx* ctx);
 FemConsts FemConstsOf(const xrt_params& p);  // at the substep dt
 int FemPrepare(xrt_ctx* ctx);
 int FemIter(xrt_ctx* ctx, int inst, int it);
+// patch_api.hip: the sweep plan of every instance (xrt_start, after the colors are uploaded),
+// one iteration's stretch and bend colors in one launch from xcur (which becomes the other
+// buffer), with the ground plane when `ground`; `it` of `iterations`; tapes as in adjoint.h
+int PatchPrepare(xrt_ctx* ctx);
+int PatchIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, int it, bool ground,
+              float4* tape_s, float4* tape_b, float4* tape_g);
+int PatchRefreshCompliance(xrt_ctx* ctx);
 // adjoint_api.hip: one substep of every instance as wide launches with the contact phases
 // above; with a tape owner and sub >= 0 the operators' inputs go to tape slot `sub`
 int WideSubstep(xrt_ctx* ctx, const StepConsts& k, const BendMode& bm, AdjointData* tape, int sub);

@@ -20,8 +20,9 @@ hipError_t LaunchLra(hipStream_t s, float4* x, const int32_t* slot_vert, float4*
                      float stretchiness);
 hipError_t LaunchGround(hipStream_t s, float4* x, const float4* x0, int n, float ground_y,
                         float mu);
+// x_out (optional): a copy of x too
 hipError_t LaunchFinalize(hipStream_t s, float4* x0, float4* v, const float4* x, int n,
-                          const StepConsts& k);
+                          const StepConsts& k, float4* x_out = nullptr);
 // unroll: 0 default, 1 light, 2 heavy (constraints per thread per round; same results)
 hipError_t LaunchBatchedSubstep(hipStream_t s, const BatchArgs& a, const StepConsts& k,
                                 int n_instances, int block, size_t lds_bytes, int unroll);

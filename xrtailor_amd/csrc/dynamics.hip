@@ -85,7 +85,8 @@ __global__ __launch_bounds__(256) void GroundKernel(float4* __restrict__ x,
 __global__ __launch_bounds__(256) void FinalizeKernel(float4* __restrict__ x0,
                                                       float4* __restrict__ v,
                                                       const float4* __restrict__ x, int n,
-                                                      float inv_dt, float damp_factor) {
+                                                      float inv_dt, float damp_factor,
+                                                      float4* __restrict__ x_out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float4 p = x[i];
@@ -93,6 +94,7 @@ __global__ __launch_bounds__(256) void FinalizeKernel(float4* __restrict__ x0,
   v[i] = make_float4((p.x - q.x) * inv_dt * damp_factor, (p.y - q.y) * inv_dt * damp_factor,
                      (p.z - q.z) * inv_dt * damp_factor, 0.0f);
   x0[i] = p;
+  if (x_out) x_out[i] = p;
 }
 
 // ------------------------------------------------------------ batched kernel
@@ -273,9 +275,9 @@ hipError_t LaunchGround(hipStream_t s, float4* x, const float4* x0, int n, float
   return hipGetLastError();
 }
 hipError_t LaunchFinalize(hipStream_t s, float4* x0, float4* v, const float4* x, int n,
-                          const StepConsts& k) {
+                          const StepConsts& k, float4* x_out) {
   if (n <= 0) return hipSuccess;
-  FinalizeKernel<<<Blocks(n, 256), 256, 0, s>>>(x0, v, x, n, 1.0f / k.dt, k.damp_factor);
+  FinalizeKernel<<<Blocks(n, 256), 256, 0, s>>>(x0, v, x, n, 1.0f / k.dt, k.damp_factor, x_out);
   return hipGetLastError();
 }
 hipError_t LaunchBatchedSubstep(hipStream_t s, const BatchArgs& a, const StepConsts& k,

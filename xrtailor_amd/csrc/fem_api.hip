@@ -122,7 +122,7 @@ FemArgs MakeFemArgs(xrt_ctx* c) {
   a.iso_k = F.iso_k.ptr;
   a.iso_c = F.iso_c.ptr;
   a.iso_lam = F.iso_lam.ptr;
-  a.x = c->x.ptr;
+  a.x = c->xcur;
   return a;
 }
 

@@ -79,7 +79,8 @@ int Hash(xrt_ctx* c, int inst) {
   hipEvent_t e0, e1;
   NextPair(P.hash_events, P.hash_next, e0, e1);
   if (e0) XRT_CHECK_HIP(hipEventRecord(e0, c->stream));
-  XRT_CHECK_HIP(LaunchParticleHash(c->stream, Bufs(c), vm, tm, P.passes, c->x.ptr));
+  XRT_CHECK_HIP(LaunchParticleHash(c->stream, Bufs(c), vm, tm, P.passes,
+                                   inst < 0 ? c->xcur : c->x.ptr));
   if (e1) XRT_CHECK_HIP(hipEventRecord(e1, c->stream));
   return XRT_OK;
 }
@@ -89,7 +90,8 @@ int Collide(xrt_ctx* c, int inst) {
   const DevMap vm = Map(P, inst < 0 ? P.all_v : P.one_v[inst]);
   hipEvent_t e0, e1;
   NextPair(P.collide_events, P.collide_next, e0, e1);
-  XRT_CHECK_HIP(LaunchCollideParticles(c->stream, Bufs(c), vm, c->x.ptr, c->x0.ptr,
+  XRT_CHECK_HIP(LaunchCollideParticles(c->stream, Bufs(c), vm,
+                                       inst < 0 ? c->xcur : c->x.ptr, c->x0.ptr,
                                        c->params.ground_friction, c->params.relaxation_factor,
                                        e0, e1));
   return XRT_OK;

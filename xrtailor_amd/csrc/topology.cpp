@@ -121,6 +121,39 @@ std::vector<int32_t> ColorConstraints(const int32_t* cons, int arity, int n, int
                                       uint64_t seed, int mode, int* n_colors) {
   *n_colors = 0;
   if (n <= 0) return {};
+  if (mode == kColorGreedy) {
+    // first fit in constraint index order: each constraint takes the smallest color no
+    // lower-indexed neighbour holds (the index order follows the mesh's face order).  The
+    // neighbours' colors are those used at its vertices so far, 64 to a word; a neighbour is
+    // met at least at one of them.
+    std::vector<int32_t> color(n, 0);
+    size_t words = 1;
+    std::vector<uint64_t> used(nv, 0);
+    int most = 0;
+    for (int c = 0; c < n; ++c) {
+      const int32_t* v = cons + static_cast<size_t>(c) * arity;
+      size_t w = 0;
+      uint64_t taken = 0;
+      for (;; ++w) {
+        if (w == words) {  // every color so far is taken: room for 64 more
+          std::vector<uint64_t> wider(static_cast<size_t>(nv) * (words + 1), 0);
+          for (int i = 0; i < nv; ++i)
+            std::copy_n(&used[i * words], words, &wider[static_cast<size_t>(i) * (words + 1)]);
+          used.swap(wider);
+          ++words;
+        }
+        taken = 0;
+        for (int a = 0; a < arity; ++a) taken |= used[v[a] * words + w];
+        if (~taken) break;
+      }
+      const int bit = __builtin_ctzll(~taken);
+      color[c] = static_cast<int32_t>(64 * w) + bit;
+      most = std::max(most, color[c] + 1);
+      for (int a = 0; a < arity; ++a) used[v[a] * words + w] |= uint64_t(1) << bit;
+    }
+    *n_colors = most;  // first fit leaves no color empty
+    return color;
+  }
   // vertex -> constraints
   std::vector<int32_t> vptr(nv + 1, 0);
   for (int i = 0; i < n * arity; ++i) vptr[cons[i] + 1]++;
@@ -144,18 +177,7 @@ std::vector<int32_t> ColorConstraints(const int32_t* cons, int arity, int n, int
     aptr[c + 1] = static_cast<int32_t>(adj.size());
   }
   std::vector<int32_t> color(n, 0);
-  if (mode == kColorGreedy) {
-    // first fit in constraint index order: each constraint takes the smallest color no
-    // lower-indexed neighbour holds (the index order follows the mesh's face order)
-    std::vector<int32_t> stamp(static_cast<size_t>(n) + 2, -1);
-    for (int c = 0; c < n; ++c) {
-      for (int k = aptr[c]; k < aptr[c + 1]; ++k)
-        if (adj[k] < c) stamp[color[adj[k]]] = c;
-      int col = 0;
-      while (stamp[col] == c) ++col;
-      color[c] = col;
-    }
-  } else {
+  {
     int min_deg = 1 << 30;
     for (int c = 0; c < n; ++c) min_deg = std::min(min_deg, aptr[c + 1] - aptr[c]);
     min_deg = std::max(min_deg, 1);
