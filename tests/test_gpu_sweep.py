@@ -10,6 +10,8 @@ from xrtailor_amd import scenes
 from xrtailor_amd.solver import build_solver, make_params
 
 pytestmark = pytest.mark.gpu
+FEM = dict(constraint_model=1, fem_xx_stiffness=1e3, fem_yy_stiffness=1e3, fem_xy_stiffness=4e2,
+           fem_bending_stiffness=1e-2)
 
 
 def _spec(side, seed, slots=False):
@@ -56,6 +58,9 @@ def _equal(a, b):
     ((65,), dict(num_iterations=4, num_substeps=2, solve_bending=0)),
     ((103, 20), dict(num_iterations=3, num_substeps=2, bend_model=0)),
     ((190, 41), dict(num_iterations=2, num_substeps=2, coloring=1)),
+    ((2, 36, 20), dict(num_iterations=3, num_substeps=3, **FEM)),
+    ((103,), dict(num_iterations=2, num_substeps=2, solve_bending=0, **FEM)),
+    ((190, 41), dict(num_iterations=3, num_substeps=2, coloring=1, **FEM)),
 ])
 def test_sweeps_equal_plain(sides, kw):
     print(f"case sweeps vs plain: sides {sides} {kw}", flush=True)
@@ -72,6 +77,29 @@ def test_sweeps_with_attachments_and_changed_compliance_equal_plain():
     rng = scenes.Rng(5)
     comp = [(1e-7 * np.exp(rng.normal(3 * n * n - 4 * n + 1))).astype(np.float32) for n in (40, 51)]
     _equal(_run(specs, xp, True, comp), _run(specs, xp, False, comp))
+
+
+def test_constraint_model_changed_after_the_start_equals_plain():
+    print("case sweeps vs plain: XPBD, then FEM, then XPBD; and FEM first", flush=True)
+    runs = []
+    for batched in (True, False):
+        got = []
+        for models in ((0, 1, 0), (1, 0)):
+            s, ids = build_solver([_spec(40, 1), _spec(27, 2)],
+                                  make_params(bend_model=1, num_iterations=3, num_substeps=2,
+                                              **{**FEM, "constraint_model": models[0]}), seed=2)
+            if batched:
+                s.set_tuning(1024, 0, 1, 1)
+            for m in models:
+                p = s.params
+                p.constraint_model = m
+                s.set_params(p)
+                s.FramesBatched(1) if batched else s.FramesPlain(1)
+            s.sync()
+            got += [a for i in ids for a in s.GetState(i)]
+            s.close()
+        runs.append(got)
+    _equal(*runs)
 
 
 def test_mesh_without_locality_equals_plain():

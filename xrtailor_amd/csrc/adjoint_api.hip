@@ -264,7 +264,7 @@ int WideSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, AdjointData
   hipStream_t s = c->stream;
   const int N = W.n_total, n_inst = static_cast<int>(c->inst.size());
   c->xcur = c->x.ptr;
-  const bool sweep = c->patches.ready && !FemOn(c);
+  const bool sweep = PatchPlanOf(c).ready;
   const bool sweep_ground = sweep && k.enable_ground && c->total_slots == 0;
   float4* T = (A && sub >= 0)
                   ? A->tape.ptr + (static_cast<size_t>(A->slot) * c->params.num_substeps + sub) *
@@ -298,12 +298,12 @@ int WideSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, AdjointData
       for (int i = 0; i < n_inst; ++i)
         if (ObsContact(c, i) && (rc = SnapshotRecords(c, i, c->contact[i]->pass_cnt - 1)) != XRT_OK)
           return rc;
-    if (FemOn(c)) {  // never taped: the adjoint refuses the FEM constraints
-      if ((rc = FemIter(c, -1, it)) != XRT_OK) return rc;
-    } else if (sweep) {  // every color (and the ground plane, when it comes next) in one launch
+    if (sweep) {  // every color (and the ground plane, when it comes next) in one launch
       if ((rc = PatchIter(c, k, bm, it, sweep_ground, TI ? TI + A->off_s : nullptr,
                           TI ? TI + A->off_b : nullptr, TI ? TI + A->off_g : nullptr)) != XRT_OK)
         return rc;
+    } else if (FemOn(c)) {  // never taped: the adjoint refuses the FEM constraints
+      if ((rc = FemIter(c, -1, it)) != XRT_OK) return rc;
     } else {
       const WideArgs wa = MakeWideArgs(c);
       for (int col = 0; col < static_cast<int>(W.s_max.size()); ++col)

@@ -364,7 +364,8 @@ int TimeCandidate(xrt_ctx* c, const SavedRun& r, int n, float* ms) {
 // persistent / sweeps: one cloth of 32 x 32 2.07 / 2.23, 64 x 64 4.08 / 2.29, 100 x 100
 // 8.16 / 2.33; 64 of 64 x 64 4.47 / 3.33; 256 of 64 x 64 4.66 / 5.64)
 int DefaultPath(const xrt_ctx* ctx) {
-  return ctx->patches.ready && ctx->patches.split && !FemOn(ctx) ? 1 : 0;
+  const PatchPlanDev& plan = PatchPlanOf(ctx);
+  return plan.ready && plan.split ? 1 : 0;
 }
 
 int CheckTuning(const xrt_tuning& t) {
@@ -521,6 +522,7 @@ int xrt_set_params(xrt_ctx* ctx, const xrt_params* p) {
   if (!ctx->started) return XRT_OK;
   int rc = FemPrepare(ctx);
   if (rc != XRT_OK) return rc;
+  if (!FemOn(ctx) && !ctx->patches.xpbd.tried && (rc = PatchPrepare(ctx)) != XRT_OK) return rc;
   if (lists && (rc = ContactResizeLists(ctx)) != XRT_OK) return rc;
   return ParticleConfigure(ctx);
 }
@@ -838,14 +840,14 @@ int xrt_start(xrt_ctx* ctx, uint64_t seed) {
     XRT_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   }
   ctx->xcur = ctx->x.ptr;
-  int rc = PatchPrepare(ctx);
+  int rc = FemOn(ctx) ? XRT_OK : PatchPrepare(ctx);  // (the quality mode's plan: FemPrepare)
   if (rc != XRT_OK) return rc;
-  ctx->tuning.path = DefaultPath(ctx);
   if ((rc = ContactStart(ctx)) != XRT_OK) return rc;
   if ((rc = ParticleStart(ctx)) != XRT_OK) return rc;
   if ((rc = BindingStart(ctx)) != XRT_OK) return rc;
   ctx->fem.seed = seed;
   if ((rc = FemPrepare(ctx)) != XRT_OK) return rc;
+  ctx->tuning.path = DefaultPath(ctx);
   ctx->started = true;
   return XRT_OK;
 }

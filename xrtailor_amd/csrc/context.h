@@ -185,6 +185,10 @@ struct FemData {
   std::vector<size_t> f_map;     // wide strain launches: per-color block maps in `maps`
   std::vector<int> f_blocks;
   DevBuf<int32_t> maps;
+  // host copies for the sweep plan, released after it
+  std::vector<StrainC> host_sc;
+  std::vector<float4> host_k;
+  std::vector<float> host_c;
 };
 
 // Per-frame cache of xrt_record_frames (record_api.hip): two device slots packed after
@@ -217,16 +221,24 @@ struct WideConfig {
   DevBuf<int32_t> maps;
 };
 
-// Fused constraint sweeps (patch.h) over every instance, built at xrt_start.
-struct PatchData {
+// Fused constraint sweeps (patch.h) over every instance: the XPBD plan is built at
+// xrt_start, the quality mode's with its rest data.
+struct PatchPlanDev {
   bool ready = false;  // false: the colors run as launches of their own
+  bool tried = false;  // built, or found not to be worth it
   bool split = false;  // some instance is cut into several patches
-  int n = 0, ns = 0, nb = 0, threads = 0;
+  int n = 0, c0 = 0, c1 = 0;  // patches, colors of the first and the second family
+  int threads = 0;
   size_t lds_bytes = 0;
   DevBuf<PatchDev> patch;
-  DevBuf<int32_t> verts, off, bcon;
-  DevBuf<int4> srec, brec;
-  DevBuf<float> slam;
+  DevBuf<int32_t> verts, off;
+};
+struct PatchData {
+  PatchPlanDev xpbd, fem;
+  DevBuf<int4> srec, brec, frec, irec;
+  DevBuf<int32_t> bcon;
+  DevBuf<float4> finv, iK;
+  DevBuf<float> slam, ilam;
   DevBuf<float4> alt;  // the second position buffer
 };
 
@@ -418,10 +430,13 @@ bool FemOn(const xrt_ctx* ctx);
 FemConsts FemConstsOf(const xrt_params& p);  // at the substep dt
 int FemPrepare(xrt_ctx* ctx);
 int FemIter(xrt_ctx* ctx, int inst, int it);
-// patch_api.hip: the sweep plan of every instance (xrt_start, after the colors are uploaded),
-// one iteration's stretch and bend colors in one launch from xcur (which becomes the other
-// buffer), with the ground plane when `ground`; `it` of `iterations`; tapes as in adjoint.h
+// patch_api.hip: the sweep plans of every instance (PatchPrepare at xrt_start after the
+// colors are uploaded, PatchPrepareFem after the FEM set-up); PatchIter runs one iteration's
+// constraint colors in one launch from xcur (which becomes the other buffer), with the
+// ground plane when `ground`; `it` of `iterations`; tapes as in adjoint.h (XPBD only)
 int PatchPrepare(xrt_ctx* ctx);
+int PatchPrepareFem(xrt_ctx* ctx);
+const PatchPlanDev& PatchPlanOf(const xrt_ctx* ctx);  // of the current constraint model
 int PatchIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, int it, bool ground,
               float4* tape_s, float4* tape_b, float4* tape_g);
 int PatchRefreshCompliance(xrt_ctx* ctx);

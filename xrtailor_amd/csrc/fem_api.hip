@@ -199,7 +199,14 @@ int FemPrepare(xrt_ctx* ctx) {
   XRT_CHECK_HIP(F.maps.Upload(maps, s));
   XRT_CHECK_HIP(hipStreamSynchronize(s));
   F.ready = true;
-  return XRT_OK;
+  F.host_sc.swap(sc);
+  F.host_k.swap(iso_k);
+  F.host_c.swap(iso_c);
+  const int rc = PatchPrepareFem(ctx);
+  std::vector<StrainC>().swap(F.host_sc);
+  std::vector<float4>().swap(F.host_k);
+  std::vector<float>().swap(F.host_c);
+  return rc;
 }
 
 int FemIter(xrt_ctx* c, int inst, int it) {

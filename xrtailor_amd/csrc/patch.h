@@ -15,6 +15,12 @@
 //   slam    float[]      the entry's multiplier (every patch keeps its own copy)
 //   brec    int4[]       bend entry: local indices (4 x 16 bits), rest angle, compliance
 //   bcon    int32[]      the bend entry's element (bit 31: owned), read by the taped sweep
+// and for the quality mode's constraints, in a plan of their own
+//   frec    int4[]       strain entry: local indices (2 x 16 bits, 32 bits), rest area
+//   finv    float4[]     its inverse rest matrix
+//   irec    int4[]       isometric bending entry: local indices (4 x 16 bits), coefficient,
+//                        element (bit 31: owned); iK float4[], ilam float[] its weights and
+//                        multiplier
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -43,6 +49,19 @@ struct PatchArgs {
   int n, ns, nb;    // patches, stretch colors, bend colors
 };
 
+struct PatchFemArgs {
+  const PatchDev* patch;
+  const int32_t* verts;
+  const int32_t* off;
+  const int4* frec;
+  const float4* finv;
+  const int4* irec;
+  const float4* iK;
+  float* ilam;
+  float* ilam_out;
+  int n, nf, nb;
+};
+
 // What a sweep does beside the constraints: ground plane after them (before any later
 // operator of the iteration), tape of the operators' inputs (see adjoint.h; null: none)
 struct PatchSweep {
@@ -58,6 +77,8 @@ struct PatchSweep {
 
 hipError_t LaunchPatchSweep(hipStream_t s, const PatchArgs& a, const PatchSweep& w,
                             const StepConsts& k, const BendMode& m, int threads, size_t lds_bytes);
+hipError_t LaunchPatchFem(hipStream_t s, const PatchFemArgs& a, const PatchSweep& w,
+                          const StepConsts& k, const FemConsts& fk, int threads, size_t lds_bytes);
 hipError_t ConfigurePatchSweep(size_t lds_bytes);
 // the entries' compliances from the constraints sc (after they changed)
 hipError_t LaunchPatchCompliance(hipStream_t s, const StretchC* sc, int4* srec, int n);

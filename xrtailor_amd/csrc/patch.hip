@@ -1,6 +1,7 @@
 #include "patch.h"
 
 #include "elements.h"
+#include "fem.h"
 
 namespace xrt {
 namespace {
@@ -27,6 +28,76 @@ struct LaneOffsets {
   }
 };
 
+// One family of entries, its colors at off[o0 ..]: walked as (color, round) steps with a
+// workgroup barrier after each color.  load(e) gives entry e's record, one step ahead of its
+// use, so that a color waits for LDS and arithmetic only; solve(e, record) projects it.
+template <class Load, class Solve>
+__device__ __forceinline__ void SweepColors(const LaneOffsets& off, int o0, int colors, Load&& load,
+                                            Solve&& solve) {
+  using Rec = decltype(load(0));
+  const int tid = threadIdx.x, bs = blockDim.x;
+  int c = 0, beg = off[o0], end = off[o0 + 1];
+  Rec rec{};
+  if (beg + tid < end) rec = load(beg + tid);
+  while (c < colors) {
+    const int e = beg + tid;
+    const bool more = beg + bs < end;        // another round of this color
+    const int nbeg = more ? beg + bs : end;  // (colors lie one after the other)
+    const int nend = more ? end : (c + 1 < colors ? off[o0 + c + 2] : nbeg);
+    Rec next{};
+    if (nbeg + tid < nend) next = load(nbeg + tid);
+    if (e < end) solve(e, rec);
+    if (!more) {
+      if (nbeg > off[o0 + c]) LdsBarrier();  // (nothing to wait for after an empty color)
+      ++c;
+    }
+    beg = nbeg;
+    end = nend;
+    rec = next;
+  }
+}
+
+// the patch's vertices into LDS
+__device__ __forceinline__ void StageVertices(float4* X, const float4* __restrict__ x,
+                                              const int32_t* __restrict__ verts, int n) {
+  const int tid = threadIdx.x, bs = blockDim.x;
+  for (int v0 = tid; v0 < n; v0 += 4 * bs) {
+    int g[4];
+    float4 p[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) g[u] = v0 + u * bs < n ? verts[v0 + u * bs] : verts[v0];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) p[u] = x[g[u]];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (v0 + u * bs < n) X[v0 + u * bs] = p[u];
+  }
+  LdsBarrier();
+}
+
+// the patch's own vertices out of LDS, through the ground plane when it comes next
+template <bool kTape>
+__device__ __forceinline__ void WriteOwn(const float4* X, const PatchSweep& w, const StepConsts& k,
+                                         const int32_t* __restrict__ verts, int n_own) {
+  for (int v = threadIdx.x; v < n_own; v += blockDim.x) {
+    const int g = verts[v];
+    float4 x = X[v];
+    if (w.ground) {
+      if constexpr (kTape) w.tape_g[g] = x;
+      if (x.w > kEps && x.y < k.ground_y) x = GroundVertex(x, w.x0[g], k.ground_y, k.friction);
+    }
+    w.out[g] = x;
+  }
+}
+
+__device__ __forceinline__ int Lo16(int v) { return v & 0xffff; }
+__device__ __forceinline__ int Hi16(int v) { return static_cast<int>(static_cast<uint32_t>(v) >> 16); }
+
+struct StretchEntry {
+  int4 r;
+  float lam;
+};
+
 // Replaces one launch per color (20 on a grid): those were bound by the launches in small
 // contexts (about 5 us each for 2.5 us of work) and by sweeping the positions through L2 in
 // large ones.  Here a color costs a workgroup barrier, LDS gathers and arithmetic; the sweep is
@@ -40,122 +111,95 @@ __global__ __launch_bounds__(1024) void PatchSweepKernel(PatchArgs a, PatchSweep
                                                          BendMode m) {
   extern __shared__ float4 X[];
   const PatchDev p = a.patch[blockIdx.x];
-  const int tid = threadIdx.x, bs = blockDim.x;
   const LaneOffsets off(a.off + p.off, a.ns + a.nb + 2);
   const int32_t* __restrict__ verts = a.verts + p.vbeg;
-
-  // the entries are walked as (color, round) steps; each step's records are loaded one step
-  // ahead, so a color waits for LDS and arithmetic only
-  int c = 0, beg = off[0], end = off[1];
-  int4 rec = make_int4(0, 0, 0, 0);
-  float lam = 0.0f;
-  if (a.ns > 0 && beg + tid < end) {
-    rec = a.srec[beg + tid];
-    if (w.iter > 0) lam = a.slam[beg + tid];
-  }
-  for (int v0 = tid; v0 < p.n_loc; v0 += 4 * bs) {
-    int g[4];
-    float4 x[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) g[u] = v0 + u * bs < p.n_loc ? verts[v0 + u * bs] : verts[v0];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) x[u] = w.x[g[u]];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (v0 + u * bs < p.n_loc) X[v0 + u * bs] = x[u];
-  }
-  LdsBarrier();
-  while (c < a.ns) {
-    const int e = beg + tid;
-    const bool more = beg + bs < end;          // another round of this color
-    const int nbeg = more ? beg + bs : end;    // (colors lie one after the other)
-    const int nend = more ? end : (c + 1 < a.ns ? off[c + 2] : nbeg);
-    int4 nrec = make_int4(0, 0, 0, 0);
-    float nlam = 0.0f;
-    if (nbeg + tid < nend) {
-      nrec = a.srec[nbeg + tid];
-      if (w.iter > 0) nlam = a.slam[nbeg + tid];
-    }
-    if (e < end) {
-      const int i0 = rec.x & 0xffff, i1 = static_cast<int>(static_cast<uint32_t>(rec.x) >> 16);
-      const StretchC sc{i0, i1, __int_as_float(rec.y), __int_as_float(rec.z)};
-      float4 xa = X[i0], xb = X[i1];
-      if constexpr (kTape) {
-        if (rec.w < 0) {
-          const int q = rec.w & 0x7fffffff;
-          w.tape_s[2 * q] = make_float4(xa.x, xa.y, xa.z, lam);
-          w.tape_s[2 * q + 1] = xb;
-        }
-      }
-      if (StretchSolve(xa, xb, sc, lam, k.inv_dt2)) {
-        X[i0] = xa;
-        X[i1] = xb;
-      }
-      a.slam[e] = lam;
-      if (w.last && rec.w < 0) a.slam_out[rec.w & 0x7fffffff] = lam;
-    }
-    if (!more) {
-      if (nbeg > off[c]) LdsBarrier();  // (nothing to wait for after an empty color)
-      ++c;
-    }
-    beg = nbeg;
-    end = nend;
-    rec = nrec;
-    lam = nlam;
-  }
-  if (k.solve_bending && a.nb > 0) {
-    const int b0 = a.ns + 1;
-    c = 0;
-    beg = off[b0];
-    end = off[b0 + 1];
-    rec = make_int4(0, 0, 0, 0);
-    if (beg + tid < end) rec = a.brec[beg + tid];
-    while (c < a.nb) {
-      const int e = beg + tid;
-      const bool more = beg + bs < end;
-      const int nbeg = more ? beg + bs : end;
-      const int nend = more ? end : (c + 1 < a.nb ? off[b0 + c + 2] : nbeg);
-      int4 nrec = make_int4(0, 0, 0, 0);
-      if (nbeg + tid < nend) nrec = a.brec[nbeg + tid];
-      if (e < end) {
-        const int i0 = rec.x & 0xffff, i1 = static_cast<int>(static_cast<uint32_t>(rec.x) >> 16);
-        const int i2 = rec.y & 0xffff, i3 = static_cast<int>(static_cast<uint32_t>(rec.y) >> 16);
-        float4 x1 = X[i0], x2 = X[i1], x3 = X[i2], x4 = X[i3];
+  StageVertices(X, w.x, verts, p.n_loc);
+  SweepColors(
+      off, 0, a.ns,
+      [&](int e) {
+        return StretchEntry{a.srec[e], w.iter > 0 ? a.slam[e] : 0.0f};
+      },
+      [&](int e, StretchEntry& s) {
+        const int i0 = Lo16(s.r.x), i1 = Hi16(s.r.x);
+        const StretchC sc{i0, i1, __int_as_float(s.r.y), __int_as_float(s.r.z)};
+        float4 xa = X[i0], xb = X[i1];
         if constexpr (kTape) {
-          const int q = a.bcon[e];
-          if (q < 0) {
-            float4* t = w.tape_b + 3 * static_cast<int64_t>(q & 0x7fffffff);
-            t[0] = make_float4(x1.x, x1.y, x1.z, x2.x);
-            t[1] = make_float4(x2.y, x2.z, x3.x, x3.y);
-            t[2] = make_float4(x3.z, x4.x, x4.y, x4.z);
+          if (s.r.w < 0) {
+            const int64_t q = s.r.w & 0x7fffffff;
+            w.tape_s[2 * q] = make_float4(xa.x, xa.y, xa.z, s.lam);
+            w.tape_s[2 * q + 1] = xb;
           }
         }
-        if (BendSolve(x1, x2, x3, x4, make_float2(__int_as_float(rec.z), __int_as_float(rec.w)),
-                      k.inv_dt2, m)) {
-          X[i0] = x1;
-          X[i1] = x2;
-          X[i2] = x3;
-          X[i3] = x4;
+        if (StretchSolve(xa, xb, sc, s.lam, k.inv_dt2)) {
+          X[i0] = xa;
+          X[i1] = xb;
         }
-      }
-      if (!more) {
-        if (nbeg > off[b0 + c]) LdsBarrier();
-        ++c;
-      }
-      beg = nbeg;
-      end = nend;
-      rec = nrec;
-    }
-  }
-  for (int v = tid; v < p.n_own; v += bs) {
-    const int g = verts[v];
-    float4 x = X[v];
-    if (w.ground) {
-      if constexpr (kTape) w.tape_g[g] = x;
-      if (x.w > kEps && x.y < k.ground_y) x = GroundVertex(x, w.x0[g], k.ground_y, k.friction);
-    }
-    w.out[g] = x;
-  }
+        a.slam[e] = s.lam;
+        if (w.last && s.r.w < 0) a.slam_out[s.r.w & 0x7fffffff] = s.lam;
+      });
+  if (k.solve_bending)
+    SweepColors(
+        off, a.ns + 1, a.nb, [&](int e) { return a.brec[e]; },
+        [&](int e, const int4& r) {
+          const int i0 = Lo16(r.x), i1 = Hi16(r.x), i2 = Lo16(r.y), i3 = Hi16(r.y);
+          float4 x1 = X[i0], x2 = X[i1], x3 = X[i2], x4 = X[i3];
+          if constexpr (kTape) {
+            const int q = a.bcon[e];
+            if (q < 0) {
+              float4* t = w.tape_b + 3 * static_cast<int64_t>(q & 0x7fffffff);
+              t[0] = make_float4(x1.x, x1.y, x1.z, x2.x);
+              t[1] = make_float4(x2.y, x2.z, x3.x, x3.y);
+              t[2] = make_float4(x3.z, x4.x, x4.y, x4.z);
+            }
+          }
+          if (BendSolve(x1, x2, x3, x4, make_float2(__int_as_float(r.z), __int_as_float(r.w)),
+                        k.inv_dt2, m)) {
+            X[i0] = x1;
+            X[i1] = x2;
+            X[i2] = x3;
+            X[i3] = x4;
+          }
+        });
+  WriteOwn<kTape>(X, w, k, verts, p.n_own);
+}
+
+struct StrainEntry {
+  int4 r;
+  float4 inv;
+};
+struct IsoEntry {
+  int4 r;
+  float4 K;
+  float lam;
+};
+
+// The same for the quality mode's constraints: strain over the face colors, then isometric
+// bending over the hinge colors.
+__global__ __launch_bounds__(1024) void PatchFemKernel(PatchFemArgs a, PatchSweep w, StepConsts k,
+                                                       FemConsts fk) {
+  extern __shared__ float4 X[];
+  const PatchDev p = a.patch[blockIdx.x];
+  const LaneOffsets off(a.off + p.off, a.nf + a.nb + 2);
+  const int32_t* __restrict__ verts = a.verts + p.vbeg;
+  StageVertices(X, w.x, verts, p.n_loc);
+  SweepColors(
+      off, 0, a.nf, [&](int e) { return StrainEntry{a.frec[e], a.finv[e]}; },
+      [&](int, const StrainEntry& s) {
+        const StrainC c{Lo16(s.r.x), Hi16(s.r.x), s.r.y, __int_as_float(s.r.z),
+                        {s.inv.x, s.inv.y, s.inv.z, s.inv.w}};
+        StrainProject(X, c, fk);
+      });
+  if (k.solve_bending)
+    SweepColors(
+        off, a.nf + 1, a.nb,
+        [&](int e) { return IsoEntry{a.irec[e], a.iK[e], w.iter > 0 ? a.ilam[e] : 0.0f}; },
+        [&](int e, IsoEntry& s) {
+          IsoProject(X, make_int4(Lo16(s.r.x), Hi16(s.r.x), Lo16(s.r.y), Hi16(s.r.y)), s.K,
+                     __int_as_float(s.r.z), &s.lam, w.iter, fk);
+          a.ilam[e] = s.lam;
+          if (w.last && s.r.w < 0) a.ilam_out[s.r.w & 0x7fffffff] = s.lam;
+        });
+  WriteOwn<false>(X, w, k, verts, p.n_own);
 }
 
 __global__ __launch_bounds__(256) void PatchComplianceKernel(const StretchC* __restrict__ sc,
@@ -177,9 +221,19 @@ hipError_t LaunchPatchSweep(hipStream_t s, const PatchArgs& a, const PatchSweep&
   return hipGetLastError();
 }
 
+hipError_t LaunchPatchFem(hipStream_t s, const PatchFemArgs& a, const PatchSweep& w,
+                          const StepConsts& k, const FemConsts& fk, int threads,
+                          size_t lds_bytes) {
+  if (a.n <= 0) return hipSuccess;
+  if (threads < 64 || threads > 1024 || threads % 64) return hipErrorInvalidValue;
+  PatchFemKernel<<<a.n, threads, lds_bytes, s>>>(a, w, k, fk);
+  return hipGetLastError();
+}
+
 hipError_t ConfigurePatchSweep(size_t lds_bytes) {
-  const void* fns[2] = {reinterpret_cast<const void*>(&PatchSweepKernel<false>),
-                        reinterpret_cast<const void*>(&PatchSweepKernel<true>)};
+  const void* fns[3] = {reinterpret_cast<const void*>(&PatchSweepKernel<false>),
+                        reinterpret_cast<const void*>(&PatchSweepKernel<true>),
+                        reinterpret_cast<const void*>(&PatchFemKernel)};
   for (const void* f : fns) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
                                              static_cast<int>(lds_bytes));

@@ -14,19 +14,15 @@ namespace {
 constexpr int kPatchMaxVerts = 10240;  // 160 KB of LDS
 constexpr double kPatchMaxWork = 6.0;  // listed constraints / constraints
 
-// families of an instance: its stretch edges and bend elements in color-sorted order
-std::vector<PatchFamily> Families(const HostInstance& h) {
-  std::vector<PatchFamily> f(2);
-  f[0].arity = 2;
-  f[0].coloff = h.s_coloff;
-  f[0].cons.resize(2 * static_cast<size_t>(h.ne()));
-  for (int p = 0; p < h.ne(); ++p)
-    for (int a = 0; a < 2; ++a) f[0].cons[2 * static_cast<size_t>(p) + a] = h.edges[2 * h.s_order[p] + a];
-  f[1].arity = 4;
-  f[1].coloff = h.b_coloff;
-  f[1].cons.resize(4 * static_cast<size_t>(h.nb()));
-  for (int p = 0; p < h.nb(); ++p)
-    for (int a = 0; a < 4; ++a) f[1].cons[4 * static_cast<size_t>(p) + a] = h.bends[4 * h.b_order[p] + a];
+// constraints of `arity` vertices in sorted order: position p is cons[order[p]]
+PatchFamily Family(int arity, const std::vector<int32_t>& cons, const std::vector<int32_t>& order,
+                   const std::vector<int32_t>& coloff) {
+  PatchFamily f;
+  f.arity = arity;
+  f.coloff = coloff;
+  f.cons.resize(order.size() * arity);
+  for (size_t p = 0; p < order.size(); ++p)
+    std::copy_n(&cons[static_cast<size_t>(order[p]) * arity], arity, &f.cons[p * arity]);
   return f;
 }
 
@@ -56,18 +52,30 @@ bool ParallelFor(int n, F&& fn) {
   return ok;
 }
 
-}  // namespace
+int Pack16(int a, int b) { return static_cast<int>(static_cast<uint32_t>(a) | static_cast<uint32_t>(b) << 16); }
+int Bits(float v) {
+  int r;
+  std::memcpy(&r, &v, 4);
+  return r;
+}
+// constraint position p of a patch (bit 31: owned) as an index over all instances
+int Global(int p, int beg) {
+  return static_cast<int>((static_cast<uint32_t>(p & 0x7fffffff) + static_cast<uint32_t>(beg)) |
+                          (static_cast<uint32_t>(p) & 0x80000000u));
+}
 
-int PatchPrepare(xrt_ctx* ctx) {
-  PatchData& P = ctx->patches;
-  P.ready = false;
+// The plan of every instance from its two families; entry0 / entry1 (instance, position with
+// the owner bit, local indices) append one entry's records.  True with D filled (on the
+// host side in `dev`, `verts`, `off`), false when there is no plan.
+struct HostPlan {
+  std::vector<PatchDev> dev;
+  std::vector<int32_t> verts, off;
+};
+template <class Families, class Entry0, class Entry1>
+bool MakePlan(xrt_ctx* ctx, int c0, int c1, Families&& families, Entry0&& entry0, Entry1&& entry1,
+              PatchPlanDev& D, HostPlan& H) {
+  if (c0 + c1 == 0 || c0 + c1 + 2 > kPatchMaxOffsets) return false;
   const int ni = static_cast<int>(ctx->inst.size());
-  int ns = 0, nb = 0;
-  for (const HostInstance& h : ctx->inst) {
-    ns = std::max(ns, h.s_ncol);
-    nb = std::max(nb, h.b_ncol);
-  }
-  if (ns + nb == 0 || ns + nb + 2 > kPatchMaxOffsets) return XRT_OK;
   const int max_local = static_cast<int>(
       std::min<size_t>(kPatchMaxVerts, std::min<size_t>(ctx->max_lds, 160 * 1024) / sizeof(float4)));
   // Own vertices per patch: what gives 4 of 5 CUs a patch, down to 256 vertices, where the
@@ -83,125 +91,208 @@ int PatchPrepare(xrt_ctx* ctx) {
   std::vector<std::vector<Patch>> plan(ni);
   const bool built = ParallelFor(ni, [&](int i) {
     const HostInstance& h = ctx->inst[i];
-    const std::vector<PatchFamily> fam = Families(h);
+    const std::vector<PatchFamily> fam = families(i);
     // a mesh with little locality gets larger patches, or none
     for (int target = h.nv <= whole ? h.nv : cut; target < 4 * kPatchMaxVerts; target *= 4)
       if (BuildPatches(h.rest_pos.data(), h.nv, fam, target, max_local, kPatchMaxWork, &plan[i]))
         return true;
     return false;
   });
-  if (!built) return XRT_OK;
-  std::vector<PatchDev> dev;
-  std::vector<int32_t> verts, off, bcon;
-  std::vector<int4> srec, brec;
-  size_t max_loc = 0, max_color = 0;
+  if (!built) return false;
+  size_t max_loc = 0, n0 = 0, n1 = 0;
+  int max_color = 0;
   for (int i = 0; i < ni; ++i) {
-    const HostInstance& h = ctx->inst[i];
     for (const Patch& q : plan[i]) {
       PatchDev d;
-      d.vbeg = static_cast<int32_t>(verts.size());
+      d.vbeg = static_cast<int32_t>(H.verts.size());
       d.n_own = q.n_own;
       d.n_loc = static_cast<int32_t>(q.verts.size());
-      d.off = static_cast<int32_t>(off.size());
-      dev.push_back(d);
+      d.off = static_cast<int32_t>(H.off.size());
+      H.dev.push_back(d);
       max_loc = std::max(max_loc, q.verts.size());
-      for (int32_t v : q.verts) verts.push_back(h.desc.vbeg + v);
-      auto offsets = [&](int f, int n, size_t base) {
-        for (int c = 0; c <= n; ++c) {
+      for (int32_t v : q.verts) H.verts.push_back(ctx->inst[i].desc.vbeg + v);
+      for (int f = 0; f < 2; ++f) {
+        const size_t base = f == 0 ? n0 : n1;
+        if (base + q.cons[f].size() > static_cast<size_t>(INT32_MAX)) return false;
+        for (int c = 0; c <= (f == 0 ? c0 : c1); ++c) {
           const int cc = std::min<int>(c, static_cast<int>(q.coloff[f].size()) - 1);
-          off.push_back(static_cast<int32_t>(base) + q.coloff[f][cc]);
-          if (c > 0) max_color = std::max<size_t>(max_color, off[off.size() - 1] - off[off.size() - 2]);
+          H.off.push_back(static_cast<int32_t>(base) + q.coloff[f][cc]);
+          if (c > 0) max_color = std::max(max_color, H.off.back() - H.off[H.off.size() - 2]);
         }
-      };
-      offsets(0, ns, srec.size());
-      offsets(1, nb, brec.size());
-      for (size_t e = 0; e < q.cons[0].size(); ++e) {
-        const int p = q.cons[0][e] & 0x7fffffff;
-        const int o = h.s_order[p];
-        const uint32_t ij = q.local[0][2 * e] | static_cast<uint32_t>(q.local[0][2 * e + 1]) << 16;
-        int4 r;
-        r.x = static_cast<int>(ij);
-        std::memcpy(&r.y, &h.rest_len[o], 4);
-        std::memcpy(&r.z, &h.s_comp[o], 4);
-        r.w = static_cast<int>(static_cast<uint32_t>(h.sbeg + p) | (q.cons[0][e] & 0x80000000u));
-        srec.push_back(r);
       }
-      for (size_t e = 0; e < q.cons[1].size(); ++e) {
-        const int p = q.cons[1][e] & 0x7fffffff;
-        const int o = h.b_order[p];
-        const uint16_t* l = &q.local[1][4 * e];
-        int4 r;
-        r.x = static_cast<int>(l[0] | static_cast<uint32_t>(l[1]) << 16);
-        r.y = static_cast<int>(l[2] | static_cast<uint32_t>(l[3]) << 16);
-        std::memcpy(&r.z, &h.theta[o], 4);
-        std::memcpy(&r.w, &h.b_comp[o], 4);
-        brec.push_back(r);
-        bcon.push_back(static_cast<int>(static_cast<uint32_t>(h.bbeg + p) | (q.cons[1][e] & 0x80000000u)));
-      }
+      const int a0 = q.cons[0].empty() ? 0 : static_cast<int>(q.local[0].size() / q.cons[0].size());
+      const int a1 = q.cons[1].empty() ? 0 : static_cast<int>(q.local[1].size() / q.cons[1].size());
+      for (size_t e = 0; e < q.cons[0].size(); ++e) entry0(i, q.cons[0][e], &q.local[0][a0 * e]);
+      for (size_t e = 0; e < q.cons[1].size(); ++e) entry1(i, q.cons[1][e], &q.local[1][a1 * e]);
+      n0 += q.cons[0].size();
+      n1 += q.cons[1].size();
     }
+    plan[i].clear();
+    plan[i].shrink_to_fit();
   }
-  if (std::max({verts.size(), srec.size(), brec.size()}) > static_cast<size_t>(INT32_MAX)) return XRT_OK;
+  if (H.verts.size() > static_cast<size_t>(INT32_MAX)) return false;
+  // block b takes patch b: the patches with most work first, so that the last ones to start
+  // are the short ones (256 cloths: 23.7 -> 21.6 ms per frame)
+  auto entries = [&](const PatchDev& d) {  // a hinge costs about four edges
+    const int32_t* o = &H.off[d.off];
+    return (o[c0] - o[0]) + 4 * static_cast<int64_t>(o[c0 + 1 + c1] - o[c0 + 1]);
+  };
+  std::stable_sort(H.dev.begin(), H.dev.end(), [&](const PatchDev& a, const PatchDev& b) {
+    return entries(a) > entries(b);
+  });
+  D.n = static_cast<int>(H.dev.size());
+  D.split = D.n > ni;
+  D.c0 = c0;
+  D.c1 = c1;
+  D.lds_bytes = sizeof(float4) * max_loc;
+  D.threads = std::min(1024, std::max(64, (max_color + 63) / 64 * 64));
+  return true;
+}
+
+hipError_t UploadPlan(xrt_ctx* ctx, PatchPlanDev& D, const HostPlan& H) {
+  hipError_t e = D.patch.Upload(H.dev, ctx->stream);
+  if (e == hipSuccess) e = D.verts.Upload(H.verts, ctx->stream);
+  if (e == hipSuccess) e = D.off.Upload(H.off, ctx->stream);
+  if (e == hipSuccess && !ctx->patches.alt.ptr) e = ctx->patches.alt.Alloc(std::max<size_t>(ctx->x.n, 1));
+  return e;
+}
+
+// a plan whose buffers did not fit is dropped: the colors then run as launches of their own
+template <class... Bufs>
+int FinishPlan(PatchPlanDev& D, hipError_t e, Bufs&... bufs) {
+  if (e == hipSuccess && D.lds_bytes > 64 * 1024) e = ConfigurePatchSweep(D.lds_bytes);
+  if (e == hipSuccess) {
+    D.ready = true;
+    return XRT_OK;
+  }
+  (bufs.Free(), ...);
+  D.patch.Free();
+  D.verts.Free();
+  D.off.Free();
+  (void)hipGetLastError();
+  if (e == hipErrorOutOfMemory) return XRT_OK;
+  SetError(std::string("constraint sweep plan: ") + hipGetErrorString(e));
+  return XRT_ERR_HIP;
+}
+
+}  // namespace
+
+int PatchPrepare(xrt_ctx* ctx) {
+  PatchData& P = ctx->patches;
+  P.xpbd.ready = false;
+  P.xpbd.tried = true;
+  int ns = 0, nb = 0;
+  for (const HostInstance& h : ctx->inst) {
+    ns = std::max(ns, h.s_ncol);
+    nb = std::max(nb, h.b_ncol);
+  }
+  HostPlan H;
+  std::vector<int4> srec, brec;
+  std::vector<int32_t> bcon;
+  const bool made = MakePlan(
+      ctx, ns, nb,
+      [&](int i) {
+        const HostInstance& h = ctx->inst[i];
+        return std::vector<PatchFamily>{Family(2, h.edges, h.s_order, h.s_coloff),
+                                        Family(4, h.bends, h.b_order, h.b_coloff)};
+      },
+      [&](int i, int p, const uint16_t* l) {
+        const HostInstance& h = ctx->inst[i];
+        const int o = h.s_order[p & 0x7fffffff];
+        srec.push_back(make_int4(Pack16(l[0], l[1]), Bits(h.rest_len[o]), Bits(h.s_comp[o]),
+                                 Global(p, h.sbeg)));
+      },
+      [&](int i, int p, const uint16_t* l) {
+        const HostInstance& h = ctx->inst[i];
+        const int o = h.b_order[p & 0x7fffffff];
+        brec.push_back(make_int4(Pack16(l[0], l[1]), Pack16(l[2], l[3]), Bits(h.theta[o]),
+                                 Bits(h.b_comp[o])));
+        bcon.push_back(Global(p, h.bbeg));
+      },
+      P.xpbd, H);
+  if (!made) return XRT_OK;
   hipStream_t s = ctx->stream;
-  // block b takes patch b: the patches with most work first, so that the last ones to start are then the short ones (256 cloths: 23.7 ->
-  // 21.6 ms per frame)
-  {
-    auto entries = [&](const PatchDev& d) {  // a bend costs about four stretches
-      const int32_t* o = &off[d.off];
-      return (o[ns] - o[0]) + 4 * static_cast<int64_t>(o[ns + 1 + nb] - o[ns + 1]);
-    };
-    std::stable_sort(dev.begin(), dev.end(), [&](const PatchDev& a, const PatchDev& b) {
-      return entries(a) > entries(b);
-    });
-  }
-  P.n = static_cast<int>(dev.size());
-  P.split = P.n > ni;
-  P.ns = ns;
-  P.nb = nb;
-  P.lds_bytes = sizeof(float4) * max_loc;
-  P.threads = static_cast<int>(std::min<size_t>(1024, std::max<size_t>(64, (max_color + 63) / 64 * 64)));
-  hipError_t e = P.patch.Upload(dev, s);
-  if (e == hipSuccess) e = P.verts.Upload(verts, s);
-  if (e == hipSuccess) e = P.off.Upload(off, s);
+  hipError_t e = UploadPlan(ctx, P.xpbd, H);
   if (e == hipSuccess) e = P.srec.Upload(srec, s);
   if (e == hipSuccess) e = P.brec.Upload(brec, s);
   if (e == hipSuccess) e = P.bcon.Upload(bcon, s);
   if (e == hipSuccess) e = P.slam.Alloc(std::max<size_t>(srec.size(), 1));
-  if (e == hipSuccess) e = P.alt.Alloc(std::max<size_t>(ctx->x.n, 1));
-  if (e != hipSuccess) {  // no memory left for the plan: the colors run as launches of their own
-    P.patch.Free();
-    P.verts.Free();
-    P.off.Free();
-    P.srec.Free();
-    P.brec.Free();
-    P.bcon.Free();
-    P.slam.Free();
-    P.alt.Free();
-    (void)hipGetLastError();
-    return e == hipErrorOutOfMemory ? XRT_OK : XRT_ERR_HIP;
+  return FinishPlan(P.xpbd, e, P.srec, P.brec, P.bcon, P.slam);
+}
+
+int PatchPrepareFem(xrt_ctx* ctx) {
+  PatchData& P = ctx->patches;
+  const FemData& F = ctx->fem;
+  P.fem.ready = false;
+  P.fem.tried = true;
+  int nf = 0, nb = 0;
+  for (size_t i = 0; i < ctx->inst.size(); ++i) {
+    nf = std::max(nf, F.inst[i].ncol);
+    nb = std::max(nb, ctx->inst[i].b_ncol);
   }
-  if (P.lds_bytes > 64 * 1024) XRT_CHECK_HIP(ConfigurePatchSweep(P.lds_bytes));
-  P.ready = true;
-  return XRT_OK;
+  HostPlan H;
+  std::vector<int4> frec, irec;
+  std::vector<float4> finv, iK;
+  const bool made = MakePlan(
+      ctx, nf, nb,
+      [&](int i) {
+        const HostInstance& h = ctx->inst[i];
+        return std::vector<PatchFamily>{Family(3, h.tris, F.inst[i].order, F.inst[i].coloff),
+                                        Family(4, h.bends, h.b_order, h.b_coloff)};
+      },
+      [&](int i, int p, const uint16_t* l) {
+        const StrainC& c = F.host_sc[F.inst[i].fbeg + (p & 0x7fffffff)];
+        frec.push_back(make_int4(Pack16(l[0], l[1]), l[2], Bits(c.area), 0));
+        finv.push_back(make_float4(c.inv[0], c.inv[1], c.inv[2], c.inv[3]));
+      },
+      [&](int i, int p, const uint16_t* l) {
+        const int b = ctx->inst[i].bbeg + (p & 0x7fffffff);
+        irec.push_back(make_int4(Pack16(l[0], l[1]), Pack16(l[2], l[3]), Bits(F.host_c[b]),
+                                 Global(p, ctx->inst[i].bbeg)));
+        iK.push_back(F.host_k[b]);
+      },
+      P.fem, H);
+  if (!made) return XRT_OK;
+  hipStream_t s = ctx->stream;
+  hipError_t e = UploadPlan(ctx, P.fem, H);
+  if (e == hipSuccess) e = P.frec.Upload(frec, s);
+  if (e == hipSuccess) e = P.finv.Upload(finv, s);
+  if (e == hipSuccess) e = P.irec.Upload(irec, s);
+  if (e == hipSuccess) e = P.iK.Upload(iK, s);
+  if (e == hipSuccess) e = P.ilam.Alloc(std::max<size_t>(irec.size(), 1));
+  return FinishPlan(P.fem, e, P.frec, P.finv, P.irec, P.iK, P.ilam);
+}
+
+const PatchPlanDev& PatchPlanOf(const xrt_ctx* ctx) {
+  return FemOn(ctx) ? ctx->patches.fem : ctx->patches.xpbd;
 }
 
 int PatchIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, int it, bool ground,
               float4* tape_s, float4* tape_b, float4* tape_g) {
   PatchData& P = ctx->patches;
-  PatchArgs a{P.patch.ptr, P.verts.ptr, P.off.ptr, P.srec.ptr, P.slam.ptr, P.brec.ptr, P.bcon.ptr,
-              ctx->slam.ptr, P.n, P.ns, P.nb};
+  const PatchPlanDev& D = PatchPlanOf(ctx);
   float4* out = ctx->xcur == ctx->x.ptr ? P.alt.ptr : ctx->x.ptr;
-  PatchSweep w{ctx->xcur, out, ctx->x0.ptr, it, it + 1 == k.iterations ? 1 : 0, ground ? 1 : 0,
-               tape_s, tape_b, tape_g};
-  const int threads = ctx->tuning.wide_per_thread == 2 ? std::max(64, (P.threads / 2 + 63) / 64 * 64)
-                                                       : P.threads;
-  XRT_CHECK_HIP(LaunchPatchSweep(ctx->stream, a, w, k, m, threads, P.lds_bytes));
+  const PatchSweep w{ctx->xcur, out, ctx->x0.ptr, it, it + 1 == k.iterations ? 1 : 0,
+                     ground ? 1 : 0, tape_s, tape_b, tape_g};
+  const int threads = ctx->tuning.wide_per_thread == 2 ? std::max(64, (D.threads / 2 + 63) / 64 * 64)
+                                                       : D.threads;
+  if (FemOn(ctx)) {
+    const PatchFemArgs a{D.patch.ptr, D.verts.ptr, D.off.ptr,  P.frec.ptr,
+                         P.finv.ptr,  P.irec.ptr,  P.iK.ptr,   P.ilam.ptr,
+                         ctx->fem.iso_lam.ptr,     D.n, D.c0, D.c1};
+    XRT_CHECK_HIP(LaunchPatchFem(ctx->stream, a, w, k, FemConstsOf(ctx->params), threads, D.lds_bytes));
+  } else {
+    const PatchArgs a{D.patch.ptr, D.verts.ptr, D.off.ptr, P.srec.ptr, P.slam.ptr, P.brec.ptr,
+                      P.bcon.ptr, ctx->slam.ptr, D.n, D.c0, D.c1};
+    XRT_CHECK_HIP(LaunchPatchSweep(ctx->stream, a, w, k, m, threads, D.lds_bytes));
+  }
   ctx->xcur = out;
   return XRT_OK;
 }
 
 int PatchRefreshCompliance(xrt_ctx* ctx) {
   PatchData& P = ctx->patches;
-  if (!P.ready) return XRT_OK;
+  if (!P.xpbd.ready) return XRT_OK;
   XRT_CHECK_HIP(LaunchPatchCompliance(ctx->stream, ctx->sc.ptr, P.srec.ptr,
                                       static_cast<int>(P.srec.n)));
   return XRT_OK;
