@@ -32,12 +32,12 @@ struct BvhView {
   Box* box = nullptr;
   int32_t* escape = nullptr;
   uint32_t* root = nullptr;  // 6 order-preserving encoded floats (lower xyz, upper xyz)
-  int32_t* flags = nullptr;     // bottom-up arrival counters (internal nodes)
+  int32_t* flags = nullptr;     // arrival counters of the merge over chunk boundaries
   uint32_t* counts = nullptr;   // pair traversal: pairs per lhs leaf
   uint32_t* offsets = nullptr;  //                 their exclusive prefix
   int32_t* total = nullptr;     //                 and their sum (1 int)
-  Box* packed = nullptr;        // traversal records (PackNodeBody), batched pair refresh
-  int32_t* lvl = nullptr;       // LevelBottomUpWG's depth and child lists (4 nf ints)
+  Box* packed = nullptr;        // traversal records (StoreNode)
+  int32_t* lvl = nullptr;       // subtree roots of the merge's chunks (MergeChunk, 2 nf ints)
   int4* leaf_face = nullptr;    // per leaf slot: its face's record (batched pair refresh)
 };
 
@@ -58,7 +58,7 @@ struct Lbvh {
   DevBuf<uint32_t> hist;  // radix histogram / offsets
   DevBuf<int32_t> counts, offsets, total;  // pair traversal scratch (per lhs leaf)
   DevBuf<Box> packed;                      // traversal records of the nodes
-  DevBuf<int32_t> lvl;                     // depth lists of the level-by-level merge
+  DevBuf<int32_t> lvl;                     // subtree roots of the merge's chunks
   DevBuf<int4> leaf_face;                  // per leaf slot: its face's record
   BvhView view() const;
   // (re)allocate for a mesh; uploads faces (host int32[3*nf])
@@ -83,7 +83,6 @@ struct TreeBuildDev {
   int32_t* escape = nullptr;
   uint32_t* root = nullptr;
   uint32_t* hist = nullptr;
-  int32_t* flags = nullptr;
 };
 
 // A set of trees rebuilt together, every build step of every tree in one launch (the

@@ -188,19 +188,13 @@ __device__ __forceinline__ void LeafNodesBody(const uint32_t* __restrict__ morto
                                               const int32_t* __restrict__ order,
                                               const Box* __restrict__ leaf, int nf, int i,
                                               int4* __restrict__ nodes, Box* __restrict__ box,
-                                              uint64_t* __restrict__ code,
-                                              int32_t* __restrict__ flags) {
+                                              uint64_t* __restrict__ code) {
   const int ni = nf - 1;
   const int obj = order[i];
   nodes[ni + i] = make_int4(-1, -1, -1, obj);
   box[ni + i] = leaf[obj];
   code[i] = (static_cast<uint64_t>(morton[i]) << 32) | static_cast<uint32_t>(obj);
-  if (i < ni) {
-    nodes[i] = make_int4(-1, -1, -1, -1);
-    flags[i] = 0;
-  } else {
-    flags[ni] = 0;  // the topology changes: LevelBottomUpWG lists the depths again
-  }
+  if (i < ni) nodes[i] = make_int4(-1, -1, -1, -1);
 }
 
 __global__ __launch_bounds__(kBlock) void LeafNodesKernel(const uint32_t* __restrict__ morton,
@@ -208,10 +202,9 @@ __global__ __launch_bounds__(kBlock) void LeafNodesKernel(const uint32_t* __rest
                                                           const Box* __restrict__ leaf, int nf,
                                                           int4* __restrict__ nodes,
                                                           Box* __restrict__ box,
-                                                          uint64_t* __restrict__ code,
-                                                          int32_t* __restrict__ flags) {
+                                                          uint64_t* __restrict__ code) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nf) LeafNodesBody(morton, order, leaf, nf, i, nodes, box, code, flags);
+  if (i < nf) LeafNodesBody(morton, order, leaf, nf, i, nodes, box, code);
 }
 
 // determine_range / find_split / ConstructInternalNodes64Bits_Kernel (BVH.cu:102-210,297-317)
@@ -278,19 +271,23 @@ __global__ __launch_bounds__(kBlock) void KarrasKernel(const uint64_t* __restric
 }
 
 
-// bottom-up boxes: the second thread to reach a node merges its two children (the
-// result is the union of the descendant leaves, as AssignAABBAtomic_Kernel's atomic
-// min / max, BVH.cu:540-557, and AssignAABBCAS_Kernel, BVH.cu:515-538).  grow = 1 keeps
-// the old box too (Update's grow-only semantics).
-__global__ __launch_bounds__(kBlock) void BottomUpKernel(const int4* __restrict__ nodes,
-                                                         Box* __restrict__ box,
-                                                         int32_t* __restrict__ flags, int nf,
-                                                         int grow) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nf) return;
-  BottomUpBody(nodes, box, flags, nf, grow, i);
+// the boxes of one tree's internal nodes (MergeChunk, MergeTop), its leaves first grown by
+// pa [and pb] when given
+__global__ __launch_bounds__(kMergeChunk) void MergeChunkKernel(BvhView t, const float4* pa,
+                                                                const float4* pb) {
+  __shared__ MergeShared m;
+  MergeChunk(t, blockIdx.x, m, [&](int i) {
+    return pa ? GrownLeaf(t, pa, pb, i) : t.box[t.nf - 1 + i];
+  });
 }
 
+__global__ __launch_bounds__(1024) void MergeTopKernel(BvhView t) { MergeTop(t); }
+
+void LaunchMerge(const BvhView& t, const float4* pa, const float4* pb, hipStream_t s) {
+  const int chunks = Blocks(t.nf, kMergeChunk);
+  MergeChunkKernel<<<chunks, kMergeChunk, 0, s>>>(t, pa, pb);
+  if (chunks > 1) MergeTopKernel<<<1, 1024, 0, s>>>(t);
+}
 
 __global__ __launch_bounds__(kBlock) void ZeroFlagsKernel(int32_t* flags, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -330,18 +327,6 @@ __global__ __launch_bounds__(kBlock) void RefitPredKernel(const float4* __restri
   RefitPredBody(x1, n1, tol, i, pred);
 }
 
-// leaf grows by its 3 pred corners (midstep) or by Face::ComputeBounds(ccd) of x [and x0]
-__global__ __launch_bounds__(kBlock) void GrowLeavesKernel(const int4* __restrict__ nodes,
-                                                           const int4* __restrict__ tris,
-                                                           const float4* __restrict__ pa,
-                                                           const float4* __restrict__ pb, int nf,
-                                                           Box* __restrict__ box,
-                                                           int32_t* __restrict__ flags) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nf) return;
-  GrowLeafBody(nodes, tris, pa, pb, nf, i, box, flags);
-}
-
 }  // namespace
 
 namespace {
@@ -355,8 +340,8 @@ __global__ __launch_bounds__(kBlock) void QueryKernel(BvhView t, const float4* _
   const float4 a = p0[q];
   int32_t* out = hits + static_cast<size_t>(q) * kMaxHits;
   int k = 0;
-  const int found = p1 ? StacklessQuery<true>(t, a, p1[q], [&](int obj) { out[k++] = obj; })
-                       : StacklessQuery<false>(t, a, a, [&](int obj) { out[k++] = obj; });
+  const int found = p1 ? StacklessQuery<true>(t.packed, t.nf, a, p1[q], [&](int obj) { out[k++] = obj; })
+                       : StacklessQuery<false>(t.packed, t.nf, a, a, [&](int obj) { out[k++] = obj; });
   counts[q] = found;
 }
 
@@ -451,7 +436,7 @@ __global__ __launch_bounds__(kBlock) void MultiRadixScatterKernel(const TreeBuil
 __global__ __launch_bounds__(kBlock) void MultiLeafNodesKernel(const TreeBuildDev* set,
                                                                const int32_t* off, int n) {
   XRT_TREE_INDEX()
-  if (i < t.nf) LeafNodesBody(t.morton, t.order, t.leaf, t.nf, i, t.nodes, t.box, t.code, t.flags);
+  if (i < t.nf) LeafNodesBody(t.morton, t.order, t.leaf, t.nf, i, t.nodes, t.box, t.code);
 }
 
 __global__ __launch_bounds__(kBlock) void MultiKarrasKernel(const TreeBuildDev* set,
@@ -494,7 +479,6 @@ hipError_t TreeSet::Setup(const std::vector<Lbvh*>& in, const std::vector<const 
     t.escape = b.escape.ptr;
     t.root = b.root.ptr;
     t.hist = b.hist.ptr;
-    t.flags = b.flags.ptr;
     d.push_back(t);
     trees.push_back(&b);
   }
@@ -596,9 +580,8 @@ hipError_t Lbvh::Setup(const int32_t* tris_host, int nfaces, int nverts, hipStre
   if ((e = escape.Alloc(nn)) != hipSuccess) return e;
   if ((e = packed.Alloc(nn)) != hipSuccess) return e;
   if ((e = flags.Alloc(std::max(nf, 1))) != hipSuccess) return e;
-  // flags[nf - 1]: the level lists of LevelBottomUpWG are not yet valid
-  if ((e = hipMemsetAsync(flags.ptr, 0, sizeof(int32_t) * flags.n, s)) != hipSuccess) return e;
-  if ((e = lvl.Alloc(4 * static_cast<size_t>(std::max(nf, 1)))) != hipSuccess) return e;
+  // (chunk c's list starts at kMergeChunk c < nf and its count is at nf + c < 2 nf)
+  if ((e = lvl.Alloc(2 * static_cast<size_t>(std::max(nf, 1)))) != hipSuccess) return e;
   if ((e = leaf_face.Alloc(std::max(nf, 1))) != hipSuccess) return e;
   if ((e = root.Alloc(6)) != hipSuccess) return e;
   if ((e = hist.Alloc(static_cast<size_t>(256) * nblocks)) != hipSuccess) return e;
@@ -636,12 +619,10 @@ hipError_t LbvhBuild(Lbvh& b, const float4* x0, const float4* x, const float4* n
     std::swap(vin, vout);
   }
   LeafNodesKernel<<<Blocks(nf), kBlock, 0, s>>>(b.morton.ptr, b.order.ptr, b.leaf.ptr, nf,
-                                                b.nodes.ptr, b.box.ptr, b.code.ptr, b.flags.ptr);
-  if (nf > 1) {
-    KarrasKernel<<<Blocks(nf - 1), kBlock, 0, s>>>(b.code.ptr, nf, b.nodes.ptr);
-    if (merge) BottomUpKernel<<<Blocks(nf), kBlock, 0, s>>>(b.nodes.ptr, b.box.ptr, b.flags.ptr, nf, 0);
-  }
+                                                b.nodes.ptr, b.box.ptr, b.code.ptr);
+  if (nf > 1) KarrasKernel<<<Blocks(nf - 1), kBlock, 0, s>>>(b.code.ptr, nf, b.nodes.ptr);
   EscapeKernel<<<Blocks(2 * nf - 1), kBlock, 0, s>>>(b.nodes.ptr, 2 * nf - 1, b.escape.ptr);
+  if (merge) LaunchMerge(b.view(), nullptr, nullptr, s);
   b.active = true;
   return hipGetLastError();
 }
@@ -649,20 +630,14 @@ hipError_t LbvhBuild(Lbvh& b, const float4* x0, const float4* x, const float4* n
 hipError_t LbvhRefitMidstep(Lbvh& b, const float4* x1, const float4* n1, float tol, hipStream_t s) {
   if (!b.active) return hipSuccess;
   RefitPredKernel<<<Blocks(b.nv), kBlock, 0, s>>>(x1, n1, tol, b.nv, b.pred.ptr);
-  GrowLeavesKernel<<<Blocks(b.nf), kBlock, 0, s>>>(b.nodes.ptr, b.tris.ptr, b.pred.ptr, nullptr,
-                                                   b.nf, b.box.ptr, b.flags.ptr);
-  if (b.nf > 1)
-    BottomUpKernel<<<Blocks(b.nf), kBlock, 0, s>>>(b.nodes.ptr, b.box.ptr, b.flags.ptr, b.nf, 0);
+  LaunchMerge(b.view(), b.pred.ptr, nullptr, s);
   return hipGetLastError();
 }
 
 hipError_t LbvhUpdate(Lbvh& b, const float4* x, const float4* x0, int ccd, hipStream_t s) {
   if (!b.active) return hipSuccess;
   RefitPredKernel<<<Blocks(b.nv), kBlock, 0, s>>>(x, nullptr, 0.0f, b.nv, b.pred.ptr);
-  GrowLeavesKernel<<<Blocks(b.nf), kBlock, 0, s>>>(b.nodes.ptr, b.tris.ptr, x, ccd ? x0 : nullptr,
-                                                   b.nf, b.box.ptr, b.flags.ptr);
-  if (b.nf > 1)
-    BottomUpKernel<<<Blocks(b.nf), kBlock, 0, s>>>(b.nodes.ptr, b.box.ptr, b.flags.ptr, b.nf, 1);
+  LaunchMerge(b.view(), x, ccd ? x0 : nullptr, s);
   return hipGetLastError();
 }
 

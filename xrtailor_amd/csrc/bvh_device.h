@@ -89,19 +89,15 @@ __device__ __forceinline__ void RefitPredBody(const float4* __restrict__ x1,
   }
 }
 
-// leaf i grows by its 3 corners of pa (midstep) or by Face::ComputeBounds(ccd) of pa [and
-// pb]; resets the arrival flag of internal node i for the bottom-up pass that follows
-__device__ __forceinline__ void GrowLeafBody(const int4* __restrict__ nodes,
-                                             const int4* __restrict__ tris,
-                                             const float4* __restrict__ pa,
-                                             const float4* __restrict__ pb, int nf, int i,
-                                             Box* __restrict__ box, int32_t* __restrict__ flags) {
-  const int ni = nf - 1;
-  const int4 t = tris[nodes[ni + i].w];
-  Box b = box[ni + i];
+// leaf i's box, grown by its 3 corners of pa (midstep) or by Face::ComputeBounds(ccd) of pa
+// [and pb]
+__device__ __forceinline__ Box GrownLeaf(const BvhView& t, const float4* pa, const float4* pb, int i) {
+  const int ni = t.nf - 1;
+  const int4 f = t.tris[t.nodes[ni + i].w];
+  const Box b = t.box[ni + i];
   float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.0f);
   float4 hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
-  const int vid[3] = {t.x, t.y, t.z};
+  const int vid[3] = {f.x, f.y, f.z};
   for (int c = 0; c < 3; ++c) {
     const float4 p = pa[vid[c]];
     lo.x = Mn(lo.x, p.x); lo.y = Mn(lo.y, p.y); lo.z = Mn(lo.z, p.z);
@@ -112,158 +108,129 @@ __device__ __forceinline__ void GrowLeafBody(const int4* __restrict__ nodes,
       hi.x = Mx(hi.x, q.x); hi.y = Mx(hi.y, q.y); hi.z = Mx(hi.z, q.z);
     }
   }
-  box[ni + i] = MergeBox(b, Box{lo, hi});
-  if (i < ni) flags[i] = 0;
+  return MergeBox(b, Box{lo, hi});
 }
 
-// bottom-up boxes from leaf i: the second thread to reach a node merges its two children
-// (the union of the descendant leaves, as AssignAABBAtomic_Kernel's atomic min / max,
-// BVH.cu:540-557, and AssignAABBCAS_Kernel, BVH.cu:515-538).  grow keeps the old box too
-// (Update's grow-only semantics).
-__device__ __forceinline__ void BottomUpBody(const int4* __restrict__ nodes, Box* __restrict__ box,
-                                             int32_t* __restrict__ flags, int nf, int grow, int i) {
-  int node = nf - 1 + i;
-  int p = nodes[node].x;
-  // a root-ward walk is at most nf - 1 levels; the bound also guards against a malformed tree
-  for (int level = 0; p >= 0 && p < nf - 1 && level < nf; ++level) {
-    __threadfence();
-    const int old = atomicAdd(&flags[p], 1);
-    if (old == 0) return;
-    __threadfence();
-    const int4 pn = nodes[p];
-    Box m = MergeBox(box[pn.y], box[pn.z]);
-    if (grow) m = MergeBox(m, box[p]);
-    box[p] = m;
+// A node's box and its traversal record: the box with lo.w = left child (internal node) or
+// -(object + 1) (leaf) and hi.w = escape, so that one 32-byte load serves a visit.  Every merge
+// writes both, so the records are current whenever the boxes are.
+__device__ __forceinline__ void StoreNode(const BvhView& t, int node, Box b, int code, int escape) {
+  t.box[node] = b;
+  b.lo.w = __int_as_float(code);
+  b.hi.w = __int_as_float(escape);
+  t.packed[node] = b;
+}
+
+// Boxes of the internal nodes from the leaves up, in two launches.
+//
+// An internal node of the radix tree covers a contiguous range of leaves and has the number of
+// one end of it.  So a workgroup that takes kMergeChunk consecutive leaves can merge every
+// node whose range lies within them out of LDS: the second child to arrive at a node (a
+// counter in LDS) merges the two.  What is left are the nodes over chunk boundaries, a few
+// percent; one workgroup per tree merges them the same way through L2 (MergeTop), starting
+// from the roots of the chunks' subtrees, which MergeChunk lists in t.lvl (chunk c's at
+// [kMergeChunk c ..), their number at nf + c).  The boxes are unions (min / max), so the
+// order of the merges changes nothing; a leaf that only grows keeps every old box inside
+// the new one.  One workgroup merging a whole tree depth by depth (as before) took 716 us for
+// the 130,050 faces of a 256 x 256 cloth and a climb over all leaves with device-wide fences
+// 435 us for 64,082; the two launches take 256 us and 89 us.
+constexpr int kMergeChunk = 1024;  // leaves per workgroup, one per thread
+
+struct MergeShared {
+  float box[6][2 * kMergeChunk];  // leaves of the chunk, then its internal nodes
+  int parent[kMergeChunk], left[kMergeChunk], right[kMergeChunk], escape[kMergeChunk];
+  int count[kMergeChunk];
+  int roots;
+};
+
+// leaf_box(i): the box of leaf slot i (called once per leaf); a workgroup of kMergeChunk threads
+template <class LeafBox>
+__device__ __forceinline__ void MergeChunk(const BvhView& t, int chunk, MergeShared& m,
+                                           LeafBox&& leaf_box) {
+  const int nf = t.nf, ni = nf - 1, cb = chunk * kMergeChunk;
+  const int tid = threadIdx.x, i = cb + tid;
+  if (i < ni) {
+    const int4 nd = t.nodes[i];
+    m.parent[tid] = nd.x;
+    m.left[tid] = nd.y;
+    m.right[tid] = nd.z;
+    m.escape[tid] = t.escape[i];
+    t.flags[i] = 0;
+  }
+  m.count[tid] = 0;
+  if (tid == 0) m.roots = 0;
+  auto put = [&](int k, const Box& b) {
+    m.box[0][k] = b.lo.x; m.box[1][k] = b.lo.y; m.box[2][k] = b.lo.z;
+    m.box[3][k] = b.hi.x; m.box[4][k] = b.hi.y; m.box[5][k] = b.hi.z;
+  };
+  auto get = [&](int k) {
+    return Box{make_float4(m.box[0][k], m.box[1][k], m.box[2][k], 0.0f),
+               make_float4(m.box[3][k], m.box[4][k], m.box[5][k], 0.0f)};
+  };
+  int node = ni + i, p = -1;
+  if (i < nf) {
+    const int4 nd = t.nodes[node];
+    p = nd.x;
+    const Box b = leaf_box(i);
+    StoreNode(t, node, b, -(nd.w + 1), t.escape[node]);
+    put(tid, b);
+  }
+  __syncthreads();
+  int stop = -1, at = -1;  // the node this thread stopped with, the parent it waits at (-1: outside)
+  while (p >= 0) {         // (a climb passes each node of the chunk at most once)
+    const int lp = p - cb;
+    if (lp < 0 || lp >= kMergeChunk) {
+      stop = node;
+      break;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    const int old = atomicAdd(&m.count[lp], 1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    if (old == 0) {
+      stop = node;
+      at = lp;
+      break;
+    }
+    // a child is a leaf (number ni + slot) or an internal node, of this chunk either way
+    const int l = m.left[lp], r = m.right[lp];
+    const Box b = MergeBox(get(l >= ni ? l - ni - cb : kMergeChunk + l - cb),
+                           get(r >= ni ? r - ni - cb : kMergeChunk + r - cb));
+    put(kMergeChunk + lp, b);
+    StoreNode(t, p, b, l, m.escape[lp]);
     node = p;
-    p = pn.x;
-  }
-}
-
-// The same merge for a whole tree by ONE workgroup, level by level: a top-down
-// breadth-first pass lists the internal nodes by depth in lvl (entries [0, nf - 1): the
-// nodes; entries nf - 1 + d: where depth d starts), then the depths are merged deepest first
-// with a workgroup barrier between them.  A node's children are one level deeper, so every
-// merge reads finished boxes.  Each thread waits on a handful of loads per level instead of
-// a chain of atomics per climbed node (an arrival-counter climb by one workgroup took 1.5 ms
-// for the batched workload's largest trees), and the boxes are unions (min / max),
-// independent of the order, hence identical to BottomUpBody's.  lvl holds 4 nf ints (the
-// order, the depth starts, the depth count at 2 nf - 1, then each listed node's two
-// children as int2 from 2 nf on); node 0 is the root; a malformed tree cannot list more than
-// nf - 1 nodes.  The lists depend on the topology only, so they are kept while flags[nf - 1]
-// (a slot the arrival counters do not use) is 1: every build clears it (LeafNodesBody).
-__device__ __forceinline__ void LevelBottomUpWG(const int4* __restrict__ nodes,
-                                                Box* __restrict__ box,
-                                                int32_t* __restrict__ lvl,
-                                                int32_t* __restrict__ flags, int nf, int grow) {
-  const int ni = nf - 1;
-  if (ni <= 0) return;
-  int32_t* order = lvl;
-  int32_t* start = lvl + ni;  // start[d], d <= depth count <= ni
-  int2* kids = reinterpret_cast<int2*>(lvl + 2 * nf);  // (first, second) child of order[t]
-  if (flags[ni] == 1) {       // the same value in every thread: written after the lists
-    const int depths = lvl[2 * ni + 1];
-    for (int d = depths - 1; d >= 0; --d) {
-      const int lo = start[d], hi = start[d + 1];
-      for (int t = lo + static_cast<int>(threadIdx.x); t < hi; t += blockDim.x) {
-        const int p = order[t];
-        const int2 ch = kids[t];  // loaded beside p: one dependent load less per node
-        Box m = MergeBox(box[ch.x], box[ch.y]);
-        if (grow) m = MergeBox(m, box[p]);
-        box[p] = m;
-      }
-      __syncthreads();
-    }
-    return;
-  }
-  __shared__ int s_end;
-  if (threadIdx.x == 0) {
-    order[0] = 0;
-    start[0] = 0;
-    start[1] = 1;
-    s_end = 1;
+    p = m.parent[lp];
   }
   __syncthreads();
-  int b = 0, e = 1, depths = 1;  // depths listed; the deepest is [b, e)
-  while (b < e) {
-    for (int t = b + static_cast<int>(threadIdx.x); t < e; t += blockDim.x) {
-      const int4 nd = nodes[order[t]];
-      if (nd.y >= 0 && nd.y < ni) {
-        const int q = atomicAdd(&s_end, 1);
-        if (q < ni) order[q] = nd.y;
-      }
-      if (nd.z >= 0 && nd.z < ni) {
-        const int q = atomicAdd(&s_end, 1);
-        if (q < ni) order[q] = nd.z;
-      }
-    }
-    __syncthreads();
-    const int next = min(s_end, ni);
-    __syncthreads();  // every thread has read s_end before the next depth adds to it
-    b = e;
-    e = next;
-    if (e > b) {
-      if (threadIdx.x == 0) start[depths + 1] = e;
-      ++depths;
-    }
-  }
-  for (int t = static_cast<int>(threadIdx.x); t < min(e, ni); t += blockDim.x) {
-    const int4 nd = nodes[order[t]];
-    kids[t] = make_int2(nd.y, nd.z);
-  }
-  if (threadIdx.x == 0) {
-    lvl[2 * ni + 1] = depths;
-    flags[ni] = 1;  // every thread read the old value before the first barrier above
-  }
+  // stopped for good where no second child of this chunk arrived
+  if (stop >= 0 && (at < 0 || m.count[at] == 1)) t.lvl[cb + atomicAdd(&m.roots, 1)] = stop;
   __syncthreads();
-  for (int d = depths - 1; d >= 0; --d) {
-    const int lo = start[d], hi = start[d + 1];
-    for (int t = lo + static_cast<int>(threadIdx.x); t < hi; t += blockDim.x) {
-      const int p = order[t];
-      const int4 pn = nodes[p];
-      Box m = MergeBox(box[pn.y], box[pn.z]);
-      if (grow) m = MergeBox(m, box[p]);
-      box[p] = m;
-    }
-    __syncthreads();
-  }
+  if (tid == 0) t.lvl[nf + chunk] = m.roots;
 }
 
-// CountPairs_Kernel (BVH.cu:1149-1179): rhs leaves overlapping lhs leaf id dilated by th
-__device__ __forceinline__ uint32_t CountPairsBody(const BvhView& l, const BvhView& r, float th,
-                                                   int id) {
-  const Box lb = l.box[l.nf - 1 + id];
-  int node = 0;
-  uint32_t c = 0;
-  const int max_steps = 2 * r.nf;  // each node is visited at most once
-  for (int step = 0; node != -1 && step < max_steps; ++step) {
-    const int4 nd = r.nodes[node];
-    if (OverlapDilated(r.box[node], lb, th)) {
-      if (nd.w >= 0) {
-        ++c;
-        node = r.escape[node];
-      } else {
-        node = nd.y;
+// the nodes over chunk boundaries, by one workgroup after every chunk of the tree
+__device__ __forceinline__ void MergeTop(const BvhView& t) {
+  const int nf = t.nf, ni = nf - 1;
+  const int chunks = (nf + kMergeChunk - 1) / kMergeChunk;
+  if (chunks <= 1) return;
+  const int lane = threadIdx.x & 63, waves = static_cast<int>(blockDim.x) >> 6;
+  for (int c = static_cast<int>(threadIdx.x) >> 6; c < chunks; c += waves) {
+    const int n = t.lvl[nf + c];
+    for (int q = lane; q < n; q += 64) {
+      int p = t.nodes[t.lvl[c * kMergeChunk + q]].x;
+      for (int level = 0; p >= 0 && p < ni && level < nf; ++level) {
+        __threadfence_block();
+        if (atomicAdd(&t.flags[p], 1) == 0) break;
+        __threadfence_block();
+        const int4 nd = t.nodes[p];
+        StoreNode(t, p, MergeBox(t.box[nd.y], t.box[nd.z]), nd.y, t.escape[p]);
+        p = nd.x;
       }
-    } else {
-      node = r.escape[node];
     }
   }
-  return c;
 }
 
-// Traversal record of node i for the pair traversal: its box with lo.w = left child
-// (internal node) or -(object + 1) (leaf) and hi.w = escape, so that one 32-byte load serves
-// a visit.  Written from nodes / box / escape after the boxes change.
-__device__ __forceinline__ void PackNodeBody(const BvhView& t, int i) {
-  const int4 nd = t.nodes[i];
-  Box b = t.box[i];
-  b.lo.w = __int_as_float(nd.w >= 0 ? -(nd.w + 1) : nd.y);
-  b.hi.w = __int_as_float(t.escape[i]);
-  t.packed[i] = b;
-}
-
-// the stackless traversal of CountPairsBody / FindPairsBody over packed records: on_leaf
-// (rhs object) for every rhs leaf overlapping lb dilated by th, in the same order
+// the stackless pair traversal (CountPairs_Kernel / FindPairs_Kernel, BVH.cu:1149-1227) over
+// the traversal records: on_leaf(rhs object) for every rhs leaf overlapping lb dilated by th
 template <class OnLeaf>
 __device__ __forceinline__ void TraversePacked(const Box* __restrict__ pk, int nf, const Box& lb,
                                                float th, OnLeaf&& on_leaf) {
@@ -312,30 +279,26 @@ __device__ __forceinline__ void TraversePackedFace(const Box* __restrict__ pk,
   }
 }
 
+// CountPairs_Kernel (BVH.cu:1149-1179): rhs leaves overlapping lhs leaf id dilated by th
+__device__ __forceinline__ uint32_t CountPairsBody(const BvhView& l, const BvhView& r, float th,
+                                                   int id) {
+  uint32_t c = 0;
+  TraversePacked(r.packed, r.nf, l.packed[l.nf - 1 + id], th, [&](int) { ++c; });
+  return c;
+}
+
 // FindPairs_Kernel (BVH.cu:1189-1227): leaf id's pairs fill [lo, lo + n) backwards; only
 // slots below cap are written
 __device__ __forceinline__ void FindPairsBody(const BvhView& l, const BvhView& r, float th, int id,
                                               int64_t lo, uint32_t n, int2* __restrict__ pairs,
                                               int64_t cap) {
-  const Box lb = l.box[l.nf - 1 + id];
-  const int lobj = l.nodes[l.nf - 1 + id].w;
+  const Box lb = l.packed[l.nf - 1 + id];
+  const int lobj = -__float_as_int(lb.lo.w) - 1;
   int64_t index = lo + n - 1;
-  int node = 0;
-  const int max_steps = 2 * r.nf;
-  for (int step = 0; node != -1 && step < max_steps; ++step) {
-    const int4 nd = r.nodes[node];
-    if (OverlapDilated(r.box[node], lb, th)) {
-      if (nd.w >= 0) {
-        if (index >= lo && index < cap) pairs[index] = make_int2(lobj, nd.w);
-        --index;
-        node = r.escape[node];
-      } else {
-        node = nd.y;
-      }
-    } else {
-      node = r.escape[node];
-    }
-  }
+  TraversePacked(r.packed, r.nf, lb, th, [&](int robj) {
+    if (index >= lo && index < cap) pairs[index] = make_int2(lobj, robj);
+    --index;
+  });
 }
 
 // UpdateNodeNormals (xrtailor/src/physics/PhysicsMeshHelper.cu:196-210,282-295) for vertex
@@ -463,35 +426,9 @@ __device__ __forceinline__ void BlockExclusiveScan(uint32_t* __restrict__ a, int
 
 // QueryDeviceStackless (xrtailor/src/physics/broad_phase/lbvh/BVH.cu:957-1021): visits the
 // leaves whose boxes contain p (segment == false) or meet segment p->q, in traversal order,
-// calling f(object) for at most kMaxHits of them.
-template <bool kSegment, typename F>
-__device__ __forceinline__ int StacklessQuery(const BvhView& t, float4 p, float4 q, F&& f) {
-  int node = 0, found = 0;
-  const int max_steps = 2 * t.nf;  // a stackless pass visits each node at most once
-  for (int step = 0; node != -1 && step < max_steps; ++step) {
-    if (found >= kMaxHits) break;
-    const Box bx = t.box[node];
-    const bool hit = kSegment ? OverlapSegment(bx, p, q) : OverlapPoint(bx, p);
-    const int4 nd = t.nodes[node];
-    if (hit) {
-      if (nd.w >= 0) {
-        f(nd.w);
-        ++found;
-        node = t.escape[node];
-      } else {
-        node = nd.y;
-      }
-    } else {
-      node = t.escape[node];
-    }
-  }
-  return found;
-}
-
-// StacklessQuery over the packed traversal records (PackNodeBody): one 32-byte load per
-// visit instead of the box, node and escape arrays; the same visits in the same order
+// calling f(object) for at most kMaxHits of them; one traversal record per visit.
 template <bool kSegment, class F>
-__device__ __forceinline__ int StacklessQueryPacked(const Box* __restrict__ pk, int nf, float4 p,
+__device__ __forceinline__ int StacklessQuery(const Box* __restrict__ pk, int nf, float4 p,
                                                     float4 q, F&& f) {
   int node = 0, found = 0;
   const int max_steps = 2 * nf;

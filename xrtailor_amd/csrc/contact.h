@@ -153,10 +153,13 @@ constexpr int kStageObjBits = 20;  // the item mask (12 bits) takes the rest of 
 // 256-thread blocks each instance needs, followed by the instance of each block (device),
 // and the block totals (host)
 struct MultiMaps {
-  enum Kind { kVert, kEdge, kFace, kObsVert, kObsFace, kPair, kKinds };
+  enum Kind { kVert, kEdge, kFace, kObsVert, kObsFace, kPair, kChunk, kObsChunk, kKinds };
   const int32_t* off[kKinds] = {};
   int blocks[kKinds] = {};
   int n = 0;
+  // a cloth / obstacle tree has more than one chunk of leaves (kChunk, kObsChunk: one block
+  // per chunk of the trees' merges, bvh_device.h)
+  bool cloth_top = false, obs_top = false;
 };
 
 // collision pass: obstacle x1 = lerp(x0, x, alpha), midstep normals, RefitMidstep(tol)

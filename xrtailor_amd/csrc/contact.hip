@@ -137,15 +137,6 @@ __device__ __forceinline__ void InterpolateBody(const float4* __restrict__ x0,
 }
 
 // GenerateVF_DCD_Kernel (PBDCollision.cu:17-43)
-// the obstacle query of the generate bodies: over the packed records when they are current
-// (the batched collision pass packs them after its refit), else over the node arrays
-template <bool kSegment, bool kPk, class F>
-__device__ __forceinline__ void ObsQuery(const BvhView& t, float4 p, float4 q, F&& f) {
-  if constexpr (kPk) StacklessQueryPacked<kSegment>(t.packed, t.nf, p, q, f);
-  else StacklessQuery<kSegment>(t, p, q, f);
-}
-
-template <bool kPk = false>
 __device__ __forceinline__ void VfDcdGenerateBody(const float4* __restrict__ x, int i,
                                                   const BvhView& t, int32_t* __restrict__ face,
                                                   float4* __restrict__ qout) {
@@ -154,7 +145,7 @@ __device__ __forceinline__ void VfDcdGenerateBody(const float4* __restrict__ x, 
   float best = kScalarMax;
   int bi = -1;
   F3 bq{0, 0, 0};
-  ObsQuery<false, kPk>(t, p4, p4, [&](int f) {
+  StacklessQuery<false>(t.packed, t.nf, p4, p4, [&](int f) {
     const int4 tr = t.tris[f];
     F3 q;
     const float d = NearestPoint(p, L3(t.pred[tr.x]), L3(t.pred[tr.y]), L3(t.pred[tr.z]), q);
@@ -165,7 +156,6 @@ __device__ __forceinline__ void VfDcdGenerateBody(const float4* __restrict__ x, 
 }
 
 // GenerateVFCCD_Kernel (PBDCollision.cu:236-270)
-template <bool kPk = false>
 __device__ __forceinline__ void VfCcdGenerateBody(const float4* __restrict__ x0,
                                                   const float4* __restrict__ x, int i,
                                                   const BvhView& t, int32_t* __restrict__ face,
@@ -179,7 +169,7 @@ __device__ __forceinline__ void VfCcdGenerateBody(const float4* __restrict__ x0,
   if (len < kEpsC) return;
   d = M(d, 1.0f / len);
   float best = kScalarMax;
-  ObsQuery<true, kPk>(t, a4, b4, [&](int f) {
+  StacklessQuery<true>(t.packed, t.nf, a4, b4, [&](int f) {
     const int4 tr = t.tris[f];
     const float s = RayIntersect(p1, d, len, L3(t.pred[tr.x]), L3(t.pred[tr.y]), L3(t.pred[tr.z]));
     if (s < best) {
@@ -192,7 +182,6 @@ __device__ __forceinline__ void VfCcdGenerateBody(const float4* __restrict__ x0,
 }
 
 // GenerateEE_DCD_Kernel (PBDCollision.cu:100-150)
-template <bool kPk = false>
 __device__ __forceinline__ void EeDcdGenerateBody(const float4* __restrict__ x,
                                                   const int2* __restrict__ edges, int e,
                                                   const BvhView& t,
@@ -205,7 +194,7 @@ __device__ __forceinline__ void EeDcdGenerateBody(const float4* __restrict__ x,
   EeRec r;
   r.a = make_float4(kScalarMax, 0.0f, 0.0f, 0.0f);
   r.p2 = r.q2 = r.fn = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  ObsQuery<true, kPk>(t, pc4, qc4, [&](int f) {
+  StacklessQuery<true>(t.packed, t.nf, pc4, qc4, [&](int f) {
     const int4 tr = t.tris[f];
     const uint32_t info = rtri[f];
     const F3 ov[3] = {L3(t.pred[tr.x]), L3(t.pred[tr.y]), L3(t.pred[tr.z])};
@@ -993,18 +982,31 @@ __global__ __launch_bounds__(kBlock) void MultiNormalPredKernel(const InstContac
   RefitPredBody(c.o_x1, c.o_n1, tol, i, c.obvh.pred);
 }
 
-__global__ __launch_bounds__(kBlock) void MultiObsGrowKernel(const InstContactDev* ic,
-                                                             const int32_t* off, int n) {
-  XRT_MULTI_INDEX(kObsFace, c.obs_nf)
-  GrowLeafBody(c.obvh.nodes, c.obvh.tris, c.obvh.pred, nullptr, c.obs_nf, i, c.obvh.box,
-               c.obvh.flags);
+// the chunk of a tree that block b of a chunk map stands for (-1: idle block)
+__device__ __forceinline__ int ChunkOf(const int32_t* off, int n, int& inst) {
+  const int lblk = XcdBlock(off, n);
+  if (lblk < 0) return -1;
+  inst = InstOfBlock(off, n, lblk);
+  return lblk - off[inst];
 }
 
-// one workgroup per instance merges its obstacle tree
-__global__ __launch_bounds__(1024) void MultiObsBottomUpKernel(const InstContactDev* ic) {
+// obstacle trees: leaves grown by the contact points (pred), merged (MergeChunk / MergeTop)
+__global__ __launch_bounds__(kMergeChunk) void MultiObsMergeKernel(const InstContactDev* ic,
+                                                                   const int32_t* off, int n,
+                                                                   int grow) {
+  __shared__ MergeShared m;
+  int k;
+  const int chunk = ChunkOf(off, n, k);
+  if (chunk < 0) return;
+  const InstContactDev& c = ic[k];
+  MergeChunk(c.obvh, chunk, m, [&](int i) {
+    return grow ? GrownLeaf(c.obvh, c.obvh.pred, nullptr, i) : c.obvh.box[c.obs_nf - 1 + i];
+  });
+}
+
+__global__ __launch_bounds__(1024) void MultiObsMergeTopKernel(const InstContactDev* ic) {
   const InstContactDev& c = ic[blockIdx.x];
-  if (c.has_obs && c.obs_nf > 1)
-    LevelBottomUpWG(c.obvh.nodes, c.obvh.box, c.obvh.lvl, c.obvh.flags, c.obs_nf, 0);
+  if (c.has_obs) MergeTop(c.obvh);
 }
 
 __global__ __launch_bounds__(kBlock) void MultiVfGenerateKernel(const InstContactDev* ic,
@@ -1013,8 +1015,8 @@ __global__ __launch_bounds__(kBlock) void MultiVfGenerateKernel(const InstContac
                                                                 const float4* __restrict__ x) {
   XRT_MULTI_INDEX(kVert, c.nv)
   if (!c.has_obs) return;
-  VfDcdGenerateBody<true>(x + c.vbeg, i, c.obvh, c.vf_face, c.vf_q);
-  VfCcdGenerateBody<true>(x0 + c.vbeg, x + c.vbeg, i, c.obvh, c.rt_face, c.rt_q);
+  VfDcdGenerateBody(x + c.vbeg, i, c.obvh, c.vf_face, c.vf_q);
+  VfCcdGenerateBody(x0 + c.vbeg, x + c.vbeg, i, c.obvh, c.rt_face, c.rt_q);
 }
 
 __global__ __launch_bounds__(kBlock) void MultiEeGenerateKernel(const InstContactDev* ic,
@@ -1022,7 +1024,7 @@ __global__ __launch_bounds__(kBlock) void MultiEeGenerateKernel(const InstContac
                                                                 const float4* __restrict__ x) {
   XRT_MULTI_INDEX(kEdge, c.ne)
   if (!c.has_obs) return;
-  EeDcdGenerateBody<true>(x + c.vbeg, c.cloth.edges, i, c.obvh, c.obs.rtri, c.ee, c.ee_none);
+  EeDcdGenerateBody(x + c.vbeg, c.cloth.edges, i, c.obvh, c.obs.rtri, c.ee, c.ee_none);
 }
 
 // cloth LBVH Update(ccd): pred = x, then leaves grow by bounds(x, x0)
@@ -1033,55 +1035,34 @@ __global__ __launch_bounds__(kBlock) void MultiClothPredKernel(const InstContact
   RefitPredBody(x + c.vbeg, nullptr, 0.0f, i, c.cbvh.pred);
 }
 
-__global__ __launch_bounds__(kBlock) void MultiClothGrowKernel(const InstContactDev* ic,
-                                                               const int32_t* off, int n,
-                                                               const float4* __restrict__ x,
-                                                               const float4* __restrict__ x0) {
-  XRT_MULTI_INDEX(kFace, c.nf)
-  GrowLeafBody(c.cbvh.nodes, c.cbvh.tris, x + c.vbeg, x0 + c.vbeg, c.nf, i, c.cbvh.box,
-               c.cbvh.flags);
+// cloth trees: with x, leaves grown by the bounds of (x, x0) and each leaf slot's face record
+// written; merged (MergeChunk / MergeTop)
+__global__ __launch_bounds__(kMergeChunk) void MultiClothMergeKernel(const InstContactDev* ic,
+                                                                     const int32_t* off, int n,
+                                                                     const float4* x,
+                                                                     const float4* x0) {
+  __shared__ MergeShared m;
+  int k;
+  const int chunk = ChunkOf(off, n, k);
+  if (chunk < 0) return;
+  const InstContactDev& c = ic[k];
+  MergeChunk(c.cbvh, chunk, m, [&](int i) {
+    if (!x) return c.cbvh.box[c.nf - 1 + i];
+    c.cbvh.leaf_face[i] = c.cloth.trir[c.cbvh.nodes[c.nf - 1 + i].w];
+    return GrownLeaf(c.cbvh, x + c.vbeg, x0 + c.vbeg, i);
+  });
 }
 
-// one workgroup per instance merges its cloth tree (grow-only)
-__global__ __launch_bounds__(1024) void MultiClothBottomUpKernel(const InstContactDev* ic) {
+__global__ __launch_bounds__(1024) void MultiClothMergeTopKernel(const InstContactDev* ic) {
   const InstContactDev& c = ic[blockIdx.x];
-  if (c.scal && c.nf > 1)
-    LevelBottomUpWG(c.cbvh.nodes, c.cbvh.box, c.cbvh.lvl, c.cbvh.flags, c.nf, 1);
+  if (c.scal) MergeTop(c.cbvh);
 }
 
-// frame start: one workgroup per tree merges the freshly built trees of every instance
-// (workgroups [0, n): cloth trees when `cloth`, [n, 2n): obstacle trees)
-__global__ __launch_bounds__(1024) void MultiBuildMergeKernel(const InstContactDev* ic, int n,
-                                                              int cloth) {
-  const bool obs = blockIdx.x >= static_cast<unsigned>(n);
-  const InstContactDev& c = ic[obs ? blockIdx.x - n : blockIdx.x];
-  if (!c.scal) return;
-  if (obs) {
-    if (c.has_obs && c.obs_nf > 1)
-      LevelBottomUpWG(c.obvh.nodes, c.obvh.box, c.obvh.lvl, c.obvh.flags, c.obs_nf, 0);
-  } else if (cloth && c.nf > 1) {
-    LevelBottomUpWG(c.cbvh.nodes, c.cbvh.box, c.cbvh.lvl, c.cbvh.flags, c.nf, 0);
-  }
-}
-
-
-// traversal records of every cloth tree (thread i: leaf nf - 1 + i and internal node i)
-__global__ __launch_bounds__(kBlock) void MultiPackClothKernel(const InstContactDev* ic,
-                                                               const int32_t* off, int n) {
-  XRT_MULTI_INDEX(kFace, c.nf)
-  PackNodeBody(c.cbvh, c.nf - 1 + i);
-  if (i < c.nf - 1) PackNodeBody(c.cbvh, i);
-  c.cbvh.leaf_face[i] = c.cloth.trir[c.cbvh.nodes[c.nf - 1 + i].w];
-}
-
-// traversal records of every obstacle tree
-__global__ __launch_bounds__(kBlock) void MultiPackObsKernel(const InstContactDev* ic,
-                                                             const int32_t* off, int n) {
+// each obstacle leaf slot's face record
+__global__ __launch_bounds__(kBlock) void MultiObsFacesKernel(const InstContactDev* ic,
+                                                              const int32_t* off, int n) {
   XRT_MULTI_INDEX(kObsFace, c.obs_nf)
-  if (!c.has_obs) return;
-  PackNodeBody(c.obvh, c.obs_nf - 1 + i);
-  if (i < c.obs_nf - 1) PackNodeBody(c.obvh, i);
-  c.obvh.leaf_face[i] = c.obs.trir[c.obvh.nodes[c.obs_nf - 1 + i].w];
+  if (c.has_obs) c.obvh.leaf_face[i] = c.obs.trir[c.obvh.nodes[c.obs_nf - 1 + i].w];
 }
 
 // pairs per cloth leaf against the obstacle (self = 0) or the cloth itself (self = 1),
@@ -1684,10 +1665,8 @@ hipError_t MultiObstacleRefit(hipStream_t s, const InstContactDev* ic, const Mul
   if (Empty(m, MK::kObsVert)) return hipSuccess;
   MultiInterpolateKernel<<<XcdGrid(m.blocks[MK::kObsVert]), kBlock, 0, s>>>(ic, m.off[MK::kObsVert], m.n, alpha);
   MultiNormalPredKernel<<<XcdGrid(m.blocks[MK::kObsVert]), kBlock, 0, s>>>(ic, m.off[MK::kObsVert], m.n, tol);
-  MultiObsGrowKernel<<<XcdGrid(m.blocks[MK::kObsFace]), kBlock, 0, s>>>(ic, m.off[MK::kObsFace], m.n);
-  MultiObsBottomUpKernel<<<m.n, 1024, 0, s>>>(ic);
-  // the generate pass that follows queries the packed records
-  MultiPackObsKernel<<<XcdGrid(m.blocks[MK::kObsFace]), kBlock, 0, s>>>(ic, m.off[MK::kObsFace], m.n);
+  MultiObsMergeKernel<<<XcdGrid(m.blocks[MK::kObsChunk]), kMergeChunk, 0, s>>>(ic, m.off[MK::kObsChunk], m.n, 1);
+  if (m.obs_top) MultiObsMergeTopKernel<<<m.n, 1024, 0, s>>>(ic);
   return hipGetLastError();
 }
 
@@ -1706,11 +1685,10 @@ hipError_t MultiPairs(hipStream_t s, const InstContactDev* ic, const MultiMaps& 
   const int fb = m.blocks[MK::kFace];
   const int32_t* fo = m.off[MK::kFace];
   MultiClothPredKernel<<<XcdGrid(m.blocks[MK::kVert]), kBlock, 0, s>>>(ic, m.off[MK::kVert], m.n, x);
-  MultiClothGrowKernel<<<XcdGrid(fb), kBlock, 0, s>>>(ic, fo, m.n, x, x0);
-  MultiClothBottomUpKernel<<<m.n, 1024, 0, s>>>(ic);
-  MultiPackClothKernel<<<XcdGrid(fb), kBlock, 0, s>>>(ic, fo, m.n);
+  MultiClothMergeKernel<<<XcdGrid(m.blocks[MK::kChunk]), kMergeChunk, 0, s>>>(ic, m.off[MK::kChunk], m.n, x, x0);
+  if (m.cloth_top) MultiClothMergeTopKernel<<<m.n, 1024, 0, s>>>(ic);
   if (!Empty(m, MK::kObsFace))
-    MultiPackObsKernel<<<XcdGrid(m.blocks[MK::kObsFace]), kBlock, 0, s>>>(ic, m.off[MK::kObsFace], m.n);
+    MultiObsFacesKernel<<<XcdGrid(m.blocks[MK::kObsFace]), kBlock, 0, s>>>(ic, m.off[MK::kObsFace], m.n);
   // obstacle pass, then the cloth pass, whose emit follows the totals (it knows whether the
   // item lists will be used)
   for (int self = 0; self < 2; ++self) {
@@ -1759,8 +1737,14 @@ hipError_t MultiEeSolve(hipStream_t s, const InstContactDev* ic, const MultiMaps
 }
 
 hipError_t MultiBuildMerge(hipStream_t s, const InstContactDev* ic, const MultiMaps& m, bool cloth) {
-  if (m.n <= 0) return hipSuccess;
-  MultiBuildMergeKernel<<<2 * m.n, 1024, 0, s>>>(ic, m.n, cloth ? 1 : 0);
+  if (cloth && !Empty(m, MK::kChunk)) {
+    MultiClothMergeKernel<<<XcdGrid(m.blocks[MK::kChunk]), kMergeChunk, 0, s>>>(ic, m.off[MK::kChunk], m.n, nullptr, nullptr);
+    if (m.cloth_top) MultiClothMergeTopKernel<<<m.n, 1024, 0, s>>>(ic);
+  }
+  if (!Empty(m, MK::kObsChunk)) {
+    MultiObsMergeKernel<<<XcdGrid(m.blocks[MK::kObsChunk]), kMergeChunk, 0, s>>>(ic, m.off[MK::kObsChunk], m.n, 0);
+    if (m.obs_top) MultiObsMergeTopKernel<<<m.n, 1024, 0, s>>>(ic);
+  }
   return hipGetLastError();
 }
 

@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "bvh_device.h"
 #include "contact.h"
 #include "context.h"
 #include "dynamics.h"
@@ -427,8 +428,9 @@ int MultiContactSetup(xrt_ctx* ctx) {
   std::vector<InstContactDev> ic(std::max(n, 1));
   std::vector<int32_t> off(MultiMaps::kKinds * static_cast<size_t>(n + 1), 0);
   auto blocks = [](int count) { return (count + 255) / 256; };
+  bool cloth_top = false, obs_top = false;
   for (int k = 0; k < n; ++k) {
-    int cnt[MultiMaps::kKinds] = {0, 0, 0, 0, 0, 0};
+    int cnt[MultiMaps::kKinds] = {};
     if (ctx->contact[k]) {
       HostInstance& h = ctx->inst[k];
       ContactData& c = *ctx->contact[k];
@@ -478,6 +480,10 @@ int MultiContactSetup(xrt_ctx* ctx) {
       cnt[MultiMaps::kObsFace] = blocks(c.obs_nf);
       // repulsion: about 4 pairs per thread at the usual ~16 pairs per face
       cnt[MultiMaps::kPair] = std::max(1, (16 * h.nt + 1023) / 1024);
+      cnt[MultiMaps::kChunk] = (h.nt + kMergeChunk - 1) / kMergeChunk;
+      cnt[MultiMaps::kObsChunk] = (c.obs_nf + kMergeChunk - 1) / kMergeChunk;
+      cloth_top = cloth_top || cnt[MultiMaps::kChunk] > 1;
+      obs_top = obs_top || cnt[MultiMaps::kObsChunk] > 1;
     }
     for (int kind = 0; kind < MultiMaps::kKinds; ++kind) {
       int32_t* o = off.data() + static_cast<size_t>(kind) * (n + 1);
@@ -512,6 +518,8 @@ int MultiContactSetup(xrt_ctx* ctx) {
     XRT_CHECK_HIP(ctx->obs_trees.Setup(ot, ox, ctx->stream));
   }
   ctx->maps.n = n;
+  ctx->maps.cloth_top = cloth_top;
+  ctx->maps.obs_top = obs_top;
   for (int kind = 0; kind < MultiMaps::kKinds; ++kind) {
     ctx->maps.off[kind] = ctx->ic_off.ptr + seg[kind];
     ctx->maps.blocks[kind] = off[static_cast<size_t>(kind) * (n + 1) + n];
