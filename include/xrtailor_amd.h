@@ -474,7 +474,8 @@ int xrt_adjoint_substep(xrt_ctx* ctx);
 int xrt_time_adjoint(xrt_ctx* ctx, int32_t n, float ms[3]);
 /* Runs n batched substeps (not captured) with HIP events around every launch of the EE
  * repulsion kernel (one edge-edge test item per thread over every instance's item list)
- * and returns its average device time per launch; counts = EE items, VF items, stored
+ * and returns its average device time per launch; counts = EE items (an edge couple of the
+ * cloth is listed once for both orders), VF items, stored
  * pairs and instances on the item path, averaged over the n substeps' pair refreshes.  The
  * state advances by n substeps.  No counterpart in the reference (measurement hook; the EE
  * tests are EvaluateEEProximity, xrtailor/src/physics/repulsion/PBDRepulsion.cu:411-468). */

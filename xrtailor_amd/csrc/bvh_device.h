@@ -279,6 +279,45 @@ __device__ __forceinline__ void TraversePackedFace(const Box* __restrict__ pk,
   }
 }
 
+// A tree against itself, each couple of leaves once: lb is the record of leaf slot `slot`, and
+// the traversal enters at its escape, where the depth-first order goes on to the leaves of
+// higher slots.  on_leaf(rhs object, its face record, fwd, rev) for every such leaf that
+// TraversePackedFace would report for lb (fwd) or would report lb for (rev).  The two differ
+// only by the rounding of the dilation, so the nodes are tested with a box grown by more than
+// that rounding, and the exact tests are made at the leaves that are left.
+template <class OnLeaf>
+__device__ __forceinline__ void TraversePackedAfter(const Box* __restrict__ pk,
+                                                    const int4* __restrict__ lf, int nf,
+                                                    const Box& lb, float th, OnLeaf&& on_leaf) {
+  const int ni = nf - 1;
+  constexpr float kUlps = 4.76837158203125e-7f;  // 2^-21
+  Box wide = lb;
+  wide.lo.x -= kUlps * (fabsf(lb.lo.x) + fabsf(th));
+  wide.lo.y -= kUlps * (fabsf(lb.lo.y) + fabsf(th));
+  wide.lo.z -= kUlps * (fabsf(lb.lo.z) + fabsf(th));
+  wide.hi.x += kUlps * (fabsf(lb.hi.x) + fabsf(th));
+  wide.hi.y += kUlps * (fabsf(lb.hi.y) + fabsf(th));
+  wide.hi.z += kUlps * (fabsf(lb.hi.z) + fabsf(th));
+  int node = __float_as_int(lb.hi.w);
+  const int max_steps = 2 * nf;
+  for (int step = 0; node != -1 && step < max_steps; ++step) {
+    const Box b = pk[node];
+    const int4 f = node >= ni ? lf[node - ni] : make_int4(0, 0, 0, 0);
+    const int code = __float_as_int(b.lo.w), esc = __float_as_int(b.hi.w);
+    if (OverlapDilated(b, wide, th)) {
+      if (code < 0) {
+        const bool fwd = OverlapDilated(b, lb, th), rev = OverlapDilated(lb, b, th);
+        if (fwd || rev) on_leaf(-code - 1, f, fwd, rev);
+        node = esc;
+      } else {
+        node = code;
+      }
+    } else {
+      node = esc;
+    }
+  }
+}
+
 // CountPairs_Kernel (BVH.cu:1149-1179): rhs leaves overlapping lhs leaf id dilated by th
 __device__ __forceinline__ uint32_t CountPairsBody(const BvhView& l, const BvhView& r, float th,
                                                    int id) {

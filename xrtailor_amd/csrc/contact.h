@@ -147,6 +147,7 @@ struct InstContactDev {
 };
 
 constexpr int kPairStage = 128;
+constexpr int kCoupleStage = 64;  // couples of cloth faces: two words each in the same memory
 constexpr int kStageObjBits = 20;  // the item mask (12 bits) takes the rest of a stage entry
 
 // block -> instance maps: per kind, the prefix sums (n + 1 entries, device) of the

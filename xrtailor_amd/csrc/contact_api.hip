@@ -713,7 +713,7 @@ int xrt_time_repulsion(xrt_ctx* ctx, int32_t n, float* avg_ms, int64_t counts[4]
         rc = XRT_ERR_HIP;
         break;
       }
-      sums[0] += sc[4];
+      sums[0] += sc[4];  // listed: an edge couple of the cloth once
       sums[1] += sc[3];
       sums[2] += std::min(sc[2], c->pair_cap);
       sums[3] += (c->ee_cap > 0 && sc[2] <= c->pair_cap && sc[4] <= c->ee_cap) ? 1 : 0;
