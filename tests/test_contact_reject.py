@@ -27,7 +27,7 @@ int main(int argc, char** argv) {
   long open_ee = 0, fail_ee = 0, rej_ee = 0, open_vf = 0, fail_vf = 0, rej_vf = 0, pass_ee = 0, pass_vf = 0;
   const float special[8] = {0.0f, -0.0f, NAN, INFINITY, -INFINITY, 1e-42f, 3e38f, -1e20f};
   for (long i = 0; i < n; ++i) {
-    const int kind = static_cast<int>(i % 8);
+    const int kind = static_cast<int>(i % 9);
     const double scale = std::pow(10.0, U(-8, 4)), off = kind == 7 ? std::pow(10.0, U(-2, 3)) * scale : 0.0;
     P o = R(off);
     P x0 = R(scale), e = R(scale), x1, y0, y1, y2;
@@ -46,6 +46,10 @@ int main(int argc, char** argv) {
       f.y = 0;
     }
     if (kind == 4) y0 = Add(x0, R(scale), tiny);  // nearly shared vertex
+    if (kind == 8) {  // all in a line but for tiny, apart or overlapping, of unlike lengths
+      f = Add(P{0, 0, 0}, Add(e, R(scale), tiny), std::pow(10.0, U(-4, 4)));
+      y0 = Add(Add(x0, e, U(-3, 3)), R(scale), tiny * std::pow(10.0, U(-3, 0)));
+    }
     y1 = Add(y0, f);
     y2 = Add(y0, R(scale));
     if (kind == 6) y2 = Add(y0, Add(f, R(scale), tiny), U(-1, 2));  // sliver
@@ -57,6 +61,10 @@ int main(int argc, char** argv) {
     const bool ee = EESigns(a, b, p[0], p[1], p[2], p[3], false, Nz(S(p[1], p[0])), Nz(S(p[3], p[2])), num);
     const bool er = EeReject(p[0], p[1], p[2], p[3]);
     if (ee && er) { printf("EE rejected but passes, kind %d case %ld\n", kind, i); return 1; }
+    if (er && EESigns(b, a, p[2], p[3], p[0], p[1], false, Nz(S(p[3], p[2])), Nz(S(p[1], p[0])), num)) {
+      printf("EE rejected but passes the other way round, kind %d case %ld\n", kind, i);
+      return 1;
+    }
     pass_ee += ee; fail_ee += !ee; rej_ee += er; open_ee += !er && !ee;
     // the vertex near an edge or a corner of the face, or anywhere
     P v = x0;

@@ -49,3 +49,28 @@ def test_couples_match_plain(noise, cap, items):
         assert ca["pairs"] == cb["pairs"]
         per_face.append(ca["pairs"] / len(sp.tris))
     print("  pairs per face", per_face, flush=True)
+
+
+# an obstacle of 2^16 vertices (items listed by 16-bit vertex ids) and one of more (by edges)
+@pytest.mark.parametrize("side", [256, 257])
+def test_large_obstacle_matches_plain(side):
+    print(f"case obstacle of {side} x {side} vertices", flush=True)
+    pos, tris = scenes.grid(side, 1.5)
+    pos = pos.astype(np.float32)
+    pos[:, 1] = -0.001 + 0.0005 * np.sin(40.0 * pos[:, 0])
+    sp = _crumpled(17, 4, 0.05)
+    sp = scenes.ClothSpec(sp.pos, sp.tris, sp.pinned, 1e-8, 1e-4, sp.x0, (pos, tris))
+    xp = make_params(bend_model=1, enable_self_contact=1, enable_obstacle_contact=1,
+                     ground_height=-1.0, num_substeps=2, num_iterations=3, num_collision_passes=3,
+                     pair_update_interval=2, pair_capacity_per_face=4096,
+                     repulsion_vf_items_per_face=4096, repulsion_ee_items_per_face=8192)
+    a, ia = build_solver([sp], xp, seed=3)
+    b, ib = build_solver([sp], xp, seed=3)
+    for _ in range(2):
+        a.SubstepBatched()
+        b.SubstepPlain(ib[0])
+    a.sync()
+    for u, v in zip(a.GetState(ia[0]), b.GetState(ib[0])):
+        np.testing.assert_array_equal(u, v)
+    c = a.Contacts(ia[0])
+    assert c["pairs"] == b.Contacts(ib[0])["pairs"] and c["obs_pairs"] > 1000

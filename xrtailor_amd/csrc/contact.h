@@ -2,7 +2,8 @@
 //
 // Per-mesh contact topology (instance-local ids):
 //   tris int4[F], edges int2[E], face_edges int4[F] (edge of nodes i,i+1), ef_ptr/ef CSR
-//   (faces per edge, ascending, <= 4 used), face_n float4[F] rest face normals,
+//   (faces per edge, ascending, <= 4 used), edge_n float4[4 E] rest normals of
+//   those faces (w of the first: how many),
 //   rtri u32[F] representative-triangle bits (vertex i: bit i, edge i: bit 3+i),
 //   trir int4[F] = (tris.xyz, rtri)
 // Contact records (per cloth vertex / edge):
@@ -26,7 +27,7 @@ struct MeshTopo {
   const int4* face_edges = nullptr;
   const int32_t* ef_ptr = nullptr;
   const int32_t* ef = nullptr;
-  const float4* face_n = nullptr;
+  const float4* edge_n = nullptr;  // 4 per edge
   const uint32_t* rtri = nullptr;
   const int4* trir = nullptr;  // (vertices, rtri bits) per face: one load for the item masks
 };
@@ -131,6 +132,10 @@ struct InstContactDev {
   int vf_cap = 0, ee_cap = 0;
   int2* rep_vf = nullptr;
   int2* rep_ee = nullptr;
+  // the items' vertices, 16 bits each, of cloths and obstacles of up to 2^16 vertices (else
+  // null): VF node, t.x, t.y, t.z; EE the two of the cloth edge, the two of the other
+  uint2* ids_vf = nullptr;
+  uint2* ids_ee = nullptr;
   uint32_t* ivf = nullptr;
   uint32_t* iee = nullptr;
   uint2* nitem = nullptr;

@@ -322,17 +322,16 @@ __device__ F3 EdgeNormal(const RMesh& m, int e) {  // Edge::ComputeNormal (Edge.
   return cnt ? M(sum, 1.0f / static_cast<float>(cnt)) : sum;
 }
 
-__device__ bool InEdge(float w, const RMesh& m0, int e0, const RMesh& m1, int e1) {
-  const int2 a = m0.t.edges[e0];
-  const F3 x = A(M(m0.X(a.x), 1 - w), M(m0.X(a.y), w));  // BasicPrimitiveTests.cu:286-301
-  bool in = true;
-  const int2 b = m1.t.edges[e1];
-  const F3 n0 = m1.X(b.x), n1 = m1.X(b.y);
-  int cnt = 0;
-  for (int k = m1.t.ef_ptr[e1]; k < m1.t.ef_ptr[e1 + 1] && cnt < 4; ++k, ++cnt) {
-    const F3 fn = L3(m1.t.face_n[m1.t.ef[k]]);
-    in &= Mixed(S(n1, n0), fn, S(x, n0)) >= 0;
-  }
+// x against edge e (vertices at n0, n1) of m (BasicPrimitiveTests.cu:286-301).  One edge couple
+// in fifty of those that get here passes, so the edge's normals lie side by side: through the
+// edge's face list they took three dependent loads
+__device__ __forceinline__ bool InEdge(F3 x, const RMesh& m, int e, F3 n0, F3 n1) {
+  const float4* en = m.t.edge_n + 4 * static_cast<int64_t>(e);
+  const float4 first = en[0];
+  const int cnt = static_cast<int>(first.w);
+  const F3 d = S(n1, n0), r = S(x, n0);
+  bool in = cnt < 1 || Mixed(d, L3(first), r) >= 0;
+  for (int k = 1; k < cnt && in; ++k) in = Mixed(d, L3(en[k]), r) >= 0;
   return in;
 }
 
@@ -429,7 +428,10 @@ __device__ void EEResponse(const RMesh& c, int2 a, const RMesh& o, int2 b, F3 x0
                            F3 y1, int e0, int e1, float h, float4 w4, long long* dq,
                            int32_t* cnt, RepOut* out = nullptr) {
   float bw[4] = {w4.x, w4.y, w4.z, w4.w};
-  if (!(InEdge(bw[1], c, e0, o, e1) && InEdge(-bw[3], o, e1, c, e0))) return;
+  const F3 xa = A(M(x0, 1 - bw[1]), M(x1, bw[1]));
+  if (!InEdge(xa, o, e1, y0, y1)) return;
+  const F3 yb = A(M(y0, 1 + bw[3]), M(y1, -bw[3]));
+  if (!InEdge(yb, c, e0, x0, x1)) return;
   float w[4];
   F3 pn;
   const float d0 = SignedEE(c.X0(a.x), c.X0(a.y), o.X0(b.x), o.X0(b.y), pn, w);
@@ -696,6 +698,25 @@ __device__ __forceinline__ bool ItemOpen(const RMesh& c, const RMesh& o, int2 it
     return !VfReject(L3(Gld(c.s.x + it.x)), L3(Gld(ox + tr.x)), L3(Gld(ox + tr.y)),
                      L3(Gld(ox + tr.z)));
   }
+}
+
+// ItemOpen of an item given by its vertices (InstContactDev::ids_ee / ids_vf)
+template <int is_ee>
+__device__ __forceinline__ bool IdsOpen(const RMesh& c, const RMesh& o, uint2 v, bool self) {
+  const int a = v.x & 0xffffu, b = v.x >> 16, d = v.y & 0xffffu, e = v.y >> 16;
+  const float4* ox = self ? c.s.x : o.s.x;
+  const int onv = self ? c.t.nv : o.t.nv;
+  if constexpr (is_ee) {
+    if (max(a, b) >= c.t.nv || max(d, e) >= onv) return false;
+    return !EeReject(L3(Gld(c.s.x + a)), L3(Gld(c.s.x + b)), L3(Gld(ox + d)), L3(Gld(ox + e)));
+  } else {
+    if (a >= c.t.nv || max(b, max(d, e)) >= onv) return false;
+    return !VfReject(L3(Gld(c.s.x + a)), L3(Gld(ox + b)), L3(Gld(ox + d)), L3(Gld(ox + e)));
+  }
+}
+__device__ __forceinline__ uint2 PackIds(int a, int b, int d, int e) {
+  return make_uint2(static_cast<uint32_t>(a) | static_cast<uint32_t>(b) << 16,
+                    static_cast<uint32_t>(d) | static_cast<uint32_t>(e) << 16);
 }
 
 // (e1, e0) of a listed cloth-cloth EE item that stands for both
@@ -1127,8 +1148,7 @@ __device__ __forceinline__ int Pick3(int4 v, int q) { return q == 0 ? v.x : (q =
 // Item layout: the 64 leaves of a wave own the contiguous range of their item counts from
 // the first leaf's offset.  The staged leaves' items fill its front in (hit j, lane, bit)
 // order: per hit index the wave takes an exclusive sum of its lanes' item counts, so each
-// store instruction writes neighbouring slots instead of 64 scattered ones (one thread per
-// leaf writing its own run took 2.0 ms per cloth pass, 0.9 ms without those stores).  The
+// store instruction writes neighbouring slots instead of 64 scattered ones.  The
 // traversed leaves' items follow, each leaf's in its hit order.  The lists hold the same
 // items as the reference's per-pair tests; the repulsion sums are fixed point, so the order
 // of the items cannot change a result bit.
@@ -1148,54 +1168,57 @@ __device__ __forceinline__ EmitRanges WaveRanges(const InstContactDev& c, int se
   return r;
 }
 
+// the vertices of edge q of face f
+__device__ __forceinline__ int2 FaceEdge(int4 f, int q) {
+  return q == 0 ? make_int2(f.x, f.y) : (q == 1 ? make_int2(f.y, f.z) : make_int2(f.z, f.x));
+}
+__device__ __forceinline__ void PutVf(const InstContactDev& c, int64_t q, int node, int face, int4 f) {
+  if (q >= c.vf_cap) return;
+  c.rep_vf[q] = make_int2(node, face);
+  if (c.ids_vf) c.ids_vf[q] = PackIds(node, f.x, f.y, f.z);
+}
+__device__ __forceinline__ void PutEe(const InstContactDev& c, int64_t q, int e0, int e1, int2 v0,
+                                      int2 v1) {
+  if (q >= c.ee_cap) return;
+  c.rep_ee[q] = make_int2(e0, e1);
+  if (c.ids_ee) c.ids_ee[q] = PackIds(v0.x, v0.y, v1.x, v1.y);
+}
+
 // the items of pair (lobj, robj) with item mask m, to slots qv, qe on
 __device__ __forceinline__ void PutPairItems(const InstContactDev& c, uint32_t m, int4 f0, int4 fe0,
                                              int robj, int64_t qv, int64_t qe) {
+  const int4 f1 = c.obs.tris[robj];
 #pragma unroll
   for (int q = 0; q < 3; ++q)
-    if ((m >> q) & 1u) {
-      if (qv < c.vf_cap) c.rep_vf[qv] = make_int2(Pick3(f0, q), robj);
-      ++qv;
-    }
+    if ((m >> q) & 1u) PutVf(c, qv++, Pick3(f0, q), robj, f1);
   if (!(m >> 3)) return;
   const int4 fe1 = c.obs.face_edges[robj];
 #pragma unroll
   for (int q = 0; q < 9; ++q)
-    if ((m >> (3 + q)) & 1u) {
-      if (qe < c.ee_cap) c.rep_ee[qe] = make_int2(Pick3(fe0, q / 3), Pick3(fe1, q % 3));
-      ++qe;
-    }
+    if ((m >> (3 + q)) & 1u)
+      PutEe(c, qe++, Pick3(fe0, q / 3), Pick3(fe1, q % 3), FaceEdge(f0, q / 3), FaceEdge(f1, q % 3));
 }
 
-// the items of the couple of cloth faces (lobj, robj) with CoupleMask m; an edge couple that is
-// a pair in one direction only is listed as that pair's (cloth edge, edge)
-__device__ __forceinline__ void PutCoupleItems(const InstContactDev& c, uint32_t m, int lobj,
-                                               int4 f0, int4 fe0, int robj, int64_t qv, int64_t qe) {
+// The items of the couple of cloth faces (lobj, robj) with CoupleMask m, in the order of the
+// mask's bits: put_vf(node, face, the face's vertices), put_ee(e0, e1, their vertices).  An edge
+// couple that is a pair in one direction only is listed as that pair's (cloth edge, edge).
+template <class PutVfItem, class PutEeItem>
+__device__ __forceinline__ void CoupleItems(uint32_t m, int lobj, int4 f0, int4 fe0, int robj,
+                                            int4 f1, int4 fe1, PutVfItem&& put_vf,
+                                            PutEeItem&& put_ee) {
 #pragma unroll
   for (int q = 0; q < 3; ++q)
-    if ((m >> q) & 1u) {
-      if (qv < c.vf_cap) c.rep_vf[qv] = make_int2(Pick3(f0, q), robj | kSelfBit);
-      ++qv;
-    }
-  if ((m >> 3) & 7u) {
-    const int4 f1 = c.cloth.tris[robj];
+    if ((m >> q) & 1u) put_vf(Pick3(f0, q), robj | kSelfBit, f1);
 #pragma unroll
-    for (int q = 0; q < 3; ++q)
-      if ((m >> (3 + q)) & 1u) {
-        if (qv < c.vf_cap) c.rep_vf[qv] = make_int2(Pick3(f1, q), lobj | kSelfBit);
-        ++qv;
-      }
-  }
-  if (!((m >> 6) & 0x1ffu)) return;
-  const int4 fe1 = c.cloth.face_edges[robj];
+  for (int q = 0; q < 3; ++q)
+    if ((m >> (3 + q)) & 1u) put_vf(Pick3(f1, q), lobj | kSelfBit, f0);
   const bool fwd = (m & kCoupleFwd) != 0, rev = (m & kCoupleRev) != 0;
 #pragma unroll
   for (int q = 0; q < 9; ++q)
     if ((m >> (6 + q)) & 1u) {
       const int a = Pick3(fe0, q / 3), b = Pick3(fe1, q % 3);
-      if (qe < c.ee_cap)
-        c.rep_ee[qe] = make_int2((fwd ? a : b) | (fwd && rev ? kBothBit : 0), (fwd ? b : a) | kSelfBit);
-      ++qe;
+      put_ee((fwd ? a : b) | (fwd && rev ? kBothBit : 0), (fwd ? b : a) | kSelfBit,
+             FaceEdge(f0, q / 3), FaceEdge(f1, q % 3));
     }
 }
 
@@ -1264,7 +1287,11 @@ __device__ __forceinline__ void EmitDirected(const InstContactDev& c, int self, 
                  });
 }
 
-// the cloth pass over the couples of the count pass
+// The cloth pass over the couples of the count pass.  The items of one step of a wave (hit j of
+// its 64 leaves) are laid out in LDS and written from there by neighboring lanes: each lane
+// storing its own, 16 bytes an item, took 1.99 ms for 256 cloths, this way 1.71 ms (97 and 64 us
+// for one of 130 k faces).
+constexpr uint32_t kEmitChunk = 192;
 __device__ __forceinline__ void EmitCouples(const InstContactDev& c, int blk, int i, int i0, float th) {
   const bool leaf = i < c.nf;
   const bool store = !(ItemsUsable(c, 0) && ItemsUsable(c, 1));
@@ -1298,6 +1325,9 @@ __device__ __forceinline__ void EmitCouples(const InstContactDev& c, int blk, in
   EmitRanges r = WaveRanges(c, 1, blk, i0, nb, staged, trav, nit);
   const uint2* st = reinterpret_cast<const uint2*>(c.stage) + i;
   const uint32_t jn = WaveMax(staged ? cnt : 0u);
+  __shared__ int4 buf[kBlock / 64][kEmitChunk];
+  int4* out = buf[threadIdx.x >> 6];
+  const uint32_t lane = threadIdx.x & 63;
   for (uint32_t j = 0; j < jn; ++j) {
     uint2 se = make_uint2(0, 0);
     if (staged && j < cnt) se = st[static_cast<int64_t>(j) * c.nf];
@@ -1307,19 +1337,56 @@ __device__ __forceinline__ void EmitCouples(const InstContactDev& c, int blk, in
     uint32_t tot;
     const uint32_t pre =
         WaveExclusiveSum(__popc(m & kCoupleVf) | (__popc((m >> 6) & 0x1ffu) << 16), &tot);
-    if (m & 0x7fffu)
-      PutCoupleItems(c, m, lobj, f0, fe0, robj, r.pv + (pre & 0xffffu), r.pe + (pre >> 16));
-    r.pv += tot & 0xffffu;
-    r.pe += tot >> 16;
+    const uint32_t tv = tot & 0xffffu, te = tot >> 16;
+    int4 f1 = make_int4(0, 0, 0, 0), fe1 = f1;
+    if (m & 0x7fffu) {
+      f1 = c.cloth.tris[robj];
+      fe1 = c.cloth.face_edges[robj];
+    }
+    // the step's VF items, then its EE items, kEmitChunk at a time
+    for (uint32_t base = 0; base < tv + te; base += kEmitChunk) {
+      uint32_t v = (pre & 0xffffu) - base, e = tv + (pre >> 16) - base;  // (wraps below base)
+      CoupleItems(m, lobj, f0, fe0, robj, f1, fe1,
+                  [&](int node, int face, int4 f) {
+                    const uint2 ids = PackIds(node, f.x, f.y, f.z);
+                    if (v < kEmitChunk)
+                      out[v] = make_int4(node, face, static_cast<int>(ids.x), static_cast<int>(ids.y));
+                    ++v;
+                  },
+                  [&](int e0, int e1, int2 v0, int2 v1) {
+                    const uint2 ids = PackIds(v0.x, v0.y, v1.x, v1.y);
+                    if (e < kEmitChunk)
+                      out[e] = make_int4(e0, e1, static_cast<int>(ids.x), static_cast<int>(ids.y));
+                    ++e;
+                  });
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      for (uint32_t t = lane; t < min(static_cast<uint32_t>(kEmitChunk), tv + te - base); t += 64) {
+        const int4 rec = out[t];
+        const bool is_vf = base + t < tv;
+        const int64_t slot = is_vf ? r.pv + base + t : r.pe + (base + t - tv);
+        if (slot >= (is_vf ? c.vf_cap : c.ee_cap)) continue;
+        (is_vf ? c.rep_vf : c.rep_ee)[slot] = make_int2(rec.x, rec.y);
+        if (c.ids_vf)
+          (is_vf ? c.ids_vf : c.ids_ee)[slot] =
+              make_uint2(static_cast<uint32_t>(rec.z), static_cast<uint32_t>(rec.w));
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    r.pv += tv;
+    r.pe += te;
   }
   if (!trav) return;
   TraversePackedAfter(c.cbvh.packed, c.cbvh.leaf_face, c.nf, lb, th,
                       [&](int robj, int4 f1, bool fwd, bool rev) {
                         const uint32_t m = CoupleMask(f0, f1, fwd, rev);
                         if (store) put_pairs(m, robj);
-                        PutCoupleItems(c, m, lobj, f0, fe0, robj, r.tv, r.te);
-                        r.tv += __popc(m & kCoupleVf);
-                        r.te += __popc((m >> 6) & 0x1ffu);
+                        CoupleItems(m, lobj, f0, fe0, robj, f1, c.cloth.face_edges[robj],
+                                    [&](int node, int face, int4 f) { PutVf(c, r.tv++, node, face, f); },
+                                    [&](int e0, int e1, int2 v0, int2 v1) {
+                                      PutEe(c, r.te++, e0, e1, v0, v1);
+                                    });
                       });
 }
 
@@ -1355,14 +1422,16 @@ __global__ __launch_bounds__(kBlock) void MultiAddTotalsKernel(const InstContact
 
 // repulsion tests of every instance, one VF (is_ee = 0) or EE item per thread; instances
 // whose list is not usable (off, overflowed, or pairs beyond the pair capacity) are left to
-// MultiRepPairsKernel.  A wave takes 64 items per step; the few that ItemOpen leaves are queued
+// MultiRepPairsKernel.  A wave takes 64 items per step; the few that are left open are queued
 // in LDS and evaluated 64 at a time (and at the end), so that the long evaluation does not run
 // in every step for one or two lanes.  The sums are fixed point: the order changes nothing.
-// Eight waves per SIMD (64 VGPRs, the spills in the evaluation).  The L1 lookups of the gathers
-// (item -> edges -> positions) bound it: 33 a load instruction, one a cycle, busy for 83 % of the
-// launch.
+// Bound by the L1 lookups of the gathers (33 a load instruction, one a cycle: busy for 83 % of the
+// launch), so an item comes as the 16-bit ids of its vertices where the meshes are small enough:
+// four gathers, without the edges' or the face's.  63 M EE and 31 M VF items of 256 cloths: 709 ->
+// 426 and 228 -> 173 us (with the sharper EeReject and the longer blocks that MultiContactSetup
+// chooses).  Six waves a SIMD for EE, eight for VF: five 473 / 183, six 425 / 183, eight 437 / 173.
 template <int is_ee>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(is_ee ? 6 : 8))) void
 MultiRepItemKernel(const InstContactDev* ic, const int32_t* off, int n,
                    const float4* __restrict__ x, const float4* __restrict__ x0, float h) {
   const int lblk = XcdBlock(off, n);
@@ -1375,28 +1444,35 @@ MultiRepItemKernel(const InstContactDev* ic, const int32_t* off, int n,
   const RMesh cm{c.cloth, MeshState{x + c.vbeg, x0 + c.vbeg, -1.0f}};
   const RMesh om{c.obs, MeshState{c.o_x, c.o_x0, 1e-3f}};  // obstacle nodes: inv mass 1e-3
   const int2* items = is_ee ? c.rep_ee : c.rep_vf;
-  __shared__ int2 queue[kBlock / 64][is_ee ? 192 : 128];
+  const uint2* ids = is_ee ? c.ids_ee : c.ids_vf;
+  const int nobs = c.scal[is_ee ? 6 : 5];  // the obstacle items come first
+  __shared__ int queue[kBlock / 64][is_ee ? 192 : 128];  // item index, the sign bit: mirrored
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  int2* qw = queue[w];
-  int qn = 0;  // queued items (the same in every lane)
+  int* qw = queue[w];
+  int qn = 0;  // queued entries (the same in every lane)
   int base = (lblk - off[k]) * kBlock + w * 64;
   const int stride = nblk * kBlock;
   while (true) {
     const bool have = base < cnt;  // uniform over the wave
     if (have) {
       const int qi = base + lane;
-      int2 it = make_int2(-1, 0);
-      if (qi < cnt) it = Gld(items + qi);
-      const bool open =
-          qi < cnt && ItemOpen<is_ee>(cm, om, make_int2(is_ee ? it.x & 0x7fffffff : it.x, it.y));
+      bool open = false;
+      if (qi < cnt) {
+        if (ids) {
+          open = IdsOpen<is_ee>(cm, om, Gld(ids + qi), qi >= nobs);
+        } else {
+          const int2 it = Gld(items + qi);
+          open = ItemOpen<is_ee>(cm, om, make_int2(is_ee ? it.x & 0x7fffffff : it.x, it.y));
+        }
+      }
       const uint64_t m = __ballot(open);
-      if (open) qw[qn + __popcll(m & below)] = make_int2(it.x & 0x7fffffff, it.y);
+      if (open) qw[qn + __popcll(m & below)] = qi;
       qn += __popcll(m);
-      if (is_ee) {  // the same two edges the other way round
-        const bool both = open && it.x < 0;  // (kBothBit)
+      if (is_ee) {
+        const bool both = open && qi >= nobs;
         const uint64_t mb = __ballot(both);
-        if (both) qw[qn + __popcll(mb & below)] = MirrorItem(it);
+        if (both) qw[qn + __popcll(mb & below)] = qi | kBothBit;
         qn += __popcll(mb);
       }
       base += stride;
@@ -1404,7 +1480,14 @@ MultiRepItemKernel(const InstContactDev* ic, const int32_t* off, int n,
     }
     while (qn >= 64 || (!have && qn > 0)) {
       const int take = qn < 64 ? qn : 64;
-      if (lane < take) ItemEval<is_ee>(cm, om, qw[qn - take + lane], h, c.dq, c.cnt);
+      if (lane < take) {
+        const int e = qw[qn - take + lane];
+        int2 it = items[e & 0x7fffffff];
+        const bool listed = e >= 0 || it.x < 0;  // (kBothBit)
+        if (e < 0) it = MirrorItem(it);
+        if (is_ee) it.x &= 0x7fffffff;
+        if (listed) ItemEval<is_ee>(cm, om, it, h, c.dq, c.cnt);
+      }
       qn -= take;
       __builtin_amdgcn_wave_barrier();
     }

@@ -37,15 +37,23 @@ int UploadTopo(const ContactTopo& t, const std::vector<int32_t>& tris,
                DevBuf<float4>& dn, DevBuf<uint32_t>& dr, DevBuf<int4>& dtr, hipStream_t s) {
   const int nt = static_cast<int>(tris.size() / 3), ne = static_cast<int>(edges.size() / 2);
   std::vector<int4> t4(std::max(nt, 1)), fe4(std::max(nt, 1)), tr4(std::max(nt, 1));
-  std::vector<float4> n4(std::max(nt, 1));
+  std::vector<float4> n4(4 * static_cast<size_t>(std::max(ne, 1)), make_float4(0, 0, 0, 0));
   for (int f = 0; f < nt; ++f) {
     t4[f] = make_int4(tris[3 * f], tris[3 * f + 1], tris[3 * f + 2], 0);
     tr4[f] = make_int4(tris[3 * f], tris[3 * f + 1], tris[3 * f + 2], static_cast<int>(t.rtri[f]));
     fe4[f] = make_int4(t.face_edges[3 * f], t.face_edges[3 * f + 1], t.face_edges[3 * f + 2], 0);
-    n4[f] = make_float4(t.face_n[3 * f], t.face_n[3 * f + 1], t.face_n[3 * f + 2], 0.0f);
   }
   std::vector<int2> e2(std::max(ne, 1));
-  for (int e = 0; e < ne; ++e) e2[e] = make_int2(edges[2 * e], edges[2 * e + 1]);
+  for (int e = 0; e < ne; ++e) {
+    e2[e] = make_int2(edges[2 * e], edges[2 * e + 1]);
+    const int cnt = std::min(4, t.ef_ptr[e + 1] - t.ef_ptr[e]);
+    float4* en = n4.data() + 4 * static_cast<size_t>(e);
+    for (int k = 0; k < cnt; ++k) {
+      const float* fn = t.face_n.data() + 3 * static_cast<size_t>(t.ef[t.ef_ptr[e] + k]);
+      en[k] = make_float4(fn[0], fn[1], fn[2], 0.0f);
+    }
+    en[0].w = static_cast<float>(cnt);
+  }
   XRT_CHECK_HIP(dt.Upload(t4, s));
   XRT_CHECK_HIP(dfe.Upload(fe4, s));
   XRT_CHECK_HIP(dn.Upload(n4, s));
@@ -67,7 +75,7 @@ MeshTopo ClothTopo(const ContactData& c, const HostInstance& h) {
   t.face_edges = c.c_fe.ptr;
   t.ef_ptr = c.c_ef_ptr.ptr;
   t.ef = c.c_ef.ptr;
-  t.face_n = c.c_face_n.ptr;
+  t.edge_n = c.c_edge_n.ptr;
   t.rtri = c.c_rtri.ptr;
   t.trir = c.c_trir.ptr;
   return t;
@@ -83,7 +91,7 @@ MeshTopo ObsTopo(const ContactData& c) {
   t.face_edges = c.o_fe.ptr;
   t.ef_ptr = c.o_ef_ptr.ptr;
   t.ef = c.o_ef.ptr;
-  t.face_n = c.o_face_n.ptr;
+  t.edge_n = c.o_edge_n.ptr;
   t.rtri = c.o_rtri.ptr;
   t.trir = c.o_trir.ptr;
   return t;
@@ -122,12 +130,18 @@ int AllocPairLists(xrt_ctx* ctx, const HostInstance& h, ContactData& c) {
   c.vf_cap = c.ee_cap = 0;
   c.rep_vf.Free();
   c.rep_ee.Free();
+  c.ids_vf.Free();
+  c.ids_ee.Free();
   if (ctx->params.enable_self_contact && vf_cap > 0 && ee_cap > 0 &&
       9 * static_cast<int64_t>(c.pair_cap) <= static_cast<int64_t>(INT32_MAX)) {
     c.vf_cap = static_cast<int>(std::min<int64_t>(vf_cap, 3 * static_cast<int64_t>(c.pair_cap)));
     c.ee_cap = static_cast<int>(std::min<int64_t>(ee_cap, 9 * static_cast<int64_t>(c.pair_cap)));
     XRT_CHECK_HIP(c.rep_vf.Alloc(c.vf_cap));
     XRT_CHECK_HIP(c.rep_ee.Alloc(c.ee_cap));
+    if (std::max(h.nv, h.obs_nv()) <= 1 << 16) {
+      XRT_CHECK_HIP(c.ids_vf.Alloc(c.vf_cap));
+      XRT_CHECK_HIP(c.ids_ee.Alloc(c.ee_cap));
+    }
     if (!c.ivf.ptr) XRT_CHECK_HIP(c.ivf.Alloc(std::max(h.nt, 1)));
     if (!c.iee.ptr) XRT_CHECK_HIP(c.iee.Alloc(std::max(h.nt, 1)));
     if (!c.nitem.ptr) XRT_CHECK_HIP(c.nitem.Alloc(std::max(h.nt, 1)));
@@ -147,7 +161,7 @@ int ContactStart(xrt_ctx* ctx) {
     auto c = std::make_unique<ContactData>();
     h.cloth_topo = BuildContactTopo(h.rest_pos.data(), h.nv, h.tris.data(), h.nt, h.edges);
     int rc = UploadTopo(h.cloth_topo, h.tris, h.edges, c->c_tris, c->c_fe, c->c_edges, c->c_ef_ptr,
-                        c->c_ef, c->c_face_n, c->c_rtri, c->c_trir, s);
+                        c->c_ef, c->c_edge_n, c->c_rtri, c->c_trir, s);
     if (rc != XRT_OK) return rc;
     XRT_CHECK_HIP(c->cloth_bvh.Setup(h.tris.data(), h.nt, h.nv, s));
     if (h.obs_nt() > 0) {
@@ -157,7 +171,7 @@ int ContactStart(xrt_ctx* ctx) {
       h.obs_topo = BuildContactTopo(h.obs_pos.data(), c->obs_nv, h.obs_tris.data(), c->obs_nf,
                                     h.obs_edges);
       rc = UploadTopo(h.obs_topo, h.obs_tris, h.obs_edges, c->o_tris, c->o_fe, c->o_edges,
-                      c->o_ef_ptr, c->o_ef, c->o_face_n, c->o_rtri, c->o_trir, s);
+                      c->o_ef_ptr, c->o_ef, c->o_edge_n, c->o_rtri, c->o_trir, s);
       if (rc != XRT_OK) return rc;
       const std::vector<float4> p = ToF4(h.obs_pos);
       XRT_CHECK_HIP(c->o_x0.Upload(p, s));
@@ -429,6 +443,17 @@ int MultiContactSetup(xrt_ctx* ctx) {
   std::vector<int32_t> off(MultiMaps::kKinds * static_cast<size_t>(n + 1), 0);
   auto blocks = [](int count) { return (count + 255) / 256; };
   bool cloth_top = false, obs_top = false;
+  // Repulsion blocks per 1024 faces (about 13 EE items a face).  16 give every wave about 200 items,
+  // which is little beside what a block costs to start and to evaluate its open items; from 16
+  // blocks a CU on the blocks grow, down to 3 per 1024 faces: more items per wave (2: no faster)
+  // would only spread the resident blocks over more cloths than the L2 holds.  EE / VF launches,
+  // us, at 2, 4, 8, 16, 32 blocks per 1024 faces: 5.0 M faces 432 / 178, 443 / 170, 496 / 174,
+  // 616 / 199, 794 / 258; 130 k faces 36 / 16, 24 / 13, 20 / 9, 18 / 9, 23 / 10.
+  int64_t faces = 0;
+  for (int k = 0; k < n; ++k)
+    if (ctx->contact[k]) faces += ctx->inst[k].nt;
+  const double per_kface = std::min(
+      16.0, std::max(3.0, 16.0 * 1024.0 * ctx->cu_count / static_cast<double>(std::max<int64_t>(faces, 1))));
   for (int k = 0; k < n; ++k) {
     int cnt[MultiMaps::kKinds] = {};
     if (ctx->contact[k]) {
@@ -467,6 +492,8 @@ int MultiContactSetup(xrt_ctx* ctx) {
       d.ee_cap = c.ee_cap;
       d.rep_vf = c.rep_vf.ptr;
       d.rep_ee = c.rep_ee.ptr;
+      d.ids_vf = c.ids_vf.ptr;
+      d.ids_ee = c.ids_ee.ptr;
       d.stage = c.stage.ptr;
       d.bsum = c.bsum.ptr;
       d.overflow = ctx->overflow.ptr;
@@ -478,8 +505,7 @@ int MultiContactSetup(xrt_ctx* ctx) {
       cnt[MultiMaps::kFace] = blocks(h.nt);
       cnt[MultiMaps::kObsVert] = blocks(c.obs_nv);
       cnt[MultiMaps::kObsFace] = blocks(c.obs_nf);
-      // repulsion: about 4 pairs per thread at the usual ~16 pairs per face
-      cnt[MultiMaps::kPair] = std::max(1, (16 * h.nt + 1023) / 1024);
+      cnt[MultiMaps::kPair] = std::max(1, static_cast<int>(std::ceil(per_kface * h.nt / 1024.0)));
       cnt[MultiMaps::kChunk] = (h.nt + kMergeChunk - 1) / kMergeChunk;
       cnt[MultiMaps::kObsChunk] = (c.obs_nf + kMergeChunk - 1) / kMergeChunk;
       cloth_top = cloth_top || cnt[MultiMaps::kChunk] > 1;

@@ -11,35 +11,58 @@
 //   b2, b1, b0 ~ s, t, q - s - t   with s = N.(d x e1), t = N.(e2 x d): one strict sign only
 //   if s > 0, t > 0 and s + t < q
 // EeReject / VfReject are true only where a product is beyond its bound by more than E, the
-// rounding of both evaluations: with u = 2^-24 and S = |ea| + |eb| + |d| (no difference of two
-// of the four points is longer) the products above are off by at most 16 u |ea| |eb| S^2 and
-// those of EESigns / VfSigns, scaled by |ea| |eb|, by at most 48 u |ea| |eb| S^2 (normalised
-// directions 6 u each, their cross product 20 u, the triple product 22 u more; VfSigns
-// normalises N once more, which scales value and error alike).
-// E = 192 u (|ea|^2 + |eb|^2) / 2 (|ea|^2 + |eb|^2 + |d|^2) >= 64 u |ea| |eb| S^2, and 1e-30 for
-// products that underflow.  NaN or infinite values compare false: nothing is rejected.
+// rounding of both evaluations; NaN or infinite values compare false: nothing is rejected.  With
+// u = 2^-24, S = |ea| + |eb| + |d| (no difference of two of the four points is longer), every
+// difference off by u relative, a product of three by 6 u, and la = |ea|, lb = |eb|:
+//   EE: with m = eb x d (p) or ea x d (r), |N| <= la lb.  EESigns takes a1, b1 as a cross product
+//   of length |m| and a0, b0 as one of at most |m| + |N|, off by 6 u S^2, times the normal, off by
+//   20 u (unit directions 6 u each); scaled by la lb that is 6 u |N| S^2 + 20 u la lb (|m| + |N|).
+//   The products here are off by 9 u la lb |m| + 6 u lb |d| |N| (p, r) and 15 u la lb |N| (q).
+//   In all less than u (17 |N| S^2 + 29 la lb |m|); E = u (144 |N| T + 32 L |m|) with L = la^2 + lb^2
+//   >= 2 la lb, T = L + |d|^2 >= S^2 / 3 is more than twice that, and 0.01 u L T covers the
+//   rounding of |N| >= 1e-3 la lb and of |m| themselves.  The bound shrinks with N and m: edges in
+//   one line, two apart on a grid line, are rejected too (with 96 u L T instead, 3.8 % of the items
+//   of 256 draped grids stayed open where 1.3 % pass EESigns).
+//   VF: the products are off by 16 u la lb S^2 and those of VfSigns, scaled by la lb, by
+//   48 u la lb S^2; E = 96 u L T >= 64 u la lb S^2.
+// and 1e-30 for products that underflow.
 // Both tests also fail where the two directions are parallel, |ua x ub|^2 < 1e-6; they are
 // rejected for it below 0.99e-6 (the rounding of both sides is 0.3 %).
 // Both are the same test with the two edges exchanged (p and r change places), so one answer
 // holds for an edge couple in either order.
-// A rejected item costs about 50 instructions instead of 225: the EE launch over the 130 M items
-// of 256 cloths went from 938 to 915 us, the VF launch over 32 M from 240 to 233 us (both are
-// bound by their gathers).
+// A rejected item costs about 60 instructions instead of 225, and what is left open three
+// dependent rounds of gathers more.
 #pragma once
+#include <cmath>
+
 #include "contact_math.h"
 
 namespace xrt {
 namespace cm {
 
+constexpr float kUnit = 1.0f / 16777216.0f;
 constexpr float kRejectErr = 192.0f * 0.5f / 16777216.0f;
+
+// within an ulp (the bounds have room for it)
+__device__ __forceinline__ float RootUp(float v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_sqrtf(v);
+#else
+  return std::sqrt(v);
+#endif
+}
 
 __device__ __forceinline__ bool EeReject(F3 x0, F3 x1, F3 y0, F3 y1) {
   const F3 ea = S(x1, x0), eb = S(y1, y0), d = S(y0, x0);
   const F3 n = C(ea, eb);
   const float q = D(n, n), la = D(ea, ea), lb = D(eb, eb);
-  const float e = kRejectErr * (la + lb) * (la + lb + D(d, d)) + 1e-30f;
-  const float p = D(n, C(eb, d)), r = D(n, C(ea, d));
-  return p > e || r > e || p + q < -e || r + q < -e || q + 1e-30f < 0.99e-6f * la * lb;
+  const F3 mb = C(eb, d), ma = C(ea, d);
+  const float l = la + lb, t = l + D(d, d);
+  const float e = kUnit * (144.0f * RootUp(q) * t + 0.01f * l * t) + 1e-30f;
+  const float f = 32.0f * kUnit * l;
+  const float p = D(n, mb), r = D(n, ma);
+  const float ep = e + f * RootUp(D(mb, mb)), er = e + f * RootUp(D(ma, ma));
+  return p > ep || r > er || p + q < -ep || r + q < -er || q + 1e-30f < 0.99e-6f * la * lb;
 }
 
 __device__ __forceinline__ bool VfReject(F3 x, F3 y0, F3 y1, F3 y2) {

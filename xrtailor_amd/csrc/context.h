@@ -68,7 +68,7 @@ struct ContactData {
   DevBuf<int4> c_tris, c_fe;
   DevBuf<int2> c_edges;
   DevBuf<int32_t> c_ef_ptr, c_ef;
-  DevBuf<float4> c_face_n;
+  DevBuf<float4> c_edge_n;
   DevBuf<uint32_t> c_rtri;
   DevBuf<int4> c_trir;
   // obstacle topology and state
@@ -76,7 +76,7 @@ struct ContactData {
   DevBuf<int4> o_tris, o_fe;
   DevBuf<int2> o_edges;
   DevBuf<int32_t> o_ef_ptr, o_ef;
-  DevBuf<float4> o_face_n;
+  DevBuf<float4> o_edge_n;
   DevBuf<uint32_t> o_rtri;
   DevBuf<int4> o_trir;
   DevBuf<float4> o_x0, o_x, o_x1, o_n1;
@@ -98,6 +98,7 @@ struct ContactData {
   // repulsion test items of the batched path (capacities 0: lists off)
   int vf_cap = 0, ee_cap = 0;
   DevBuf<int2> rep_vf, rep_ee;
+  DevBuf<uint2> ids_vf, ids_ee;
   DevBuf<uint32_t> ivf, iee;  // per cloth leaf item offsets (block-local prefix)
   DevBuf<uint2> nitem;        // per cloth leaf item counts (VF, EE)
   DevBuf<uint32_t> stage;  // kPairStage hits per cloth leaf of the batched pair refresh
