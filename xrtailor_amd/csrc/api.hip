@@ -6,6 +6,7 @@
 #include <numeric>
 #include <string>
 
+#include "adjoint.h"
 #include "context.h"
 #include "dynamics.h"
 #include "topology.h"
@@ -76,39 +77,83 @@ int CheckStarted(xrt_ctx* c, int32_t inst) {
 }
 
 
+// the next slot of the context's pinned staging memory (8 floats for each vertex of the largest
+// instance), free to be written: the copy issued from it two calls earlier has completed
+int StateSlot(xrt_ctx* c, float4** out) {
+  SkinStage& st = c->state_stage;
+  size_t need = 0;
+  for (const HostInstance& h : c->inst) need = std::max(need, 8 * static_cast<size_t>(std::max(h.nv, 1)));
+  if (st.per < need) {
+    st.Release();
+    XRT_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&st.host), 2 * need * sizeof(float), 0));
+    st.per = need;
+  }
+  for (auto& e : st.ev)
+    if (!e) XRT_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  st.slot ^= 1;
+  if (!st.fresh[st.slot]) XRT_CHECK_HIP(hipEventSynchronize(st.ev[st.slot]));
+  *out = reinterpret_cast<float4*>(st.host + st.slot * st.per);
+  return XRT_OK;
+}
+
+// queued on the context's stream; the caller's arrays are copied before it returns
 int UploadState(xrt_ctx* c, int32_t inst, const float* x0, const float* v) {
+  if (!x0 && !v) return XRT_OK;
   xrt::HostInstance& h = c->inst[inst];
   const int nv = h.nv;
+  float4* buf = nullptr;
+  const int rc = StateSlot(c, &buf);
+  if (rc != XRT_OK) return rc;
   if (x0) {
-    std::vector<float4> buf(nv);
     for (int i = 0; i < nv; ++i)
       buf[i] = make_float4(x0[3 * i], x0[3 * i + 1], x0[3 * i + 2], h.inv_mass[i]);
-    XRT_CHECK_HIP(hipMemcpyAsync(c->x0.ptr + h.desc.vbeg, buf.data(), sizeof(float4) * nv,
+    XRT_CHECK_HIP(hipMemcpyAsync(c->x0.ptr + h.desc.vbeg, buf, sizeof(float4) * nv,
                                  hipMemcpyHostToDevice, c->stream));
-    XRT_CHECK_HIP(hipMemcpyAsync(c->x.ptr + h.desc.vbeg, buf.data(), sizeof(float4) * nv,
-                                 hipMemcpyHostToDevice, c->stream));
-    XRT_CHECK_HIP(hipStreamSynchronize(c->stream));
+    XRT_CHECK_HIP(LaunchCopy4(c->stream, c->x.ptr + h.desc.vbeg, c->x0.ptr + h.desc.vbeg, nv));
   }
   if (v) {
-    std::vector<float4> buf(nv);
-    for (int i = 0; i < nv; ++i) buf[i] = make_float4(v[3 * i], v[3 * i + 1], v[3 * i + 2], 0.0f);
-    XRT_CHECK_HIP(hipMemcpyAsync(c->v.ptr + h.desc.vbeg, buf.data(), sizeof(float4) * nv,
+    float4* bv = buf + nv;
+    for (int i = 0; i < nv; ++i) bv[i] = make_float4(v[3 * i], v[3 * i + 1], v[3 * i + 2], 0.0f);
+    XRT_CHECK_HIP(hipMemcpyAsync(c->v.ptr + h.desc.vbeg, bv, sizeof(float4) * nv,
                                  hipMemcpyHostToDevice, c->stream));
-    XRT_CHECK_HIP(hipStreamSynchronize(c->stream));
+  }
+  SkinStage& st = c->state_stage;
+  XRT_CHECK_HIP(hipEventRecord(st.ev[st.slot], c->stream));
+  st.fresh[st.slot] = false;
+  return XRT_OK;
+}
+
+// the n first components of up to two device arrays, one wait for both
+int Download3(xrt_ctx* c, const float4* dev, float* out, const float4* dev2, float* out2, int n) {
+  float4* buf = nullptr;
+  const int rc = StateSlot(c, &buf);
+  if (rc != XRT_OK) return rc;
+  if (out) XRT_CHECK_HIP(hipMemcpyAsync(buf, dev, sizeof(float4) * n, hipMemcpyDeviceToHost, c->stream));
+  if (out2)
+    XRT_CHECK_HIP(hipMemcpyAsync(buf + n, dev2, sizeof(float4) * n, hipMemcpyDeviceToHost, c->stream));
+  XRT_CHECK_HIP(hipStreamSynchronize(c->stream));
+  c->state_stage.fresh[c->state_stage.slot] = true;
+  for (int k = 0; k < 2; ++k) {
+    float* o = k ? out2 : out;
+    if (!o) continue;
+    const float4* b = buf + (k ? n : 0);
+    for (int i = 0; i < n; ++i) {
+      o[3 * i] = b[i].x;
+      o[3 * i + 1] = b[i].y;
+      o[3 * i + 2] = b[i].z;
+    }
   }
   return XRT_OK;
 }
 
-int Download3(xrt_ctx* c, const float4* dev, int n, float* out) {
-  std::vector<float4> buf(n);
-  XRT_CHECK_HIP(hipMemcpyAsync(buf.data(), dev, sizeof(float4) * n, hipMemcpyDeviceToHost, c->stream));
-  XRT_CHECK_HIP(hipStreamSynchronize(c->stream));
-  for (int i = 0; i < n; ++i) {
-    out[3 * i] = buf[i].x;
-    out[3 * i + 1] = buf[i].y;
-    out[3 * i + 2] = buf[i].z;
+bool AllFinite(const float* p, size_t n) {
+  uint32_t bad = 0;
+  for (size_t i = 0; i < n; ++i) {
+    uint32_t u;
+    std::memcpy(&u, p + i, 4);
+    bad |= (u & 0x7f800000u) == 0x7f800000u ? 1u : 0u;
   }
-  return XRT_OK;
+  return bad == 0;
 }
 
 BatchArgs MakeBatchArgs(xrt_ctx* c) {
@@ -924,12 +969,9 @@ int xrt_set_state(xrt_ctx* ctx, int32_t inst, const float* x0, const float* v) {
   int rc = CheckInst(ctx, inst);
   if (rc != XRT_OK) return rc;
   HostInstance& h = ctx->inst[inst];
-  if (x0)
-    for (int i = 0; i < 3 * h.nv; ++i)
-      XRT_REQUIRE(std::isfinite(x0[i]), XRT_ERR_NOT_FINITE, "non-finite position");
-  if (v)
-    for (int i = 0; i < 3 * h.nv; ++i)
-      XRT_REQUIRE(std::isfinite(v[i]), XRT_ERR_NOT_FINITE, "non-finite velocity");
+  const size_t n3 = 3 * static_cast<size_t>(h.nv);
+  XRT_REQUIRE(!x0 || AllFinite(x0, n3), XRT_ERR_NOT_FINITE, "non-finite position");
+  XRT_REQUIRE(!v || AllFinite(v, n3), XRT_ERR_NOT_FINITE, "non-finite velocity");
   if (!ctx->started) {
     if (x0) h.x0_init.assign(x0, x0 + 3 * h.nv);
     if (v) h.v_init.assign(v, v + 3 * h.nv);
@@ -945,9 +987,8 @@ int xrt_get_state(xrt_ctx* ctx, int32_t inst, float* x0, float* v) {
   int rc = CheckStarted(ctx, inst);
   if (rc != XRT_OK) return rc;
   const InstDesc& d = ctx->inst[inst].desc;
-  if (x0 && (rc = Download3(ctx, ctx->x0.ptr + d.vbeg, d.nv, x0)) != XRT_OK) return rc;
-  if (v && (rc = Download3(ctx, ctx->v.ptr + d.vbeg, d.nv, v)) != XRT_OK) return rc;
-  return XRT_OK;
+  if (!x0 && !v) return XRT_OK;
+  return Download3(ctx, ctx->x0.ptr + d.vbeg, x0, ctx->v.ptr + d.vbeg, v, d.nv);
 }
 
 int xrt_get_predicted(xrt_ctx* ctx, int32_t inst, float* x) {
@@ -955,7 +996,7 @@ int xrt_get_predicted(xrt_ctx* ctx, int32_t inst, float* x) {
   if (rc != XRT_OK) return rc;
   XRT_REQUIRE(x, XRT_ERR_INVALID_ARG, "null output");
   const InstDesc& d = ctx->inst[inst].desc;
-  return Download3(ctx, ctx->x.ptr + d.vbeg, d.nv, x);
+  return Download3(ctx, ctx->x.ptr + d.vbeg, x, nullptr, nullptr, d.nv);
 }
 
 int xrt_predict_positions(xrt_ctx* ctx, int32_t inst, float dt) {

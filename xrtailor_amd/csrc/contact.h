@@ -88,6 +88,9 @@ hipError_t LaunchRepulsion(hipStream_t s, const MeshTopo& cloth, const MeshState
                            const MeshTopo& obs, const MeshState& os, const int2* pairs,
                            const int32_t* n_obs_pairs, const int32_t* n_total, int cap, float h,
                            long long* dq, int32_t* cnt);
+// no contact records: faces -1, EE records zero
+hipError_t LaunchClearRecords(hipStream_t s, int32_t* vf_face, int32_t* rt_face, int nv, EeRec* ee,
+                              uint8_t* ee_none, int ne);
 // FindPairs into pairs + *base (device offset), only slots < cap
 hipError_t LbvhFindPairsAt(Lbvh& lhs, const Lbvh& rhs, float thickness, int2* pairs,
                            const int32_t* base, int cap, hipStream_t s);

@@ -658,6 +658,19 @@ __device__ __forceinline__ void NotePairOverflow(int total, int cap, int nf, int
   if (total > cap && overflow) atomicMax(overflow, (total + max(nf, 1) - 1) / max(nf, 1));
 }
 
+__global__ __launch_bounds__(kBlock) void ClearRecordsKernel(int32_t* __restrict__ vf_face,
+                                                             int32_t* __restrict__ rt_face, int nv,
+                                                             EeRec* __restrict__ ee,
+                                                             uint8_t* __restrict__ ee_none, int ne) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < nv) vf_face[i] = rt_face[i] = -1;
+  if (i < ne) {
+    const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    ee[i] = EeRec{z, z, z, z};
+    ee_none[i] = 0;
+  }
+}
+
 __global__ void AddTotalsKernel(const int32_t* a, const int32_t* b, int32_t* out, int cap, int nf,
                                 int32_t* overflow) {
   if (threadIdx.x == 0) {
@@ -1755,6 +1768,13 @@ hipError_t LbvhFindPairsAt(Lbvh& lhs, const Lbvh& rhs, float thickness, int2* pa
   FindPairsAtKernel<<<Blocks(lhs.nf), kBlock, 0, s>>>(
       lhs.view(), rhs.view(), thickness, reinterpret_cast<const uint32_t*>(lhs.counts.ptr),
       reinterpret_cast<const uint32_t*>(lhs.offsets.ptr), base, pairs, cap);
+  return hipGetLastError();
+}
+hipError_t LaunchClearRecords(hipStream_t s, int32_t* vf_face, int32_t* rt_face, int nv, EeRec* ee,
+                              uint8_t* ee_none, int ne) {
+  const int n = std::max(nv, ne);
+  if (n <= 0) return hipSuccess;
+  ClearRecordsKernel<<<Blocks(n), kBlock, 0, s>>>(vf_face, rt_face, nv, ee, ee_none, ne);
   return hipGetLastError();
 }
 hipError_t LaunchAddTotals(hipStream_t s, const int32_t* a, const int32_t* b, int32_t* out, int cap,

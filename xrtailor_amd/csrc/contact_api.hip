@@ -226,14 +226,11 @@ int ContactStateReset(xrt_ctx* ctx, int inst) {
   ContactData& c = *ctx->contact[inst];
   const HostInstance& h = ctx->inst[inst];
   hipStream_t s = ctx->stream;
-  XRT_CHECK_HIP(hipMemsetAsync(c.vf_face.ptr, 0xff, sizeof(int32_t) * h.nv, s));
-  XRT_CHECK_HIP(hipMemsetAsync(c.rt_face.ptr, 0xff, sizeof(int32_t) * h.nv, s));
-  XRT_CHECK_HIP(hipMemsetAsync(c.ee.ptr, 0, c.ee.n, s));
-  XRT_CHECK_HIP(hipMemsetAsync(c.ee_none.ptr, 0, c.ee_none.n, s));
+  XRT_CHECK_HIP(LaunchClearRecords(s, c.vf_face.ptr, c.rt_face.ptr, h.nv,
+                                   reinterpret_cast<EeRec*>(c.ee.ptr), c.ee_none.ptr, h.ne()));
   if (ctx->params.enable_self_contact)
     XRT_CHECK_HIP(LbvhBuild(c.cloth_bvh, ctx->x0.ptr + h.desc.vbeg, nullptr, nullptr, 0.0f, 0,
                             0.0f, s));
-  XRT_CHECK_HIP(hipStreamSynchronize(s));
   return XRT_OK;
 }
 

@@ -127,7 +127,7 @@ struct ParticleData {
 };
 
 // Bindings, nearest-face records and obstacle skinning of every instance (binding.h).
-// Pinned two-slot staging of the joint transforms (xrt_skin_obstacle[s]): the upload is
+// Pinned two-slot staging of the joint transforms (xrt_skin_obstacle[s]) and of states: an upload is
 // queued on the stream without waiting for it; a slot is written again only after the copy
 // issued from it two calls earlier has completed.
 struct SkinStage {
@@ -344,6 +344,8 @@ struct xrt_ctx {
   xrt::ParticleData particles;
   // obstacle skinning and cloth-to-body bindings
   xrt::BindingData binding;
+  // pinned staging of xrt_set_state / xrt_get_state
+  xrt::SkinStage state_stage;
   // per-frame cache (xrt_record_frames)
   xrt::RecordData record;
   // quality-mode FEM constraints

@@ -220,10 +220,7 @@ int ParticleStateReset(xrt_ctx* ctx, int inst) {
   if (!ParticlesOn(ctx) || !ctx->particles.sized) return XRT_OK;
   XRT_REQUIRE(inst >= 0 && static_cast<size_t>(inst) < ctx->particles.one_v.size(), XRT_ERR_STATE,
               "particle maps missing for the instance");
-  const int rc = Hash(ctx, inst);
-  if (rc != XRT_OK) return rc;
-  XRT_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-  return XRT_OK;
+  return Hash(ctx, inst);
 }
 
 int ParticleSubstepEnd(xrt_ctx* ctx, int inst) {
