@@ -920,22 +920,33 @@ __global__ __launch_bounds__(1024) void MultiObsMergeTopKernel(const InstContact
   if (c.has_obs) MergeTop(c.obvh);
 }
 
-__global__ __launch_bounds__(kBlock) void MultiVfGenerateKernel(const InstContactDev* ic,
-                                                                const int32_t* off, int n,
-                                                                const float4* __restrict__ x0,
-                                                                const float4* __restrict__ x) {
-  XRT_MULTI_INDEX(kVert, c.nv)
-  if (!c.has_obs) return;
-  VfDcdGenerateBody(x + c.vbeg, i, c.obvh, c.vf_face, c.vf_q);
-  VfCcdGenerateBody(x0 + c.vbeg, x + c.vbeg, i, c.obvh, c.rt_face, c.rt_q);
-}
-
-__global__ __launch_bounds__(kBlock) void MultiEeGenerateKernel(const InstContactDev* ic,
-                                                                const int32_t* off, int n,
-                                                                const float4* __restrict__ x) {
-  XRT_MULTI_INDEX(kEdge, c.ne)
-  if (!c.has_obs) return;
-  EeDcdGenerateBody(x + c.vbeg, c.cloth.edges, i, c.obvh, c.obs.rtri, c.ee, c.ee_none);
+// The contact generation of every instance, one query of the obstacle tree per thread: edges in
+// the first `edge_grid` blocks, then each vertex's point query, then its segment query
+// (vert_grid blocks each).  A query is a chain of dependent node loads (85 us for the edges of 8
+// cloths, 55 us for both of the vertices, with most of the chip idle), so the three run side by
+// side in one launch: together as long as the edges alone.
+__global__ __launch_bounds__(kBlock) void MultiGenerateKernel(const InstContactDev* ic,
+                                                              const int32_t* off_e,
+                                                              const int32_t* off_v, int n,
+                                                              uint32_t edge_grid, uint32_t vert_grid,
+                                                              const float4* __restrict__ x0,
+                                                              const float4* __restrict__ x) {
+  const bool edge = blockIdx.x < edge_grid;
+  const bool segment = blockIdx.x >= edge_grid + vert_grid;
+  const int32_t* off = edge ? off_e : off_v;
+  const int lblk = XcdBlockOf(
+      off, n, edge ? blockIdx.x : blockIdx.x - edge_grid - (segment ? vert_grid : 0u));
+  if (lblk < 0) return;
+  const int k = InstOfBlock(off, n, lblk);
+  const InstContactDev& c = ic[k];
+  const int i = (lblk - off[k]) * kBlock + threadIdx.x;
+  if (!c.has_obs || i >= (edge ? c.ne : c.nv)) return;
+  if (edge)
+    EeDcdGenerateBody(x + c.vbeg, c.cloth.edges, i, c.obvh, c.obs.rtri, c.ee, c.ee_none);
+  else if (!segment)
+    VfDcdGenerateBody(x + c.vbeg, i, c.obvh, c.vf_face, c.vf_q);
+  else
+    VfCcdGenerateBody(x0 + c.vbeg, x + c.vbeg, i, c.obvh, c.rt_face, c.rt_q);
 }
 
 // cloth LBVH Update(ccd): pred = x, then leaves grow by bounds(x, x0)
@@ -1802,9 +1813,10 @@ hipError_t MultiObstacleRefit(hipStream_t s, const InstContactDev* ic, const Mul
 hipError_t MultiGenerate(hipStream_t s, const InstContactDev* ic, const MultiMaps& m,
                          const float4* x0, const float4* x) {
   if (Empty(m, MK::kVert)) return hipSuccess;
-  MultiVfGenerateKernel<<<XcdGrid(m.blocks[MK::kVert]), kBlock, 0, s>>>(ic, m.off[MK::kVert], m.n, x0, x);
-  if (!Empty(m, MK::kEdge))
-    MultiEeGenerateKernel<<<XcdGrid(m.blocks[MK::kEdge]), kBlock, 0, s>>>(ic, m.off[MK::kEdge], m.n, x);
+  const uint32_t eg = Empty(m, MK::kEdge) ? 0u : static_cast<uint32_t>(XcdGrid(m.blocks[MK::kEdge]));
+  const uint32_t vg = static_cast<uint32_t>(XcdGrid(m.blocks[MK::kVert]));
+  MultiGenerateKernel<<<eg + 2 * vg, kBlock, 0, s>>>(ic, m.off[MK::kEdge], m.off[MK::kVert], m.n, eg,
+                                                     vg, x0, x);
   return hipGetLastError();
 }
 

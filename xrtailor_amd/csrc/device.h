@@ -25,10 +25,15 @@ constexpr float kEps = 1e-6f;  // EPSILON (xrtailor/include/xrtailor/core/Scalar
 // in that XCD's L2.  -1: idle block.
 inline int XcdGrid(int blocks) { return (blocks + 7) / 8 * 8; }
 
-__device__ __forceinline__ int XcdBlock(const int32_t* __restrict__ off, int n) {
+// the logical block of physical block b (blockIdx.x, or that less a multiple of 8 where a grid
+// holds several maps one after the other)
+__device__ __forceinline__ int XcdBlockOf(const int32_t* __restrict__ off, int n, uint32_t b) {
   const int total = off[n];
-  const int l = static_cast<int>(blockIdx.x & 7u) * ((total + 7) >> 3) + static_cast<int>(blockIdx.x >> 3);
+  const int l = static_cast<int>(b & 7u) * ((total + 7) >> 3) + static_cast<int>(b >> 3);
   return l < total ? l : -1;
+}
+__device__ __forceinline__ int XcdBlock(const int32_t* __restrict__ off, int n) {
+  return XcdBlockOf(off, n, blockIdx.x);
 }
 
 // the instance of logical block b of such a map
