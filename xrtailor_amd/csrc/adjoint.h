@@ -24,6 +24,7 @@
 #include "bvh.h"
 #include "contact.h"
 #include "device.h"
+#include "patch.h"
 
 namespace xrt {
 
@@ -38,6 +39,32 @@ struct WideArgs {
   float4* x;         // iterate
   const float4* xw;  // a state array whose .w is the inverse mass (reverse kernels)
 };
+
+// Plan and state of the reverse sweep (PatchAdjKernel): patches and color offsets as in patch.h
+// with the colors reversed, bends first; per entry its local indices (16 bits each) and its
+// constraint (bit 31: owned by this patch), per stretch entry the multiplier's adjoint
+struct PatchAdjArgs {
+  const PatchDev* patch;
+  const int32_t* verts;
+  const int32_t* off;
+  const int4* bent;
+  const int2* sent;
+  const float2* bpar;
+  const StretchC* sc;
+  const float4* xw;
+  const double4* gx;
+  double4* out;  // not gx
+  double* glam;
+  double* gcomp;
+  double* gbcomp;
+  int n, nb, ns;
+};
+constexpr size_t kPatchAdjVertBytes = 3 * sizeof(double) + sizeof(float);
+// one iteration's bends (if any) and stretches; first: the substep's last iteration
+hipError_t LaunchPatchAdj(hipStream_t s, const PatchAdjArgs& a, float inv_dt2, const BendMode& m,
+                          int bends, int first, const float4* tape_b, const float4* tape_s,
+                          int threads, size_t lds_bytes);
+hipError_t ConfigurePatchAdj(size_t lds_bytes);
 
 // ------------------------------------------------------------------ forward
 // map (optional): this color's block map -- n_inst + 1 prefix sums of the instances' block

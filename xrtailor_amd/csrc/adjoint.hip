@@ -222,13 +222,47 @@ __global__ __launch_bounds__(kBs) void GroundAdjKernel(const float4* __restrict_
   gx[i] = out;
 }
 
+// One stretch constraint in reverse: tape (x_i, lambda before) and x_j, inverse masses w1, w2,
+// adjoints ga, gb and gl of the positions and the multiplier; gc receives the compliance's share.
+// False: the forward did not move (ga and gb stand; gl is the caller's to clear at iteration 0).
+__device__ __forceinline__ bool StretchAdj(float4 ta, float4 tb, float w1, float w2, float rest,
+                                           float compliance, float inv_dt2, D3& ga, D3& gb,
+                                           double& gl, double& gc) {
+#pragma clang fp contract(off)
+  {  // the forward's test (StretchSolve, FP32)
+    const float fx = ta.x - tb.x, fy = ta.y - tb.y, fz = ta.z - tb.z;
+    const float fdist = sqrtf(fx * fx + fy * fy + fz * fz);
+    if (!(fdist != rest && w1 + w2 > 0.0f)) return false;
+  }
+  const double lam = ta.w;
+  const double dx = static_cast<double>(ta.x) - tb.x, dy = static_cast<double>(ta.y) - tb.y,
+               dz = static_cast<double>(ta.z) - tb.z;
+  const double dist = sqrt(dx * dx + dy * dy + dz * dz);
+  const double inv = 1.0 / (dist + static_cast<double>(kEps));
+  const double at = static_cast<double>(compliance) * inv_dt2;
+  const double D = static_cast<double>(w1) + w2 + at;
+  const double dl = (-(dist - rest) - at * lam) / D;
+  const double s = dl * inv;
+  const double ux = w1 * ga.x - w2 * gb.x, uy = w1 * ga.y - w2 * gb.y, uz = w1 * ga.z - w2 * gb.z;
+  const double gs = ux * dx + uy * dy + uz * dz;
+  const double gdl = gl + gs * inv;
+  const double ginv = gs * dl;
+  const double gdist = -gdl / D - ginv * inv * inv;
+  gc = -gdl * (lam + dl) / D * inv_dt2;
+  gl = gl - gdl * at / D;
+  const double gd = dist > 0.0 ? gdist / dist : 0.0;
+  const double ex = s * ux + gd * dx, ey = s * uy + gd * dy, ez = s * uz + gd * dz;
+  ga = D3{ga.x + ex, ga.y + ey, ga.z + ez};
+  gb = D3{gb.x - ex, gb.y - ey, gb.z - ez};
+  return true;
+}
+
 __global__ __launch_bounds__(kBs) void WideStretchAdjKernel(WideArgs a, int color, float inv_dt2,
                                                             int iter,
                                                             const float4* __restrict__ tape,
                                                             double4* __restrict__ gx,
                                                             double* __restrict__ glam,
                                                             double* __restrict__ gcomp) {
-#pragma clang fp contract(off)
   const InstDesc di = a.inst[blockIdx.y];
   if (color >= di.s_ncol) return;
   const int beg = a.s_coloff[di.s_cbeg + color], end = a.s_coloff[di.s_cbeg + color + 1];
@@ -236,59 +270,26 @@ __global__ __launch_bounds__(kBs) void WideStretchAdjKernel(WideArgs a, int colo
   if (k >= end) return;
   const StretchC c = a.sc[k];
   const int i0 = di.vbeg + c.i0, i1 = di.vbeg + c.i1;
-  const float4 ta = tape[2 * k], tb = tape[2 * k + 1];
-  const float w1 = a.xw[i0].w, w2 = a.xw[i1].w;
-  double gl = glam[k];
-  {  // the forward's test (StretchSolve, FP32)
-    const float fx = ta.x - tb.x, fy = ta.y - tb.y, fz = ta.z - tb.z;
-    const float fdist = sqrtf(fx * fx + fy * fy + fz * fz);
-    if (!(fdist != c.rest && w1 + w2 > 0.0f)) {
-      glam[k] = iter == 0 ? 0.0 : gl;
-      return;
-    }
+  D3 ga = d3(gx[i0]), gb = d3(gx[i1]);
+  double gl = glam[k], gc;
+  if (StretchAdj(tape[2 * k], tape[2 * k + 1], a.xw[i0].w, a.xw[i1].w, c.rest, c.compliance, inv_dt2,
+                 ga, gb, gl, gc)) {
+    gcomp[k] += gc;
+    gx[i0] = d4(ga);
+    gx[i1] = d4(gb);
   }
-  const double lam = ta.w;
-  const double dx = static_cast<double>(ta.x) - tb.x, dy = static_cast<double>(ta.y) - tb.y,
-               dz = static_cast<double>(ta.z) - tb.z;
-  const double dist = sqrt(dx * dx + dy * dy + dz * dz);
-  const double4 ga = gx[i0], gb = gx[i1];
-  const double inv = 1.0 / (dist + static_cast<double>(kEps));
-  const double at = static_cast<double>(c.compliance) * inv_dt2;
-  const double D = static_cast<double>(w1) + w2 + at;
-  const double dl = (-(dist - c.rest) - at * lam) / D;
-  const double s = dl * inv;
-  const double ux = w1 * ga.x - w2 * gb.x, uy = w1 * ga.y - w2 * gb.y, uz = w1 * ga.z - w2 * gb.z;
-  const double gs = ux * dx + uy * dy + uz * dz;
-  const double gdl = gl + gs * inv;
-  const double ginv = gs * dl;
-  const double gdist = -gdl / D - ginv * inv * inv;
-  gcomp[k] += -gdl * (lam + dl) / D * inv_dt2;
-  gl = gl - gdl * at / D;
-  const double gd = dist > 0.0 ? gdist / dist : 0.0;
-  const double ex = s * ux + gd * dx, ey = s * uy + gd * dy, ez = s * uz + gd * dz;
-  gx[i0] = make_double4(ga.x + ex, ga.y + ey, ga.z + ez, 0.0);
-  gx[i1] = make_double4(gb.x - ex, gb.y - ey, gb.z - ez, 0.0);
   glam[k] = iter == 0 ? 0.0 : gl;
 }
 
-__global__ __launch_bounds__(kBs) void WideBendAdjKernel(WideArgs a, int color, float inv_dt2,
-                                                         BendMode m,
-                                                         const float4* __restrict__ tape,
-                                                         double4* __restrict__ gx,
-                                                         double* __restrict__ gbcomp) {
+// One bend element in reverse: its tape record, inverse masses and parameters (rest angle,
+// compliance), the adjoints g1..g4; gc receives the compliance's share.  False: the forward did
+// not move.
+__device__ __forceinline__ bool BendAdj(float4 t0, float4 t1, float4 t2, float w1, float w2,
+                                        float w3, float w4, float2 par, float inv_dt2, BendMode m,
+                                        D3& g1, D3& g2, D3& g3, D3& g4, double& gc) {
 #pragma clang fp contract(off)
-  const InstDesc di = a.inst[blockIdx.y];
-  if (color >= di.b_ncol) return;
-  const int beg = a.b_coloff[di.b_cbeg + color], end = a.b_coloff[di.b_cbeg + color + 1];
-  const int k = beg + blockIdx.x * kBs + threadIdx.x;
-  if (k >= end) return;
-  const int4 lid = a.bidx[k];
-  const int id1 = di.vbeg + lid.x, id2 = di.vbeg + lid.y, id3 = di.vbeg + lid.z, id4 = di.vbeg + lid.w;
-  const float4 t0 = tape[3 * k], t1 = tape[3 * k + 1], t2 = tape[3 * k + 2];
   const float3 fx1 = make_float3(t0.x, t0.y, t0.z), fx2 = make_float3(t0.w, t1.x, t1.y);
   const float3 fx3 = make_float3(t1.z, t1.w, t2.x), fx4 = make_float3(t2.y, t2.z, t2.w);
-  const float w1 = a.xw[id1].w, w2 = a.xw[id2].w, w3 = a.xw[id3].w, w4 = a.xw[id4].w;
-  const float2 par = a.bpar[k];
   float fdraw;
   {  // the forward's tests (BendSolve, FP32)
     const float3 p2 = Sub(fx2, fx1), p3 = Sub(fx3, fx1), p4 = Sub(fx4, fx1);
@@ -296,9 +297,9 @@ __global__ __launch_bounds__(kBs) void WideBendAdjKernel(WideArgs a, int color, 
     const float3 n1 = Scale(c23, 1.0f / sqrtf(Dot(c23, c23)));
     const float3 n2 = Scale(c24, 1.0f / sqrtf(Dot(c24, c24)));
     fdraw = Dot(n1, n2);
-    if (fdraw != fdraw) return;
+    if (fdraw != fdraw) return false;
     const float fd = fminf(fmaxf(fdraw, m.dlo), 1.0f);
-    if (acosf(fd) < kEps) return;
+    if (acosf(fd) < kEps) return false;
     const float i23 = 1.0f / (sqrtf(Dot(c23, c23)) + kEps), i24 = 1.0f / (sqrtf(Dot(c24, c24)) + kEps);
     const float3 q3 = Scale(Add(Cross(p2, n2), Scale(Cross(n1, p2), fd)), i23);
     const float3 q4 = Scale(Add(Cross(p2, n1), Scale(Cross(n2, p2), fd)), i24);
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(kBs) void WideBendAdjKernel(WideArgs a, int color, 
     const float3 q1 = Scale(Add(Add(q2, q3), q4), -1.0f);
     const float fden = par.y * inv_dt2 +
                        (w1 * Dot(q1, q1) + w2 * Dot(q2, q2) + w3 * Dot(q3, q3) + w4 * Dot(q4, q4));
-    if (fden < kEps) return;
+    if (fden < kEps) return false;
   }
   // forward quantities in double
   const D3 x1 = d3(fx1), x2 = d3(fx2), x3 = d3(fx3), x4 = d3(fx4);
@@ -333,10 +334,9 @@ __global__ __launch_bounds__(kBs) void WideBendAdjKernel(WideArgs a, int color, 
   const double lam = m.sgn * s * (ang - th) / denom;
 
   // reverse
-  const D3 g1 = d3(gx[id1]), g2 = d3(gx[id2]), g3 = d3(gx[id3]), g4 = d3(gx[id4]);
   const double glam = w1 * Dt(q1, g1) + w2 * Dt(q2, g2) + w3 * Dt(q3, g3) + w4 * Dt(q4, g4);
   const double gden = -glam * lam / denom;
-  gbcomp[k] += gden * inv_dt2;
+  gc = gden * inv_dt2;
   D3 gq1 = Ad(Sc(g1, w1 * lam), Sc(q1, 2.0 * gden * w1));
   D3 gq2 = Ad(Sc(g2, w2 * lam), Sc(q2, 2.0 * gden * w2));
   D3 gq3 = Ad(Sc(g3, w3 * lam), Sc(q3, 2.0 * gden * w3));
@@ -382,10 +382,158 @@ __global__ __launch_bounds__(kBs) void WideBendAdjKernel(WideArgs a, int color, 
   Ac(gp2, Cr(p3, gc23)); Ac(gp3, Cr(gc23, p2));
   Ac(gp2, Cr(p4, gc24)); Ac(gp4, Cr(gc24, p2));
   // p_k = x_k - x1, plus the identity part of x' = x + w lam q
-  gx[id1] = d4(Sb(g1, Ad(Ad(gp2, gp3), gp4)));
-  gx[id2] = d4(Ad(g2, gp2));
-  gx[id3] = d4(Ad(g3, gp3));
-  gx[id4] = d4(Ad(g4, gp4));
+  g1 = Sb(g1, Ad(Ad(gp2, gp3), gp4));
+  g2 = Ad(g2, gp2);
+  g3 = Ad(g3, gp3);
+  g4 = Ad(g4, gp4);
+  return true;
+}
+
+__global__ __launch_bounds__(kBs) void WideBendAdjKernel(WideArgs a, int color, float inv_dt2,
+                                                         BendMode m,
+                                                         const float4* __restrict__ tape,
+                                                         double4* __restrict__ gx,
+                                                         double* __restrict__ gbcomp) {
+  const InstDesc di = a.inst[blockIdx.y];
+  if (color >= di.b_ncol) return;
+  const int beg = a.b_coloff[di.b_cbeg + color], end = a.b_coloff[di.b_cbeg + color + 1];
+  const int k = beg + blockIdx.x * kBs + threadIdx.x;
+  if (k >= end) return;
+  const int4 lid = a.bidx[k];
+  const int id1 = di.vbeg + lid.x, id2 = di.vbeg + lid.y, id3 = di.vbeg + lid.z, id4 = di.vbeg + lid.w;
+  D3 g1 = d3(gx[id1]), g2 = d3(gx[id2]), g3 = d3(gx[id3]), g4 = d3(gx[id4]);
+  double gc;
+  if (!BendAdj(tape[3 * k], tape[3 * k + 1], tape[3 * k + 2], a.xw[id1].w, a.xw[id2].w, a.xw[id3].w,
+               a.xw[id4].w, a.bpar[k], inv_dt2, m, g1, g2, g3, g4, gc))
+    return;
+  gbcomp[k] += gc;
+  gx[id1] = d4(g1);
+  gx[id2] = d4(g2);
+  gx[id3] = d4(g3);
+  gx[id4] = d4(g4);
+}
+
+// ------------------------------------------------ every color in reverse, in one launch
+// The reverse of PatchSweepKernel: a workgroup per patch of a plan made for the reversed order
+// (bend colors from the last to the first, then the stretch colors), adjoints in LDS (3 doubles
+// and the inverse mass a vertex), written to the other of two adjoint buffers.  The entries'
+// indices are loaded two steps ahead and the tape one, so that a color waits for neither.  What
+// bounds it is the length of one bend's reverse in FP64 (14 colors of it on a grid, a wave or two
+// a SIMD): an iteration of a 128 x 128 cloth takes 67 us, as one launch per color it took 104 us
+// and the gaps of 20 launches.
+struct AdjPos {
+  int c, beg, end;
+};
+
+template <class Index, class Load, class Solve>
+__device__ __forceinline__ void SweepReverse(const int32_t* __restrict__ off, int colors, Index&& index,
+                                             Load&& load, Solve&& solve) {
+  const int tid = threadIdx.x, bs = blockDim.x;
+  auto next = [&](AdjPos p) {  // the next round of the color, or the next color with entries
+    if (p.beg + bs < p.end) return AdjPos{p.c, p.beg + bs, p.end};
+    int c = p.c + 1;
+    while (c < colors && off[c] == off[c + 1]) ++c;
+    return c < colors ? AdjPos{c, off[c], off[c + 1]} : AdjPos{colors, 0, 0};
+  };
+  AdjPos p0 = next(AdjPos{-1, 0, 0}), p1 = next(p0);
+  auto i0 = index(p0.beg + tid, p0.beg + tid < p0.end);
+  auto i1 = index(p1.beg + tid, p1.beg + tid < p1.end);
+  auto r0 = load(i0, p0.beg + tid < p0.end);
+  while (p0.c < colors) {
+    const AdjPos p2 = next(p1);
+    const auto i2 = index(p2.beg + tid, p2.beg + tid < p2.end);
+    const auto r1 = load(i1, p1.beg + tid < p1.end);
+    if (p0.beg + tid < p0.end) solve(p0.beg + tid, i0, r0);
+    if (p1.c != p0.c) {  // LDS only: the loads ahead stay in flight
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    }
+    p0 = p1;
+    p1 = p2;
+    i0 = i1;
+    i1 = i2;
+    r0 = r1;
+  }
+}
+
+struct BendTape {
+  float4 t0, t1, t2;
+  float2 par;
+};
+struct StretchTape {
+  float4 ta, tb;
+  float rest, compliance;
+};
+
+constexpr int kAdjSweepThreads = 512;  // FP64 needs the registers: up to 256 a lane
+
+__global__ __launch_bounds__(kAdjSweepThreads) void PatchAdjKernel(PatchAdjArgs a, float inv_dt2,
+                                                                   BendMode m, int bends, int first,
+                                                                   const float4* __restrict__ tape_b,
+                                                                   const float4* __restrict__ tape_s) {
+  extern __shared__ double G[];  // 3 n_loc adjoints, then n_loc inverse masses
+  const PatchDev p = a.patch[blockIdx.x];
+  const int32_t* __restrict__ off = a.off + p.off;
+  const int32_t* __restrict__ verts = a.verts + p.vbeg;
+  D3* X = reinterpret_cast<D3*>(G);
+  float* W = reinterpret_cast<float*>(X + p.n_loc);
+  for (int v = threadIdx.x; v < p.n_loc; v += blockDim.x) {
+    const int g = verts[v];
+    X[v] = d3(a.gx[g]);
+    W[v] = a.xw[g].w;
+  }
+  __syncthreads();
+  if (bends)
+    SweepReverse(
+        off, a.nb, [&](int e, bool in) { return in ? a.bent[e] : make_int4(0, 0, 0, 0); },
+        [&](const int4& i, bool in) {
+          BendTape t{};
+          if (in) {
+            const int64_t q = i.z & 0x7fffffff;
+            t = BendTape{tape_b[3 * q], tape_b[3 * q + 1], tape_b[3 * q + 2], a.bpar[q]};
+          }
+          return t;
+        },
+        [&](int, const int4& i, const BendTape& t) {
+          const int v1 = i.x & 0xffff, v2 = static_cast<int>(static_cast<uint32_t>(i.x) >> 16);
+          const int v3 = i.y & 0xffff, v4 = static_cast<int>(static_cast<uint32_t>(i.y) >> 16);
+          D3 g1 = X[v1], g2 = X[v2], g3 = X[v3], g4 = X[v4];
+          double gc;
+          if (!BendAdj(t.t0, t.t1, t.t2, W[v1], W[v2], W[v3], W[v4], t.par, inv_dt2, m, g1, g2, g3,
+                       g4, gc))
+            return;
+          if (i.z < 0) a.gbcomp[i.z & 0x7fffffff] += gc;
+          X[v1] = g1;
+          X[v2] = g2;
+          X[v3] = g3;
+          X[v4] = g4;
+        });
+  __syncthreads();
+  SweepReverse(
+      off + a.nb + 1, a.ns, [&](int e, bool in) { return in ? a.sent[e] : make_int2(0, 0); },
+      [&](const int2& i, bool in) {
+        StretchTape t{};
+        if (in) {
+          const int64_t q = i.y & 0x7fffffff;
+          const StretchC c = a.sc[q];
+          t = StretchTape{tape_s[2 * q], tape_s[2 * q + 1], c.rest, c.compliance};
+        }
+        return t;
+      },
+      [&](int e, const int2& i, const StretchTape& t) {
+        const int v0 = i.x & 0xffff, v1 = static_cast<int>(static_cast<uint32_t>(i.x) >> 16);
+        D3 ga = X[v0], gb = X[v1];
+        double gl = first ? 0.0 : a.glam[e], gc;
+        if (StretchAdj(t.ta, t.tb, W[v0], W[v1], t.rest, t.compliance, inv_dt2, ga, gb, gl, gc)) {
+          if (i.y < 0) a.gcomp[i.y & 0x7fffffff] += gc;
+          X[v0] = ga;
+          X[v1] = gb;
+        }
+        a.glam[e] = gl;
+      });
+  __syncthreads();
+  for (int v = threadIdx.x; v < p.n_own; v += blockDim.x) a.out[verts[v]] = d4(X[v]);
 }
 
 // LRA (reverse): one target vertex of any instance per thread.  y = x - u + u R / |u|
@@ -581,6 +729,18 @@ hipError_t LaunchWideStretchAdj(hipStream_t s, const WideArgs& a, int n_inst, in
   WideStretchAdjKernel<<<dim3(Blocks(max_cnt), n_inst), kBs, 0, s>>>(a, color, inv_dt2, iter, tape,
                                                                       gx, glam, gcomp);
   return hipGetLastError();
+}
+hipError_t LaunchPatchAdj(hipStream_t s, const PatchAdjArgs& a, float inv_dt2, const BendMode& m,
+                          int bends, int first, const float4* tape_b, const float4* tape_s,
+                          int threads, size_t lds_bytes) {
+  if (a.n <= 0) return hipSuccess;
+  threads = std::min(threads, kAdjSweepThreads);
+  PatchAdjKernel<<<a.n, threads, lds_bytes, s>>>(a, inv_dt2, m, bends, first, tape_b, tape_s);
+  return hipGetLastError();
+}
+hipError_t ConfigurePatchAdj(size_t lds_bytes) {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&PatchAdjKernel),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes));
 }
 hipError_t LaunchWideBendAdj(hipStream_t s, const WideArgs& a, int n_inst, int color, int max_cnt,
                              float inv_dt2, const BendMode& m, const float4* tape, double4* gx,

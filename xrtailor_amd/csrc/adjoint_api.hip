@@ -75,6 +75,7 @@ int AdjSetup(xrt_ctx* c, int want_slots = 1) {
   const size_t N = static_cast<size_t>(A.n_total);
   const bool bend = p.solve_bending != 0, ground = p.enable_ground != 0;
   A.lra = c->total_slots > 0;
+  if (const int prc = PatchPrepareAdj(c); prc != XRT_OK) return prc;
   if (A.lra) {  // slot -> constraints (transpose of the per-target CSR), in constraint order
     std::vector<int32_t> cnt(c->total_slots + 1, 0), sinst(c->total_slots), cons;
     size_t total_k = 0;
@@ -368,7 +369,8 @@ int ReverseSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, int sub)
   // the forward's finalize: v = (x - x0) * (1 / dt) * damp_factor (FP32 factors)
   const double fin = static_cast<double>(1.0f / k.dt) * static_cast<double>(k.damp_factor);
   XRT_CHECK_HIP(LaunchFinalizeAdj(s, A.gx0.ptr, A.gv.ptr, A.gx.ptr, N, fin));
-  XRT_CHECK_HIP(LaunchZeroD1(s, A.glam.ptr, static_cast<int>(A.glam.n)));
+  const bool sweep = c->patches.adj.ready;
+  if (!sweep) XRT_CHECK_HIP(LaunchZeroD1(s, A.glam.ptr, static_cast<int>(A.glam.n)));
   for (int it = k.iterations - 1; it >= 0; --it) {
     const float4* TI = T + N + static_cast<size_t>(it) * A.it_stride;
     if (A.contacts) {
@@ -399,11 +401,15 @@ int ReverseSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, int sub)
                                      c->lra_slot.ptr, c->lra_rest.ptr, k.stretchiness,
                                      A.lra_xs.ptr, A.lra_gslot.ptr, A.slot_inst.ptr,
                                      A.slot_ptr.ptr, A.slot_cons.ptr, A.gx.ptr));
-    if (k.solve_bending)
+    if (sweep) {  // every color in one launch
+      const int rc = PatchAdjIter(c, k, bm, it + 1 == k.iterations, TI + A.off_b, TI + A.off_s);
+      if (rc != XRT_OK) return rc;
+    }
+    if (k.solve_bending && !sweep)
       for (int col = static_cast<int>(A.b_max.size()) - 1; col >= 0; --col)
         XRT_CHECK_HIP(LaunchWideBendAdj(s, wa, n_inst, col, A.b_max[col], k.inv_dt2, bm,
                                         TI + A.off_b, A.gx.ptr, A.gbcomp.ptr));
-    for (int col = static_cast<int>(A.s_max.size()) - 1; col >= 0; --col)
+    for (int col = static_cast<int>(A.s_max.size()) - 1; !sweep && col >= 0; --col)
       XRT_CHECK_HIP(LaunchWideStretchAdj(s, wa, n_inst, col, A.s_max[col], k.inv_dt2, it,
                                          TI + A.off_s, A.gx.ptr, A.glam.ptr, A.gcomp.ptr));
     if (A.rep) {  // the iteration's repulsion pass came first

@@ -236,6 +236,10 @@ struct PatchPlanDev {
 };
 struct PatchData {
   PatchPlanDev xpbd, fem;
+  PatchPlanDev adj;      // the reverse sweep's: families bends, stretches, colors reversed
+  DevBuf<int4> bent;
+  DevBuf<int2> sent;
+  DevBuf<double> glam;
   DevBuf<int4> srec, brec, frec, irec;
   DevBuf<int32_t> bcon;
   DevBuf<float4> finv, iK;
@@ -271,6 +275,7 @@ struct AdjointData {
   DevBuf<float4> fstart;  // (x0, v) at each frame start of a segment: [ckpt_every][2][n_total]
   DevBuf<float4> final_state;  // (x0, v) after the recorded frames
   DevBuf<double4> gx0, gv, gx;  // FP64 adjoints
+  DevBuf<double4> gx_alt;       // the reverse sweep writes it, then it and gx change places
   DevBuf<double> glam, gcomp, gbcomp;
   DevBuf<int32_t> ee_cnt;
   // PBD repulsion (self contact): per frame slot a pool of the responses of every repulsion
@@ -443,6 +448,9 @@ const PatchPlanDev& PatchPlanOf(const xrt_ctx* ctx);  // of the current constrai
 int PatchIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, int it, bool ground,
               float4* tape_s, float4* tape_b, float4* tape_g);
 int PatchRefreshCompliance(xrt_ctx* ctx);
+int PatchPrepareAdj(xrt_ctx* ctx);
+int PatchAdjIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, bool first,
+                 const float4* tape_b, const float4* tape_s);
 // adjoint_api.hip: one substep of every instance as wide launches with the contact phases
 // above; with a tape owner and sub >= 0 the operators' inputs go to tape slot `sub`
 int WideSubstep(xrt_ctx* ctx, const StepConsts& k, const BendMode& bm, AdjointData* tape, int sub);

@@ -5,13 +5,15 @@
 #include <thread>
 
 #include "context.h"
+#include "adjoint.h"
 #include "patch.h"
 #include "patch_plan.h"
 
 namespace xrt {
 namespace {
 
-constexpr int kPatchMaxVerts = 10240;  // 160 KB of LDS
+constexpr size_t kPatchMaxLds = 160 * 1024;
+constexpr int kPatchMaxVerts = kPatchMaxLds / sizeof(float4);
 constexpr double kPatchMaxWork = 6.0;  // listed constraints / constraints
 
 // constraints of `arity` vertices in sorted order: position p is cons[order[p]]
@@ -73,11 +75,12 @@ struct HostPlan {
 };
 template <class Families, class Entry0, class Entry1>
 bool MakePlan(xrt_ctx* ctx, int c0, int c1, Families&& families, Entry0&& entry0, Entry1&& entry1,
-              PatchPlanDev& D, HostPlan& H) {
+              PatchPlanDev& D, HostPlan& H, size_t vert_bytes = sizeof(float4),
+              bool hinges_first = false) {
   if (c0 + c1 == 0 || c0 + c1 + 2 > kPatchMaxOffsets) return false;
   const int ni = static_cast<int>(ctx->inst.size());
   const int max_local = static_cast<int>(
-      std::min<size_t>(kPatchMaxVerts, std::min<size_t>(ctx->max_lds, 160 * 1024) / sizeof(float4)));
+      std::min<size_t>(kPatchMaxVerts, std::min<size_t>(ctx->max_lds, kPatchMaxLds) / vert_bytes));
   // Own vertices per patch: what gives 4 of 5 CUs a patch, down to 256 vertices, where the
   // ring of neighbors already quadruples the stretch work of a grid, and up to 4096 (a grid's
   // patch then needs 117 KB of LDS, 1.4x the stretch and 1.2x the bend work).  ms per frame at
@@ -135,7 +138,8 @@ bool MakePlan(xrt_ctx* ctx, int c0, int c1, Families&& families, Entry0&& entry0
   // are the short ones (256 cloths: 23.7 -> 21.6 ms per frame)
   auto entries = [&](const PatchDev& d) {  // a hinge costs about four edges
     const int32_t* o = &H.off[d.off];
-    return (o[c0] - o[0]) + 4 * static_cast<int64_t>(o[c0 + 1 + c1] - o[c0 + 1]);
+    const int64_t n0 = o[c0] - o[0], n1 = o[c0 + 1 + c1] - o[c0 + 1];
+    return hinges_first ? 4 * n0 + n1 : n0 + 4 * n1;
   };
   std::stable_sort(H.dev.begin(), H.dev.end(), [&](const PatchDev& a, const PatchDev& b) {
     return entries(a) > entries(b);
@@ -144,7 +148,7 @@ bool MakePlan(xrt_ctx* ctx, int c0, int c1, Families&& families, Entry0&& entry0
   D.split = D.n > ni;
   D.c0 = c0;
   D.c1 = c1;
-  D.lds_bytes = sizeof(float4) * max_loc;
+  D.lds_bytes = vert_bytes * max_loc;
   D.threads = std::min(1024, std::max(64, (max_color + 63) / 64 * 64));
   return true;
 }
@@ -159,8 +163,8 @@ hipError_t UploadPlan(xrt_ctx* ctx, PatchPlanDev& D, const HostPlan& H) {
 
 // a plan whose buffers did not fit is dropped: the colors then run as launches of their own
 template <class... Bufs>
-int FinishPlan(PatchPlanDev& D, hipError_t e, Bufs&... bufs) {
-  if (e == hipSuccess && D.lds_bytes > 64 * 1024) e = ConfigurePatchSweep(D.lds_bytes);
+int FinishPlan(PatchPlanDev& D, hipError_t e, hipError_t (*configure)(size_t), Bufs&... bufs) {
+  if (e == hipSuccess && D.lds_bytes > 64 * 1024) e = configure(kPatchMaxLds);
   if (e == hipSuccess) {
     D.ready = true;
     return XRT_OK;
@@ -217,7 +221,7 @@ int PatchPrepare(xrt_ctx* ctx) {
   if (e == hipSuccess) e = P.brec.Upload(brec, s);
   if (e == hipSuccess) e = P.bcon.Upload(bcon, s);
   if (e == hipSuccess) e = P.slam.Alloc(std::max<size_t>(srec.size(), 1));
-  return FinishPlan(P.xpbd, e, P.srec, P.brec, P.bcon, P.slam);
+  return FinishPlan(P.xpbd, e, ConfigurePatchSweep, P.srec, P.brec, P.bcon, P.slam);
 }
 
 int PatchPrepareFem(xrt_ctx* ctx) {
@@ -260,7 +264,83 @@ int PatchPrepareFem(xrt_ctx* ctx) {
   if (e == hipSuccess) e = P.irec.Upload(irec, s);
   if (e == hipSuccess) e = P.iK.Upload(iK, s);
   if (e == hipSuccess) e = P.ilam.Alloc(std::max<size_t>(irec.size(), 1));
-  return FinishPlan(P.fem, e, P.frec, P.finv, P.irec, P.iK, P.ilam);
+  return FinishPlan(P.fem, e, ConfigurePatchSweep, P.frec, P.finv, P.irec, P.iK, P.ilam);
+}
+
+// The reverse sweep's plan (built when the first adjoint begins): what a vertex's adjoint depends
+// on in the reversed order of the colors.
+int PatchPrepareAdj(xrt_ctx* ctx) {
+  PatchData& P = ctx->patches;
+  if (P.adj.tried) return XRT_OK;
+  P.adj.tried = true;
+  const size_t ni = ctx->inst.size();
+  int ns = 0, nb = 0;
+  for (const HostInstance& h : ctx->inst) {
+    ns = std::max(ns, h.s_ncol);
+    nb = std::max(nb, h.b_ncol);
+  }
+  // color-sorted positions in reversed color order, and that order's color offsets
+  auto reversed = [](const std::vector<int32_t>& coloff, std::vector<int32_t>& pos,
+                     std::vector<int32_t>& off) {
+    pos.clear();
+    off.assign(1, 0);
+    for (size_t c = coloff.size(); c-- > 1;) {
+      for (int32_t p = coloff[c - 1]; p < coloff[c]; ++p) pos.push_back(p);
+      off.push_back(static_cast<int32_t>(pos.size()));
+    }
+  };
+  auto orders = [](const std::vector<int32_t>& pos, const std::vector<int32_t>& order) {
+    std::vector<int32_t> o(pos.size());
+    for (size_t k = 0; k < pos.size(); ++k) o[k] = order[pos[k]];
+    return o;
+  };
+  std::vector<std::vector<int32_t>> spos(ni), bpos(ni);
+  std::vector<int2> sent;
+  std::vector<int4> bent;
+  HostPlan H;
+  const bool made = MakePlan(
+      ctx, nb, ns,
+      [&](int i) {
+        const HostInstance& h = ctx->inst[i];
+        std::vector<int32_t> soff, boff;
+        reversed(h.s_coloff, spos[i], soff);
+        reversed(h.b_coloff, bpos[i], boff);
+        return std::vector<PatchFamily>{Family(4, h.bends, orders(bpos[i], h.b_order), boff),
+                                        Family(2, h.edges, orders(spos[i], h.s_order), soff)};
+      },
+      [&](int i, int p, const uint16_t* l) {
+        const int q = bpos[i][p & 0x7fffffff] | (p & static_cast<int>(0x80000000u));
+        bent.push_back(make_int4(Pack16(l[0], l[1]), Pack16(l[2], l[3]), Global(q, ctx->inst[i].bbeg), 0));
+      },
+      [&](int i, int p, const uint16_t* l) {
+        const int q = spos[i][p & 0x7fffffff] | (p & static_cast<int>(0x80000000u));
+        sent.push_back(make_int2(Pack16(l[0], l[1]), Global(q, ctx->inst[i].sbeg)));
+      },
+      P.adj, H, kPatchAdjVertBytes, true);
+  if (!made) return XRT_OK;
+  hipStream_t s = ctx->stream;
+  hipError_t e = P.adj.patch.Upload(H.dev, s);
+  if (e == hipSuccess) e = P.adj.verts.Upload(H.verts, s);
+  if (e == hipSuccess) e = P.adj.off.Upload(H.off, s);
+  if (e == hipSuccess) e = P.bent.Upload(bent, s);
+  if (e == hipSuccess) e = P.sent.Upload(sent, s);
+  if (e == hipSuccess) e = P.glam.Alloc(std::max<size_t>(sent.size(), 1));
+  return FinishPlan(P.adj, e, ConfigurePatchAdj, P.bent, P.sent, P.glam);
+}
+
+int PatchAdjIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, bool first,
+                 const float4* tape_b, const float4* tape_s) {
+  PatchData& P = ctx->patches;
+  AdjointData& A = *ctx->adj;
+  const PatchPlanDev& D = P.adj;
+  if (A.gx_alt.n != A.gx.n) XRT_CHECK_HIP(A.gx_alt.Alloc(A.gx.n));
+  const PatchAdjArgs a{D.patch.ptr, D.verts.ptr, D.off.ptr, P.bent.ptr,   P.sent.ptr,
+                       ctx->bpar.ptr, ctx->sc.ptr, ctx->x0.ptr, A.gx.ptr, A.gx_alt.ptr,
+                       P.glam.ptr,  A.gcomp.ptr, A.gbcomp.ptr, D.n, D.c0, D.c1};
+  XRT_CHECK_HIP(LaunchPatchAdj(ctx->stream, a, k.inv_dt2, m, k.solve_bending ? 1 : 0, first ? 1 : 0,
+                               tape_b, tape_s, D.threads, D.lds_bytes));
+  std::swap(A.gx.ptr, A.gx_alt.ptr);
+  return XRT_OK;
 }
 
 const PatchPlanDev& PatchPlanOf(const xrt_ctx* ctx) {
