@@ -273,6 +273,11 @@ int WideSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, AdjointData
                   : nullptr;
   bool obs_contact = false;
   for (int i = 0; i < n_inst; ++i) obs_contact = obs_contact || ObsContact(c, i);
+  // the vertex-face solves end the sweep when every patch has a CU (one launch of 4.5 us and its
+  // gap less an iteration, 1.6 us more sweep); with more patches than CUs their loads, at a few
+  // waves a CU, cost more than the launch (256 cloths: 344 us against 295 + 18)
+  const bool sweep_vf =
+      sweep && obs_contact && c->total_slots == 0 && PatchPlanOf(c).n <= c->cu_count;
   int rc;
   if ((rc = MultiContactSubstepBegin(c)) != XRT_OK) return rc;
   if (T) XRT_CHECK_HIP(LaunchCopy4(s, T, c->x0.ptr, N));
@@ -299,10 +304,10 @@ int WideSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, AdjointData
       for (int i = 0; i < n_inst; ++i)
         if (ObsContact(c, i) && (rc = SnapshotRecords(c, i, c->contact[i]->pass_cnt - 1)) != XRT_OK)
           return rc;
-    if (sweep) {  // every color (and the ground plane, when it comes next) in one launch
-      if ((rc = PatchIter(c, k, bm, it, sweep_ground, TI ? TI + A->off_s : nullptr,
-                          TI ? TI + A->off_b : nullptr, TI ? TI + A->off_g : nullptr)) != XRT_OK)
-        return rc;
+    if (sweep) {  // every color (and what comes next a vertex at a time) in one launch
+      PatchTape t;
+      if (TI) t = PatchTape{TI + A->off_s, TI + A->off_b, TI + A->off_g, TI + A->off_c, TI + A->off_e};
+      if ((rc = PatchIter(c, k, bm, it, sweep_ground, sweep_vf, t)) != XRT_OK) return rc;
     } else if (FemOn(c)) {  // never taped: the adjoint refuses the FEM constraints
       if ((rc = FemIter(c, -1, it)) != XRT_OK) return rc;
     } else {
@@ -330,9 +335,11 @@ int WideSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, AdjointData
       XRT_CHECK_HIP(LaunchGround(s, c->xcur, c->x0.ptr, N, k.ground_y, k.friction));
     }
     if (obs_contact) {
-      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_c, c->xcur, N));
-      if ((rc = MultiContactVfSolve(c)) != XRT_OK) return rc;
-      if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_e, c->xcur, N));
+      if (!sweep_vf) {
+        if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_c, c->xcur, N));
+        if ((rc = MultiContactVfSolve(c)) != XRT_OK) return rc;
+        if (TI) XRT_CHECK_HIP(LaunchCopy4(s, TI + A->off_e, c->xcur, N));
+      }
       if ((rc = MultiContactEeSolve(c)) != XRT_OK) return rc;
     }
     if ((rc = BindingIter(c, -1)) != XRT_OK) return rc;  // never taped: the adjoint refuses

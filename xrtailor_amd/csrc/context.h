@@ -445,8 +445,12 @@ int FemIter(xrt_ctx* ctx, int inst, int it);
 int PatchPrepare(xrt_ctx* ctx);
 int PatchPrepareFem(xrt_ctx* ctx);
 const PatchPlanDev& PatchPlanOf(const xrt_ctx* ctx);  // of the current constraint model
+// ground, contacts: the sweep goes on with the ground plane, with the vertex-face solves
+struct PatchTape {
+  float4 *s = nullptr, *b = nullptr, *g = nullptr, *c = nullptr, *e = nullptr;
+};
 int PatchIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, int it, bool ground,
-              float4* tape_s, float4* tape_b, float4* tape_g);
+              bool contacts, const PatchTape& t);
 int PatchRefreshCompliance(xrt_ctx* ctx);
 int PatchPrepareAdj(xrt_ctx* ctx);
 int PatchAdjIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, bool first,

@@ -26,6 +26,7 @@
 
 #include <cstdint>
 
+#include "contact.h"
 #include "device.h"
 
 namespace xrt {
@@ -33,6 +34,7 @@ namespace xrt {
 struct PatchDev {
   int32_t vbeg, n_own, n_loc;  // verts[vbeg, vbeg + n_loc)
   int32_t off;                 // the patch's color offsets
+  int32_t inst;
 };
 
 constexpr int kPatchMaxOffsets = 128;  // stretch + bend colors + 2 that a sweep can hold
@@ -62,8 +64,8 @@ struct PatchFemArgs {
   int n, nf, nb;
 };
 
-// What a sweep does beside the constraints: ground plane after them (before any later
-// operator of the iteration), tape of the operators' inputs (see adjoint.h; null: none)
+// What a sweep does beside the constraints: ground plane and vertex-face contacts after them
+// (before any later operator of the iteration), tape of the operators' inputs (see adjoint.h; null: none)
 struct PatchSweep {
   const float4* x;   // input positions
   float4* out;       // output positions (not x)
@@ -73,6 +75,12 @@ struct PatchSweep {
   float4* tape_s;
   float4* tape_b;
   float4* tape_g;
+  // the vertex-face solves against the obstacles (null: they follow as a launch of their own),
+  // with the tape of the positions before and after them
+  const InstContactDev* ic;
+  float mu, inv_ns;
+  float4* tape_c;
+  float4* tape_e;
 };
 
 hipError_t LaunchPatchSweep(hipStream_t s, const PatchArgs& a, const PatchSweep& w,

@@ -111,6 +111,7 @@ bool MakePlan(xrt_ctx* ctx, int c0, int c1, Families&& families, Entry0&& entry0
       d.n_own = q.n_own;
       d.n_loc = static_cast<int32_t>(q.verts.size());
       d.off = static_cast<int32_t>(H.off.size());
+      d.inst = i;
       H.dev.push_back(d);
       max_loc = std::max(max_loc, q.verts.size());
       for (int32_t v : q.verts) H.verts.push_back(ctx->inst[i].desc.vbeg + v);
@@ -348,12 +349,14 @@ const PatchPlanDev& PatchPlanOf(const xrt_ctx* ctx) {
 }
 
 int PatchIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, int it, bool ground,
-              float4* tape_s, float4* tape_b, float4* tape_g) {
+              bool contacts, const PatchTape& t) {
   PatchData& P = ctx->patches;
   const PatchPlanDev& D = PatchPlanOf(ctx);
   float4* out = ctx->xcur == ctx->x.ptr ? P.alt.ptr : ctx->x.ptr;
   const PatchSweep w{ctx->xcur, out, ctx->x0.ptr, it, it + 1 == k.iterations ? 1 : 0,
-                     ground ? 1 : 0, tape_s, tape_b, tape_g};
+                     ground ? 1 : 0, t.s, t.b, t.g, contacts ? ctx->ic.ptr : nullptr,
+                     ctx->params.contact_friction,
+                     1.0f / static_cast<float>(ctx->params.num_substeps), t.c, t.e};
   const int threads = ctx->tuning.wide_per_thread == 2 ? std::max(64, (D.threads / 2 + 63) / 64 * 64)
                                                        : D.threads;
   if (FemOn(ctx)) {
