@@ -143,8 +143,9 @@ struct InstContactDev {
   uint32_t* iee = nullptr;
   uint2* nitem = nullptr;
   // pair refresh: the first kPairStage hits of each cloth leaf, hit j of leaf i at
-  // stage[j * nf + i] as rhs object | item mask << kStageObjBits (null: the pairs are found
-  // by a second traversal; also for meshes of 2^kStageObjBits faces or more)
+  // stage[j * nf + i] as rhs object | item mask << kStageObjBits, or with the item lists on the
+  // first kCoupleStage couples of the cloth pass as two words, object and CoupleMask (null: the
+  // pairs are found by a second traversal; also for meshes of 2^kStageObjBits faces or more)
   uint32_t* stage = nullptr;
   // pair refresh: per 256-leaf block of the count pass, its pair / VF / EE item sums
   // (3 x Blocks(nf)), then their exclusive prefix
