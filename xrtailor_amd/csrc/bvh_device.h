@@ -469,7 +469,8 @@ __device__ __forceinline__ void RadixScatterBody(
 
 // exclusive scan of n uint32 in place by one 1024-thread workgroup; *total (if given)
 // receives the sum.  4096 elements a step, neighboring threads on neighboring elements: a
-// contiguous run per thread took 33 us for the 16 k counters of a 130 k face sort, this 11.49 us on average.
+// contiguous run per thread took 33 us a scan of a 64 k face tree's sort and pair counts, this
+// 11 us.
 __device__ __forceinline__ void BlockExclusiveScan(uint32_t* __restrict__ a, int n,
                                                    int32_t* __restrict__ total) {
   constexpr int kRows = 4, kWaves = 16;
