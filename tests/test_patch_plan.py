@@ -69,7 +69,10 @@ int main(int argc, char** argv) {
     id += n;
   }
   std::vector<Patch> plan;
-  if (!BuildPatches(pos.data(), nv, fam, target, max_local, max_work, &plan)) {
+  const int n_total = argc > 6 ? atoi(argv[6]) : 0;  // > 0: the sizes of such a context on 256 CUs
+  if (!(n_total > 0 ? CutInstance(pos.data(), nv, fam, ChoosePatchSizes(n_total, 256), max_local,
+                                  max_work, &plan)
+                    : BuildPatches(pos.data(), nv, fam, target, max_local, max_work, &plan))) {
     printf("no plan\n");
     return plan.empty() ? 42 : 11;
   }
@@ -132,6 +135,8 @@ def driver(tmp_path_factory):
 def _mesh(kind):
     if kind == "grid":
         return scenes.grid(33, 1.0)
+    if kind.startswith("grid"):
+        return scenes.grid(int(kind[4:]), 1.0)
     if kind == "strip":
         pos, tris = scenes.grid(41, 1.0)
         keep = np.all(tris < 5 * 41, axis=1)
@@ -147,11 +152,11 @@ def _mesh(kind):
     return rng.rand(60, 3), tris
 
 
-def _run(driver, kind, mode, target, max_local, first, max_work):
+def _run(driver, kind, mode, target, max_local, first, max_work, n_total=0):
     pos, tris = _mesh(kind)
     text = f"{len(pos)} {len(tris)}\n" + " ".join(f"{v:.9g}" for v in np.ravel(pos)) + "\n" + \
         " ".join(str(v) for v in np.ravel(tris)) + "\n"
-    r = subprocess.run([str(driver), *map(str, (mode, target, max_local, first, max_work))],
+    r = subprocess.run([str(driver), *map(str, (mode, target, max_local, first, max_work, n_total))],
                        input=text, capture_output=True, text=True)
     print(r.stdout.strip())
     return r.returncode
@@ -169,3 +174,13 @@ def test_no_plan_beyond_the_work_or_size_limit(driver):
     assert _run(driver, "grid", 0, 64, 10240, 1, 2.0) == 42   # needs six times the constraints
     assert _run(driver, "grid", 0, 64, 50, 1, 1e9) == 42      # one vertex needs more than 50
     assert _run(driver, "grid", 0, 2000, 10240, 1, 1.0) == 0  # one patch: nothing twice
+
+
+# cloths of 40,960 vertices and more in contexts where an instance of their size is to stay whole
+# (more vertices than that per CU), and around; 5,851 vertices hold the reverse sweep's adjoints
+@pytest.mark.parametrize("kind,copies", [("grid203", 204), ("grid203", 210), ("grid256", 216),
+                                         ("grid100", 1000), ("grid203", 1)])
+@pytest.mark.parametrize("first,max_local", [(1, 10240), (0, 10240), (1, 5851)])
+def test_instances_of_any_size_get_a_plan(driver, kind, copies, first, max_local):
+    n_total = copies * int(kind[4:]) ** 2
+    assert _run(driver, kind, 0, 0, max_local, first, 6.0, n_total) == 0

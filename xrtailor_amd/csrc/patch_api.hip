@@ -81,25 +81,12 @@ bool MakePlan(xrt_ctx* ctx, int c0, int c1, Families&& families, Entry0&& entry0
   const int ni = static_cast<int>(ctx->inst.size());
   const int max_local = static_cast<int>(
       std::min<size_t>(kPatchMaxVerts, std::min<size_t>(ctx->max_lds, kPatchMaxLds) / vert_bytes));
-  // Own vertices per patch: what gives 4 of 5 CUs a patch, down to 256 vertices, where the
-  // ring of neighbors already quadruples the stretch work of a grid, and up to 4096 (a grid's
-  // patch then needs 117 KB of LDS, 1.4x the stretch and 1.2x the bend work).  ms per frame at
-  // 144 / 256 / 400 / 1024 / 2304 / 4096 own vertices: one 64 x 64 cloth 2.22 / 2.28 / 2.40 /
-  // 2.75 / 3.51 / 4.43, 16 garments (93 k vertices) - / 10.3 / 8.25 / 8.66 / 9.67 / 10.5, 256
-  // cloths (2.53 M vertices) 115 / 108 / 75 / 44.6 / 29.3 / 23.7.  An instance stays whole
-  // (nothing is solved twice) when there are patches enough without cutting it, and below
-  // 1200 vertices, where a color takes one or two rounds of one workgroup anyway.
-  const int per_cu = ctx->wide.n_total / std::max(1, ctx->cu_count * 4 / 5);
-  const int cut = std::min(4096, std::max(256, per_cu)), whole = std::max(1200, per_cu);
+  const PatchSizes sizes = ChoosePatchSizes(ctx->wide.n_total, ctx->cu_count);
   std::vector<std::vector<Patch>> plan(ni);
   const bool built = ParallelFor(ni, [&](int i) {
     const HostInstance& h = ctx->inst[i];
     const std::vector<PatchFamily> fam = families(i);
-    // a mesh with little locality gets larger patches, or none
-    for (int target = h.nv <= whole ? h.nv : cut; target < 4 * kPatchMaxVerts; target *= 4)
-      if (BuildPatches(h.rest_pos.data(), h.nv, fam, target, max_local, kPatchMaxWork, &plan[i]))
-        return true;
-    return false;
+    return CutInstance(h.rest_pos.data(), h.nv, fam, sizes, max_local, kPatchMaxWork, &plan[i]);
   });
   if (!built) return false;
   size_t max_loc = 0, n0 = 0, n1 = 0;

@@ -148,4 +148,26 @@ bool BuildPatches(const float* pos, int nv, const std::vector<PatchFamily>& fami
   return true;
 }
 
+// Own vertices per patch: what gives 4 of 5 CUs a patch, down to 256 vertices, where the
+// ring of neighbors already quadruples the stretch work of a grid, and up to 4096 (a grid's
+// patch then needs 117 KB of LDS, 1.4x the stretch and 1.2x the bend work).  ms per frame at
+// 144 / 256 / 400 / 1024 / 2304 / 4096 own vertices: one 64 x 64 cloth 2.22 / 2.28 / 2.40 /
+// 2.75 / 3.51 / 4.43, 16 garments (93 k vertices) - / 10.3 / 8.25 / 8.66 / 9.67 / 10.5, 256
+// cloths (2.53 M vertices) 115 / 108 / 75 / 44.6 / 29.3 / 23.7.  An instance stays whole
+// (nothing is solved twice) when there are patches enough without cutting it, and below
+// 1200 vertices, where a color takes one or two rounds of one workgroup anyway.
+PatchSizes ChoosePatchSizes(int n_total, int cu_count) {
+  const int per_cu = n_total / std::max(1, cu_count * 4 / 5);
+  return PatchSizes{std::min(4096, std::max(256, per_cu)), std::max(1200, per_cu)};
+}
+
+bool CutInstance(const float* pos, int nv, const std::vector<PatchFamily>& families, PatchSizes sizes,
+                 int max_local, double max_work, std::vector<Patch>* out) {
+  // (BuildPatches halves what a workgroup cannot hold, however large the instance is)
+  if (nv <= sizes.whole) return BuildPatches(pos, nv, families, nv, max_local, max_work, out);
+  for (int target = sizes.cut; target < 40960; target *= 4)
+    if (BuildPatches(pos, nv, families, target, max_local, max_work, out)) return true;
+  return false;
+}
+
 }  // namespace xrt

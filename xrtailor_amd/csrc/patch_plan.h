@@ -41,4 +41,16 @@ struct Patch {
 bool BuildPatches(const float* pos, int nv, const std::vector<PatchFamily>& families, int target,
                   int max_local, double max_work, std::vector<Patch>* out);
 
+// How a context's instances are cut: one of up to `whole` vertices stays whole (as far as
+// max_local allows), a larger one gets patches of about `cut` own vertices.
+struct PatchSizes {
+  int cut, whole;
+};
+PatchSizes ChoosePatchSizes(int n_total, int cu_count);
+
+// BuildPatches for one instance at these sizes.  A mesh with little locality gets larger patches,
+// or none.
+bool CutInstance(const float* pos, int nv, const std::vector<PatchFamily>& families, PatchSizes sizes,
+                 int max_local, double max_work, std::vector<Patch>* out);
+
 }  // namespace xrt
