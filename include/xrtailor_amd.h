@@ -133,10 +133,11 @@ typedef struct xrt_tuning {
                               * constraint launches: 1 (default) or 2 (half the threads) */
   int32_t path;              /* 0 persistent substep (one workgroup per instance), 1 wide
                               * substep (each instance over as many workgroups as it needs;
-                              * the colors of an iteration in one launch).  xrt_start sets
-                              * the default from the instances' sizes; contexts with
-                              * contacts, particles or bindings always take the wide
-                              * substep */
+                              * the colors of an iteration in one launch).  Until
+                              * xrt_set_tuning or xrt_autotune has set it, xrt_start and
+                              * xrt_set_params choose it by the instances' sizes and the
+                              * constraint model; contexts with contacts, particles or
+                              * bindings always take the wide substep */
   float best_ms;             /* set by xrt_autotune: ms per substep of the chosen shapes */
   float default_ms;          /* set by xrt_autotune: ms per substep of the defaults */
   int32_t candidates;        /* set by xrt_autotune: configurations timed */

@@ -111,3 +111,44 @@ def test_autotune_between_substeps_of_a_frame_changes_nothing():
         runs.append(_states(s, ids))
         s.close()
     _equal(runs[0], runs[1])
+
+
+def _pinwheel(k):
+    """k triangles around one vertex: 2 k edge colors, k face colors, no hinges"""
+    a = np.pi * np.arange(2 * k) / k
+    pos = np.concatenate([[[0, 0, 0]], np.stack([np.cos(a), 0 * a, np.sin(a)], 1)])
+    i = np.arange(k)
+    tris = np.stack([0 * i, 1 + 2 * i, 2 + 2 * i], 1).astype(np.int32)
+    return scenes.ClothSpec(pos, tris, np.zeros(0, np.int32), 1e-6, 1e-3, pos.astype(np.float32))
+
+
+def test_path_set_by_the_caller_stays_and_the_default_follows_the_model():
+    print("case tuning set before the start; the default path by constraint model", flush=True)
+    specs = [scenes.hanging_cloth(seed=1, n=64), _pinwheel(80)]
+    xp = make_params(bend_model=1, num_substeps=2, num_iterations=2)
+    for path in (0, 1):
+        s, ids = build_solver(specs[:1], xp, seed=4,
+                              before_start=lambda s, _: s.set_tuning(512, 1, 2, path))
+        t = s.tuning()
+        assert (t["persistent_block"], t["persistent_unroll"], t["wide_per_thread"],
+                t["path"]) == (512, 1, 2, path)
+        s.set_params(s.params)
+        assert s.tuning()["path"] == path
+        s.close()
+    s, ids = build_solver(specs[:1], xp, seed=4)
+    assert s.tuning()["path"] == 1                  # cut into patches
+    s.close()
+    # too many edge colors for a sweep, few enough face colors
+    runs = []
+    for batched in (True, False):
+        s, ids = build_solver(specs, xp, seed=4)
+        for model, path in ((0, 0), (1, 1), (0, 0)):
+            p = s.params
+            p.constraint_model = model
+            s.set_params(p)
+            assert s.tuning()["path"] == path
+            s.FramesBatched(1) if batched else s.FramesPlain(1)
+        s.sync()
+        runs.append(_states(s, ids))
+        s.close()
+    _equal(*runs)

@@ -568,6 +568,7 @@ int xrt_set_params(xrt_ctx* ctx, const xrt_params* p) {
   int rc = FemPrepare(ctx);
   if (rc != XRT_OK) return rc;
   if (!FemOn(ctx) && !ctx->patches.xpbd.tried && (rc = PatchPrepare(ctx)) != XRT_OK) return rc;
+  if (!ctx->tuning_set) ctx->tuning.path = DefaultPath(ctx);  // (the model may have changed)
   if (lists && (rc = ContactResizeLists(ctx)) != XRT_OK) return rc;
   return ParticleConfigure(ctx);
 }
@@ -892,7 +893,7 @@ int xrt_start(xrt_ctx* ctx, uint64_t seed) {
   if ((rc = BindingStart(ctx)) != XRT_OK) return rc;
   ctx->fem.seed = seed;
   if ((rc = FemPrepare(ctx)) != XRT_OK) return rc;
-  ctx->tuning.path = DefaultPath(ctx);
+  if (!ctx->tuning_set) ctx->tuning.path = DefaultPath(ctx);
   ctx->started = true;
   return XRT_OK;
 }
@@ -1125,6 +1126,7 @@ int xrt_set_tuning(xrt_ctx* ctx, const xrt_tuning* t) {
   ctx->tuning.persistent_unroll = t->persistent_unroll;
   ctx->tuning.wide_per_thread = t->wide_per_thread;
   ctx->tuning.path = t->path;
+  ctx->tuning_set = true;
   DestroyGraph(ctx);  // the next batched frame captures the new shapes
   return XRT_OK;
 }
@@ -1187,6 +1189,7 @@ int xrt_autotune(xrt_ctx* ctx, int32_t substeps, xrt_tuning* out) {
   best.default_ms = default_ms;
   best.candidates = static_cast<int32_t>(cand.size());
   ctx->tuning = best;
+  ctx->tuning_set = true;
   DestroyGraph(ctx);
   if ((rc = CheckPairOverflow(ctx)) != XRT_OK) return rc;
   if (out) *out = best;

@@ -326,6 +326,7 @@ struct xrt_ctx {
   // batched launch configuration
   // launch shapes picked by xrt_autotune (defaults until it runs); none changes a result
   xrt_tuning tuning{1024, 0, 1, 0, 0.0f, 0.0f, 0};
+  bool tuning_set = false;  // by xrt_set_tuning or xrt_autotune: the path is no default
   size_t batched_lds = 0;
   int lds_verts = 0;
   int max_slots = 0;
