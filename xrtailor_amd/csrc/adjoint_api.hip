@@ -96,7 +96,7 @@ int AdjSetup(xrt_ctx* c, int want_slots = 1) {
     XRT_CHECK_HIP(A.slot_inst.Upload(sinst, c->stream));
     XRT_CHECK_HIP(A.slot_ptr.Upload(cnt, c->stream));
     XRT_CHECK_HIP(A.slot_cons.Upload(cons, c->stream));
-    if (A.lra_xs.n < cons.size()) {
+    if (A.lra_gslot.n < cons.size()) {  // (the last of a group: all are there)
       XRT_CHECK_HIP(A.lra_xs.Alloc(cons.size()));
       XRT_CHECK_HIP(A.lra_gslot.Alloc(cons.size()));
     }
@@ -178,14 +178,14 @@ int AdjSetup(xrt_ctx* c, int want_slots = 1) {
     }
     A.rec[i] = std::move(r);
   }
-  if (A.gx0.n != N) {
+  if (A.ee_cnt.n != N) {
     XRT_CHECK_HIP(A.gx0.Alloc(N));
     XRT_CHECK_HIP(A.gv.Alloc(N));
     XRT_CHECK_HIP(A.gx.Alloc(N));
     XRT_CHECK_HIP(A.ee_cnt.Alloc(N));
     XRT_CHECK_HIP(hipMemsetAsync(A.ee_cnt.ptr, 0, sizeof(int32_t) * N, c->stream));
   }
-  if (A.glam.n != static_cast<size_t>(std::max(A.e_total, 1))) {
+  if (A.gcomp.n != static_cast<size_t>(std::max(A.e_total, 1))) {
     XRT_CHECK_HIP(A.glam.Alloc(std::max(A.e_total, 1)));
     XRT_CHECK_HIP(A.gcomp.Alloc(std::max(A.e_total, 1)));
   }
@@ -197,7 +197,7 @@ int AdjSetup(xrt_ctx* c, int want_slots = 1) {
     if (A.rep_count.n != static_cast<size_t>(A.slots)) XRT_CHECK_HIP(A.rep_count.Alloc(A.slots));
     if (A.rep_marks.n != marks) XRT_CHECK_HIP(A.rep_marks.Alloc(marks));
     if (A.rep_flags.n != 1) XRT_CHECK_HIP(A.rep_flags.Alloc(1));
-    if (A.rep_cnt.n != N) {
+    if (A.rep_add.n != 6 * N) {
       XRT_CHECK_HIP(A.rep_cnt.Alloc(N));
       XRT_CHECK_HIP(A.rep_add.Alloc(6 * N));
     }

@@ -42,11 +42,17 @@ struct DevBuf {
     ptr = nullptr;
     n = 0;
   }
+  // n is count only when the memory is there: callers that keep a buffer of the right n must not
+  // take a null one for it after a failure
   hipError_t Alloc(size_t count) {
     Free();
-    n = count;
     if (count == 0) return hipSuccess;
-    return hipMalloc(reinterpret_cast<void**>(&ptr), count * sizeof(T));
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&ptr), count * sizeof(T));
+    if (e == hipSuccess)
+      n = count;
+    else
+      ptr = nullptr;
+    return e;
   }
   // The copy has completed when this returns: callers upload from temporaries (set-up
   // vectors that die at the end of their scope), and HIP does not promise that an
