@@ -2,9 +2,12 @@
 mirrors an instance (same topology, colors, LRA CSR and FP32-rounded state)."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 
 from oracle import oracle as orc
+from xrtailor_amd import _ffi
 from xrtailor_amd.solver import ClothSolver, build_solver, make_params  # noqa: F401
 
 
@@ -13,6 +16,13 @@ def rel_err(x, ref) -> float:
     x = np.asarray(x, np.float64)
     ref = np.asarray(ref, np.float64)
     return float(np.abs(x - ref).max() / max(np.abs(ref).max(), 1.0))
+
+
+def free_device_memory() -> int:
+    """Free bytes of the device, from the HIP runtime that the library is linked with."""
+    free, total = C.c_size_t(), C.c_size_t()
+    assert _ffi.load().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
 
 
 def build(specs, params, seed=0):

@@ -4,6 +4,7 @@ lists within their sizes and beyond them."""
 import numpy as np
 import pytest
 
+from gpu_helpers import free_device_memory
 from xrtailor_amd import scenes
 from xrtailor_amd._ffi import XrtError
 from xrtailor_amd.solver import build_solver, make_params
@@ -74,3 +75,29 @@ def test_large_obstacle_matches_plain(side):
         np.testing.assert_array_equal(u, v)
     c = a.Contacts(ia[0])
     assert c["pairs"] == b.Contacts(ib[0])["pairs"] and c["obs_pairs"] > 1000
+
+
+def test_lists_without_room_for_vertex_ids_match_small_ones():
+    """Item lists of 0.7 of the free memory: their 16-bit vertex ids do not fit beside all of them."""
+    n = 17
+    faces = 2 * (n - 1) ** 2
+    cap = (2 ** 31 - 1) // (9 * faces)              # pairs a face: the largest with lists on
+    free = free_device_memory()
+    k = int(0.7 * free / (8 * 13 * cap * faces))    # pairs, 3 VF and 9 EE items each
+    print(f"case lists of {k} x {8e-9 * 13 * cap * faces:.1f} GB of {1e-9 * free:.0f} GB",
+          flush=True)
+    assert k >= 1
+    specs = [_crumpled(n, 40 + j, 0.2) for j in range(k)]
+    runs = []
+    for kw in (dict(pair_capacity_per_face=cap, repulsion_vf_items_per_face=3 * cap,
+                    repulsion_ee_items_per_face=9 * cap), dict(pair_capacity_per_face=128)):
+        s, ids = build_solver(specs, make_params(bend_model=1, enable_self_contact=1,
+                                                 ground_height=-1.0, num_substeps=2,
+                                                 num_iterations=3, **kw), seed=3)
+        s.FramesBatched(2)
+        s.sync()
+        runs.append([a for i in ids for a in s.GetState(i)])
+        s.close()
+        print("  ran", flush=True)
+    for a, b in zip(*runs):
+        np.testing.assert_array_equal(a, b)

@@ -893,6 +893,7 @@ int xrt_start(xrt_ctx* ctx, uint64_t seed) {
   if ((rc = BindingStart(ctx)) != XRT_OK) return rc;
   ctx->fem.seed = seed;
   if ((rc = FemPrepare(ctx)) != XRT_OK) return rc;
+  if ((rc = ContactItemIds(ctx)) != XRT_OK) return rc;
   if (!ctx->tuning_set) ctx->tuning.path = DefaultPath(ctx);
   ctx->started = true;
   return XRT_OK;

@@ -138,10 +138,6 @@ int AllocPairLists(xrt_ctx* ctx, const HostInstance& h, ContactData& c) {
     c.ee_cap = static_cast<int>(std::min<int64_t>(ee_cap, 9 * static_cast<int64_t>(c.pair_cap)));
     XRT_CHECK_HIP(c.rep_vf.Alloc(c.vf_cap));
     XRT_CHECK_HIP(c.rep_ee.Alloc(c.ee_cap));
-    if (std::max(h.nv, h.obs_nv()) <= 1 << 16) {
-      XRT_CHECK_HIP(c.ids_vf.Alloc(c.vf_cap));
-      XRT_CHECK_HIP(c.ids_ee.Alloc(c.ee_cap));
-    }
     if (!c.ivf.ptr) XRT_CHECK_HIP(c.ivf.Alloc(std::max(h.nt, 1)));
     if (!c.iee.ptr) XRT_CHECK_HIP(c.iee.Alloc(std::max(h.nt, 1)));
     if (!c.nitem.ptr) XRT_CHECK_HIP(c.nitem.Alloc(std::max(h.nt, 1)));
@@ -415,7 +411,8 @@ int ContactResizeLists(xrt_ctx* ctx) {
     const int rc = AllocPairLists(ctx, ctx->inst[k], *ctx->contact[k]);
     if (rc != XRT_OK) return rc;
   }
-  return MultiContactSetup(ctx);
+  const int rc = MultiContactSetup(ctx);
+  return rc != XRT_OK ? rc : ContactItemIds(ctx);
 }
 
 int CheckPairOverflow(xrt_ctx* ctx) {
@@ -434,9 +431,62 @@ int CheckPairOverflow(xrt_ctx* ctx) {
   return XRT_ERR_CAPACITY;
 }
 
+namespace {
+// the device records of every instance's contact data
+std::vector<InstContactDev> ContactViews(const xrt_ctx* ctx) {
+  std::vector<InstContactDev> ic(std::max<size_t>(ctx->inst.size(), 1));
+  for (size_t k = 0; k < ctx->inst.size(); ++k) {
+    if (!ctx->contact[k]) continue;
+    const HostInstance& h = ctx->inst[k];
+    const ContactData& c = *ctx->contact[k];
+    InstContactDev& d = ic[k];
+    d.vbeg = h.desc.vbeg;
+    d.nv = h.nv;
+    d.nf = h.nt;
+    d.ne = h.ne();
+    d.has_obs = c.obs_nf > 0;
+    d.obs_nv = c.obs_nv;
+    d.obs_nf = c.obs_nf;
+    d.pair_cap = c.pair_cap;
+    d.cloth = ClothTopo(c, h);
+    d.obs = ObsTopo(c);
+    d.cbvh = c.cloth_bvh.view();
+    d.obvh = c.obs_bvh.view();
+    d.o_x0 = c.o_x0.ptr;
+    d.o_x = c.o_x.ptr;
+    d.o_x1 = c.o_x1.ptr;
+    d.o_n1 = c.o_n1.ptr;
+    d.o_vptr = c.o_vptr.ptr;
+    d.o_corner = c.o_corner.ptr;
+    d.vf_face = c.vf_face.ptr;
+    d.rt_face = c.rt_face.ptr;
+    d.vf_q = c.vf_q.ptr;
+    d.rt_q = c.rt_q.ptr;
+    d.ee = reinterpret_cast<EeRec*>(c.ee.ptr);
+    d.ee_none = c.ee_none.ptr;
+    d.dq = c.dq.ptr;
+    d.cnt = c.cnt.ptr;
+    d.pairs = c.pairs.ptr;
+    d.scal = c.scal.ptr;
+    d.vf_cap = c.vf_cap;
+    d.ee_cap = c.ee_cap;
+    d.rep_vf = c.rep_vf.ptr;
+    d.rep_ee = c.rep_ee.ptr;
+    d.ids_vf = c.ids_vf.ptr;
+    d.ids_ee = c.ids_ee.ptr;
+    d.stage = c.stage.ptr;
+    d.bsum = c.bsum.ptr;
+    d.overflow = ctx->overflow.ptr;
+    d.ivf = c.ivf.ptr;
+    d.iee = c.iee.ptr;
+    d.nitem = c.nitem.ptr;
+  }
+  return ic;
+}
+}  // namespace
+
 int MultiContactSetup(xrt_ctx* ctx) {
   const int n = static_cast<int>(ctx->inst.size());
-  std::vector<InstContactDev> ic(std::max(n, 1));
   std::vector<int32_t> off(MultiMaps::kKinds * static_cast<size_t>(n + 1), 0);
   auto blocks = [](int count) { return (count + 255) / 256; };
   bool cloth_top = false, obs_top = false;
@@ -454,49 +504,8 @@ int MultiContactSetup(xrt_ctx* ctx) {
   for (int k = 0; k < n; ++k) {
     int cnt[MultiMaps::kKinds] = {};
     if (ctx->contact[k]) {
-      HostInstance& h = ctx->inst[k];
-      ContactData& c = *ctx->contact[k];
-      InstContactDev& d = ic[k];
-      d.vbeg = h.desc.vbeg;
-      d.nv = h.nv;
-      d.nf = h.nt;
-      d.ne = h.ne();
-      d.has_obs = c.obs_nf > 0;
-      d.obs_nv = c.obs_nv;
-      d.obs_nf = c.obs_nf;
-      d.pair_cap = c.pair_cap;
-      d.cloth = ClothTopo(c, h);
-      d.obs = ObsTopo(c);
-      d.cbvh = c.cloth_bvh.view();
-      d.obvh = c.obs_bvh.view();
-      d.o_x0 = c.o_x0.ptr;
-      d.o_x = c.o_x.ptr;
-      d.o_x1 = c.o_x1.ptr;
-      d.o_n1 = c.o_n1.ptr;
-      d.o_vptr = c.o_vptr.ptr;
-      d.o_corner = c.o_corner.ptr;
-      d.vf_face = c.vf_face.ptr;
-      d.rt_face = c.rt_face.ptr;
-      d.vf_q = c.vf_q.ptr;
-      d.rt_q = c.rt_q.ptr;
-      d.ee = reinterpret_cast<EeRec*>(c.ee.ptr);
-      d.ee_none = c.ee_none.ptr;
-      d.dq = c.dq.ptr;
-      d.cnt = c.cnt.ptr;
-      d.pairs = c.pairs.ptr;
-      d.scal = c.scal.ptr;
-      d.vf_cap = c.vf_cap;
-      d.ee_cap = c.ee_cap;
-      d.rep_vf = c.rep_vf.ptr;
-      d.rep_ee = c.rep_ee.ptr;
-      d.ids_vf = c.ids_vf.ptr;
-      d.ids_ee = c.ids_ee.ptr;
-      d.stage = c.stage.ptr;
-      d.bsum = c.bsum.ptr;
-      d.overflow = ctx->overflow.ptr;
-      d.ivf = c.ivf.ptr;
-      d.iee = c.iee.ptr;
-      d.nitem = c.nitem.ptr;
+      const HostInstance& h = ctx->inst[k];
+      const ContactData& c = *ctx->contact[k];
       cnt[MultiMaps::kVert] = blocks(h.nv);
       cnt[MultiMaps::kEdge] = blocks(h.ne());
       cnt[MultiMaps::kFace] = blocks(h.nt);
@@ -522,7 +531,7 @@ int MultiContactSetup(xrt_ctx* ctx) {
     maps.insert(maps.end(), o, o + n + 1);
     for (int k = 0; k < n; ++k) maps.insert(maps.end(), static_cast<size_t>(o[k + 1] - o[k]), k);
   }
-  XRT_CHECK_HIP(ctx->ic.Upload(ic, ctx->stream));
+  XRT_CHECK_HIP(ctx->ic.Upload(ContactViews(ctx), ctx->stream));
   XRT_CHECK_HIP(ctx->ic_off.Upload(maps, ctx->stream));
   {  // the trees rebuilt at every frame start of the batched path
     std::vector<Lbvh*> ct, ot;
@@ -548,6 +557,39 @@ int MultiContactSetup(xrt_ctx* ctx) {
     ctx->maps.blocks[kind] = off[static_cast<size_t>(kind) * (n + 1) + n];
   }
   XRT_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  return XRT_OK;
+}
+
+// The 16-bit vertex ids of the items (InstContactDev::ids_vf, ids_ee) for the instances whose
+// meshes have no more vertices than that.  They are as large as the lists themselves and the item
+// launches run without them (256 cloths: EE 709 us instead of 426), so they are the last memory
+// taken, a quarter of what is left at most, which leaves room for what is allocated later (the
+// adjoint's tape, recorded frames); instances beyond that go without.
+int ContactItemIds(xrt_ctx* ctx) {
+  size_t left = 0, total = 0;
+  bool any = false;
+  for (size_t k = 0; k < ctx->contact.size(); ++k) {
+    ContactData* c = ctx->contact[k].get();
+    const HostInstance& h = ctx->inst[k];
+    if (!c || c->ee_cap <= 0 || std::max(h.nv, h.obs_nv()) > 1 << 16) continue;
+    if (!any) {
+      XRT_CHECK_HIP(hipMemGetInfo(&left, &total));
+      left /= 4;
+      any = true;
+    }
+    const size_t need = sizeof(uint2) * (static_cast<size_t>(c->vf_cap) + c->ee_cap);
+    if (need > left) continue;
+    if (c->ids_vf.Alloc(c->vf_cap) != hipSuccess || c->ids_ee.Alloc(c->ee_cap) != hipSuccess) {
+      c->ids_vf.Free();
+      c->ids_ee.Free();
+      (void)hipGetLastError();
+      break;
+    }
+    left -= need;
+  }
+  if (!any) return XRT_OK;
+  const std::vector<InstContactDev> ic = ContactViews(ctx);
+  XRT_CHECK_HIP(ctx->ic.Upload(ic.data(), ic.size(), ctx->stream));
   return XRT_OK;
 }
 

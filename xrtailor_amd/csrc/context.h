@@ -401,6 +401,7 @@ int ContactStateReset(xrt_ctx* ctx, int inst);
 // the same phases for every instance at once (multi-instance kernels)
 bool ContactsActive(const xrt_ctx* ctx);
 int MultiContactSetup(xrt_ctx* ctx);
+int ContactItemIds(xrt_ctx* ctx);  // after every other allocation of the start
 int MultiContactSubstepBegin(xrt_ctx* ctx);
 // with `rep_tape` (the adjoint's taped forward): the state before the repulsion pass is
 // copied to rep_tape->x_out and the pass's responses recorded (MultiRepRecord)
