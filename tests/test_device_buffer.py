@@ -27,6 +27,7 @@ hipError_t hipFree(void* p) {
   return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 }
 int main() {

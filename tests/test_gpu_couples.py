@@ -101,3 +101,37 @@ def test_lists_without_room_for_vertex_ids_match_small_ones():
         print("  ran", flush=True)
     for a, b in zip(*runs):
         np.testing.assert_array_equal(a, b)
+
+
+def test_lists_that_cannot_be_resized_are_empty():
+    """Capacities beyond the device's memory are refused.  The instance that met the limit then runs
+    without lists (without a pair list its pairs are reported as lost) until others are set."""
+    n = 17
+    faces = 2 * (n - 1) ** 2
+    cap = (2 ** 31 - 1) // (9 * faces)
+    k = int(1.3 * free_device_memory() / (8 * 13 * cap * faces)) + 1
+    print(f"case resize of {k} x {8e-9 * 13 * cap * faces:.1f} GB", flush=True)
+    specs = [_crumpled(n, 60 + j, 0.2) for j in range(k)]
+    small = dict(bend_model=1, enable_self_contact=1, ground_height=-1.0, num_substeps=2,
+                 num_iterations=3, pair_capacity_per_face=128)
+    large = dict(small, pair_capacity_per_face=cap, repulsion_vf_items_per_face=3 * cap,
+                 repulsion_ee_items_per_face=9 * cap)
+    s, ids = build_solver(specs, make_params(**small), seed=3)
+    with pytest.raises(XrtError, match="memory"):
+        s.set_params(make_params(**large))
+    print("  refused", flush=True)
+    s.FramesBatched(1)
+    try:
+        s.sync()
+    except XrtError as e:                           # not even its pairs fit
+        assert "overflow" in str(e)
+    s.set_params(make_params(**small))
+    for i, sp in zip(ids, specs):
+        s.SetState(i, sp.x0, np.zeros_like(sp.x0))
+    r, jds = build_solver(specs, make_params(**small), seed=3)
+    for c, cids in ((s, ids), (r, jds)):
+        c.FramesBatched(1)
+        c.sync()
+    for i, j in zip(ids, jds):
+        for u, v in zip(s.GetState(i), r.GetState(j)):
+            np.testing.assert_array_equal(u, v)

@@ -48,10 +48,12 @@ struct DevBuf {
     Free();
     if (count == 0) return hipSuccess;
     const hipError_t e = hipMalloc(reinterpret_cast<void**>(&ptr), count * sizeof(T));
-    if (e == hipSuccess)
+    if (e == hipSuccess) {
       n = count;
-    else
+    } else {
       ptr = nullptr;
+      (void)hipGetLastError();  // else the next launch would report it again
+    }
     return e;
   }
   // The copy has completed when this returns: callers upload from temporaries (set-up

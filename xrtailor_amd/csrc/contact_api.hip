@@ -120,27 +120,29 @@ int AllocPairLists(xrt_ctx* ctx, const HostInstance& h, ContactData& c) {
   const int64_t per_face = std::max(1, ctx->params.pair_capacity_per_face);
   XRT_REQUIRE(per_face * std::max(h.nt, 1) <= static_cast<int64_t>(INT32_MAX), XRT_ERR_INVALID_ARG,
               "pair_capacity_per_face x faces exceeds 2^31 - 1");
-  c.pair_cap = static_cast<int>(std::max<int64_t>(1, per_face * h.nt));
-  XRT_CHECK_HIP(c.pairs.Alloc(c.pair_cap));
-  // repulsion item lists (at most 3 VF and 9 EE items per pair; an instance whose items
-  // overflow a list falls back to the per-pair tests for that half); off when either
-  // capacity is 0 or the counts could overflow an int
-  const int64_t vf_cap = static_cast<int64_t>(std::max(0, ctx->params.repulsion_vf_items_per_face)) * h.nt;
-  const int64_t ee_cap = static_cast<int64_t>(std::max(0, ctx->params.repulsion_ee_items_per_face)) * h.nt;
-  c.vf_cap = c.ee_cap = 0;
+  c.pair_cap = c.vf_cap = c.ee_cap = 0;  // a list that could not be allocated holds nothing
+  c.pairs.Free();
   c.rep_vf.Free();
   c.rep_ee.Free();
   c.ids_vf.Free();
   c.ids_ee.Free();
+  const int64_t pair_cap = std::max<int64_t>(1, per_face * h.nt);
+  XRT_CHECK_HIP(c.pairs.Alloc(pair_cap));
+  c.pair_cap = static_cast<int>(pair_cap);
+  // repulsion item lists (at most 3 VF and 9 EE items per pair; an instance whose items
+  // overflow a list falls back to the per-pair tests for that half); off when either
+  // capacity is 0 or the counts could overflow an int
+  const int64_t vf_cap = std::min(3 * pair_cap, h.nt * int64_t{std::max(0, ctx->params.repulsion_vf_items_per_face)});
+  const int64_t ee_cap = std::min(9 * pair_cap, h.nt * int64_t{std::max(0, ctx->params.repulsion_ee_items_per_face)});
   if (ctx->params.enable_self_contact && vf_cap > 0 && ee_cap > 0 &&
-      9 * static_cast<int64_t>(c.pair_cap) <= static_cast<int64_t>(INT32_MAX)) {
-    c.vf_cap = static_cast<int>(std::min<int64_t>(vf_cap, 3 * static_cast<int64_t>(c.pair_cap)));
-    c.ee_cap = static_cast<int>(std::min<int64_t>(ee_cap, 9 * static_cast<int64_t>(c.pair_cap)));
-    XRT_CHECK_HIP(c.rep_vf.Alloc(c.vf_cap));
-    XRT_CHECK_HIP(c.rep_ee.Alloc(c.ee_cap));
+      9 * pair_cap <= static_cast<int64_t>(INT32_MAX)) {
+    XRT_CHECK_HIP(c.rep_vf.Alloc(vf_cap));
+    XRT_CHECK_HIP(c.rep_ee.Alloc(ee_cap));
     if (!c.ivf.ptr) XRT_CHECK_HIP(c.ivf.Alloc(std::max(h.nt, 1)));
     if (!c.iee.ptr) XRT_CHECK_HIP(c.iee.Alloc(std::max(h.nt, 1)));
     if (!c.nitem.ptr) XRT_CHECK_HIP(c.nitem.Alloc(std::max(h.nt, 1)));
+    c.vf_cap = static_cast<int>(vf_cap);
+    c.ee_cap = static_cast<int>(ee_cap);
   }
   return XRT_OK;
 }
@@ -404,17 +406,6 @@ bool ContactsActive(const xrt_ctx* ctx) {
 }
 
 // device views of every instance's contact state and the block -> instance maps
-int ContactResizeLists(xrt_ctx* ctx) {
-  XRT_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-  for (size_t k = 0; k < ctx->inst.size(); ++k) {
-    if (!ctx->contact[k]) continue;
-    const int rc = AllocPairLists(ctx, ctx->inst[k], *ctx->contact[k]);
-    if (rc != XRT_OK) return rc;
-  }
-  const int rc = MultiContactSetup(ctx);
-  return rc != XRT_OK ? rc : ContactItemIds(ctx);
-}
-
 int CheckPairOverflow(xrt_ctx* ctx) {
   XRT_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   if (!ctx->overflow.ptr) return XRT_OK;
@@ -560,6 +551,18 @@ int MultiContactSetup(xrt_ctx* ctx) {
   return XRT_OK;
 }
 
+// Every instance's lists at the context's capacities.  The device's records follow also when a list
+// could not be allocated: its instance then has no item lists or, if it was the pair list, reports
+// its pairs as lost.
+int ContactResizeLists(xrt_ctx* ctx) {
+  XRT_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  int rc = XRT_OK;
+  for (size_t k = 0; k < ctx->inst.size() && rc == XRT_OK; ++k)
+    if (ctx->contact[k]) rc = AllocPairLists(ctx, ctx->inst[k], *ctx->contact[k]);
+  const int views = ContactItemIds(ctx);
+  return rc != XRT_OK ? rc : views;
+}
+
 // The 16-bit vertex ids of the items (InstContactDev::ids_vf, ids_ee) for the instances whose
 // meshes have no more vertices than that.  They are as large as the lists themselves and the item
 // launches run without them (256 cloths: EE 709 us instead of 426), so they are the last memory
@@ -573,7 +576,7 @@ int ContactItemIds(xrt_ctx* ctx) {
     const HostInstance& h = ctx->inst[k];
     if (!c || c->ee_cap <= 0 || std::max(h.nv, h.obs_nv()) > 1 << 16) continue;
     if (!any) {
-      XRT_CHECK_HIP(hipMemGetInfo(&left, &total));
+      if (hipMemGetInfo(&left, &total) != hipSuccess) break;
       left /= 4;
       any = true;
     }
@@ -582,13 +585,11 @@ int ContactItemIds(xrt_ctx* ctx) {
     if (c->ids_vf.Alloc(c->vf_cap) != hipSuccess || c->ids_ee.Alloc(c->ee_cap) != hipSuccess) {
       c->ids_vf.Free();
       c->ids_ee.Free();
-      (void)hipGetLastError();
       break;
     }
     left -= need;
   }
-  if (!any) return XRT_OK;
-  const std::vector<InstContactDev> ic = ContactViews(ctx);
+  const std::vector<InstContactDev> ic = ContactViews(ctx);  // (no allocation: of the same size)
   XRT_CHECK_HIP(ctx->ic.Upload(ic.data(), ic.size(), ctx->stream));
   return XRT_OK;
 }
