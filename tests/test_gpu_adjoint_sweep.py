@@ -4,6 +4,7 @@ than a sweep holds makes its whole context run per color."""
 import numpy as np
 import pytest
 
+from gpu_helpers import free_device_memory
 from xrtailor_amd import scenes
 from xrtailor_amd.solver import ClothSolver, make_params
 
@@ -58,3 +59,25 @@ def test_sweep_matches_launch_per_color(sides, iters, bending, lra):
     for x, y in zip(a, b):
         np.testing.assert_array_equal(x, y)
     assert any(np.abs(x).max() > 0 for x in a)
+
+
+def test_backward_takes_no_memory():
+    """What the reverse sweep needs is there when AdjointBegin returns (a second context, so that
+    the runtime has taken its own memory for these kernels)."""
+    print("case reverse sweep: memory after AdjointBegin", flush=True)
+    xp = make_params(bend_model=1, ground_height=-0.01, num_substeps=2, num_iterations=2)
+    pos, tris = scenes.grid(400, 1.0)
+    taken = []
+    for _ in range(2):
+        s = ClothSolver(params=xp)
+        i = s.AddCloth(pos, tris, 1e-6, 1e-3)
+        s.Start(3)
+        s.AdjointBegin(1, 1)
+        s.AdjointSeed(i, np.ones_like(pos, dtype=np.float32), None)
+        before = free_device_memory()
+        s.AdjointBackward()
+        s.sync()
+        taken.append(before - free_device_memory())
+        s.close()
+    print("  bytes", taken, flush=True)
+    assert taken[1] == 0

@@ -75,7 +75,6 @@ int AdjSetup(xrt_ctx* c, int want_slots = 1) {
   const size_t N = static_cast<size_t>(A.n_total);
   const bool bend = p.solve_bending != 0, ground = p.enable_ground != 0;
   A.lra = c->total_slots > 0;
-  if (const int prc = PatchPrepareAdj(c); prc != XRT_OK) return prc;
   if (A.lra) {  // slot -> constraints (transpose of the per-target CSR), in constraint order
     std::vector<int32_t> cnt(c->total_slots + 1, 0), sinst(c->total_slots), cons;
     size_t total_k = 0;
@@ -207,7 +206,7 @@ int AdjSetup(xrt_ctx* c, int want_slots = 1) {
     XRT_CHECK_HIP(hipMemsetAsync(A.rep_add.ptr, 0, sizeof(unsigned long long) * 6 * N, c->stream));
     XRT_CHECK_HIP(hipStreamSynchronize(c->stream));
   }
-  return XRT_OK;
+  return PatchPrepareAdj(c);  // (left out where its memory does not fit beside the tape)
 }
 
 int ZeroAdjoints(xrt_ctx* c) {

@@ -567,10 +567,11 @@ int xrt_set_params(xrt_ctx* ctx, const xrt_params* p) {
   if (!ctx->started) return XRT_OK;
   int rc = FemPrepare(ctx);
   if (rc != XRT_OK) return rc;
+  if (lists && (rc = ContactResizeLists(ctx)) != XRT_OK) return rc;
+  if ((rc = ParticleConfigure(ctx)) != XRT_OK) return rc;
   if (!FemOn(ctx) && !ctx->patches.xpbd.tried && (rc = PatchPrepare(ctx)) != XRT_OK) return rc;
   if (!ctx->tuning_set) ctx->tuning.path = DefaultPath(ctx);  // (the model may have changed)
-  if (lists && (rc = ContactResizeLists(ctx)) != XRT_OK) return rc;
-  return ParticleConfigure(ctx);
+  return XRT_OK;
 }
 
 int xrt_get_params(xrt_ctx* ctx, xrt_params* p) {
@@ -886,13 +887,15 @@ int xrt_start(xrt_ctx* ctx, uint64_t seed) {
     XRT_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   }
   ctx->xcur = ctx->x.ptr;
-  int rc = FemOn(ctx) ? XRT_OK : PatchPrepare(ctx);  // (the quality mode's plan: FemPrepare)
+  int rc = ContactStart(ctx);
   if (rc != XRT_OK) return rc;
-  if ((rc = ContactStart(ctx)) != XRT_OK) return rc;
   if ((rc = ParticleStart(ctx)) != XRT_OK) return rc;
   if ((rc = BindingStart(ctx)) != XRT_OK) return rc;
   ctx->fem.seed = seed;
   if ((rc = FemPrepare(ctx)) != XRT_OK) return rc;
+  // what only makes the substep faster comes last and is left out where memory ends (the quality
+  // mode's sweep plan: at the end of FemPrepare)
+  if (!FemOn(ctx) && (rc = PatchPrepare(ctx)) != XRT_OK) return rc;
   if ((rc = ContactItemIds(ctx)) != XRT_OK) return rc;
   if (!ctx->tuning_set) ctx->tuning.path = DefaultPath(ctx);
   ctx->started = true;

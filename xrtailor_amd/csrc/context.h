@@ -240,6 +240,7 @@ struct PatchData {
   DevBuf<int4> bent;
   DevBuf<int2> sent;
   DevBuf<double> glam;
+  DevBuf<double4> gx_alt;  // the reverse sweep writes it, then it and AdjointData::gx change places
   DevBuf<int4> srec, brec, frec, irec;
   DevBuf<int32_t> bcon;
   DevBuf<float4> finv, iK;
@@ -275,7 +276,6 @@ struct AdjointData {
   DevBuf<float4> fstart;  // (x0, v) at each frame start of a segment: [ckpt_every][2][n_total]
   DevBuf<float4> final_state;  // (x0, v) after the recorded frames
   DevBuf<double4> gx0, gv, gx;  // FP64 adjoints
-  DevBuf<double4> gx_alt;       // the reverse sweep writes it, then it and gx change places
   DevBuf<double> glam, gcomp, gbcomp;
   DevBuf<int32_t> ee_cnt;
   // PBD repulsion (self contact): per frame slot a pool of the responses of every repulsion
@@ -440,8 +440,8 @@ bool FemOn(const xrt_ctx* ctx);
 FemConsts FemConstsOf(const xrt_params& p);  // at the substep dt
 int FemPrepare(xrt_ctx* ctx);
 int FemIter(xrt_ctx* ctx, int inst, int it);
-// patch_api.hip: the sweep plans of every instance (PatchPrepare at xrt_start after the
-// colors are uploaded, PatchPrepareFem after the FEM set-up); PatchIter runs one iteration's
+// patch_api.hip: the sweep plans of every instance (PatchPrepare at the end of xrt_start,
+// PatchPrepareFem after the FEM set-up, PatchPrepareAdj after the adjoint's); PatchIter runs one iteration's
 // constraint colors in one launch from xcur (which becomes the other buffer), with the
 // ground plane when `ground`; `it` of `iterations`; tapes as in adjoint.h (XPBD only)
 int PatchPrepare(xrt_ctx* ctx);

@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <new>
 #include <thread>
 
 #include "context.h"
@@ -68,7 +69,7 @@ int Global(int p, int beg) {
 
 // The plan of every instance from its two families; entry0 / entry1 (instance, position with
 // the owner bit, local indices) append one entry's records.  True with D filled (on the
-// host side in `dev`, `verts`, `off`), false when there is no plan.
+// host side in `dev`, `verts`, `off`), false when there is no plan, for want of host memory too.
 struct HostPlan {
   std::vector<PatchDev> dev;
   std::vector<int32_t> verts, off;
@@ -76,7 +77,7 @@ struct HostPlan {
 template <class Families, class Entry0, class Entry1>
 bool MakePlan(xrt_ctx* ctx, int c0, int c1, Families&& families, Entry0&& entry0, Entry1&& entry1,
               PatchPlanDev& D, HostPlan& H, size_t vert_bytes = sizeof(float4),
-              bool hinges_first = false) {
+              bool hinges_first = false) try {
   if (c0 + c1 == 0 || c0 + c1 + 2 > kPatchMaxOffsets) return false;
   const int ni = static_cast<int>(ctx->inst.size());
   const int max_local = static_cast<int>(
@@ -139,6 +140,8 @@ bool MakePlan(xrt_ctx* ctx, int c0, int c1, Families&& families, Entry0&& entry0
   D.lds_bytes = vert_bytes * max_loc;
   D.threads = std::min(1024, std::max(64, (max_color + 63) / 64 * 64));
   return true;
+} catch (const std::bad_alloc&) {
+  return false;
 }
 
 hipError_t UploadPlan(xrt_ctx* ctx, PatchPlanDev& D, const HostPlan& H) {
@@ -313,7 +316,8 @@ int PatchPrepareAdj(xrt_ctx* ctx) {
   if (e == hipSuccess) e = P.bent.Upload(bent, s);
   if (e == hipSuccess) e = P.sent.Upload(sent, s);
   if (e == hipSuccess) e = P.glam.Alloc(std::max<size_t>(sent.size(), 1));
-  return FinishPlan(P.adj, e, ConfigurePatchAdj, P.bent, P.sent, P.glam);
+  if (e == hipSuccess) e = P.gx_alt.Alloc(ctx->x0.n);
+  return FinishPlan(P.adj, e, ConfigurePatchAdj, P.bent, P.sent, P.glam, P.gx_alt);
 }
 
 int PatchAdjIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, bool first,
@@ -321,13 +325,12 @@ int PatchAdjIter(xrt_ctx* ctx, const StepConsts& k, const BendMode& m, bool firs
   PatchData& P = ctx->patches;
   AdjointData& A = *ctx->adj;
   const PatchPlanDev& D = P.adj;
-  if (A.gx_alt.n != A.gx.n) XRT_CHECK_HIP(A.gx_alt.Alloc(A.gx.n));
   const PatchAdjArgs a{D.patch.ptr, D.verts.ptr, D.off.ptr, P.bent.ptr,   P.sent.ptr,
-                       ctx->bpar.ptr, ctx->sc.ptr, ctx->x0.ptr, A.gx.ptr, A.gx_alt.ptr,
+                       ctx->bpar.ptr, ctx->sc.ptr, ctx->x0.ptr, A.gx.ptr, P.gx_alt.ptr,
                        P.glam.ptr,  A.gcomp.ptr, A.gbcomp.ptr, D.n, D.c0, D.c1};
   XRT_CHECK_HIP(LaunchPatchAdj(ctx->stream, a, k.inv_dt2, m, k.solve_bending ? 1 : 0, first ? 1 : 0,
                                tape_b, tape_s, D.threads, D.lds_bytes));
-  std::swap(A.gx.ptr, A.gx_alt.ptr);
+  std::swap(A.gx.ptr, P.gx_alt.ptr);
   return XRT_OK;
 }
 
