@@ -81,8 +81,7 @@ int CheckStarted(xrt_ctx* c, int32_t inst) {
 // instance), free to be written: the copy issued from it two calls earlier has completed
 int StateSlot(xrt_ctx* c, float4** out) {
   SkinStage& st = c->state_stage;
-  size_t need = 0;
-  for (const HostInstance& h : c->inst) need = std::max(need, 8 * static_cast<size_t>(std::max(h.nv, 1)));
+  const size_t need = 8 * static_cast<size_t>(c->max_nv);
   if (st.per < need) {
     st.Release();
     XRT_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&st.host), 2 * need * sizeof(float), 0));
