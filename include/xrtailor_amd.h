@@ -165,6 +165,12 @@ int xrt_sync(xrt_ctx* ctx);
 /* device properties: [0]=compute units, [1]=max LDS bytes per workgroup,
  * [2]=wavefront size, [3]=L2 bytes */
 int xrt_device_info(xrt_ctx* ctx, int64_t info[4]);
+/* patches of the constraint sweeps' plans (every color of an iteration in one launch): [0] the
+ * XPBD constraints', [1] the FEM constraints', [2] the reverse sweep's.  0: no such plan, its
+ * colors run as launches of their own (a mesh without locality, more colors than a sweep holds,
+ * no memory), or it is not built yet ([0], [1]: with the first use of the model, [2]: by
+ * xrt_adjoint_begin).  No counterpart in the reference. */
+int xrt_sweep_patches(xrt_ctx* ctx, int32_t patches[3]);
 
 /* ------------------------------------------------- host-only setup helpers */
 /* These run on the host and need no device; xrt_add_cloth / xrt_start use the same code. */

@@ -40,6 +40,8 @@ def _grad(sides, per_color, xp, lra):
     got = []
     for seed in (1.0, -2.0):                     # the second pass reuses the buffers
         s.AdjointBegin(2, 1)
+        patches, cut = s.sweep_patches()["adjoint"], sum(n * n > 1200 for n in sides)
+        assert patches == 0 if per_color else patches >= len(sides) + cut
         for i, g in zip(ids, seeds):
             s.AdjointSeed(i, seed * g, 0.01 * g)
         s.AdjointBackward()

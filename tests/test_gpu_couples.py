@@ -21,10 +21,13 @@ def _crumpled(n, seed, noise):
 
 
 # noise 3: some hundred pairs a face, more than the 64 couples of a leaf's stage (found again);
-# the capacities: ample, lists too short (pairs stored), pairs lost
-@pytest.mark.parametrize("noise,cap,items", [(0.2, 128, 128), (3.0, 2048, 4096), (3.0, 2048, 60),
-                                             (0.2, 9, 128), (3.0, 100, 64)])
-def test_couples_match_plain(noise, cap, items):
+# the capacities: ample, lists too short (pairs stored), pairs lost.  listed: all instances on
+# the item path
+@pytest.mark.parametrize("noise,cap,items,lost,listed",
+                         [(0.2, 128, 128, False, True), (3.0, 2048, 4096, False, True),
+                          (3.0, 2048, 60, False, False), (0.2, 9, 128, True, False),
+                          (3.0, 100, 64, True, False)])
+def test_couples_match_plain(noise, cap, items, lost, listed):
     print(f"case couples noise={noise} cap={cap} items={items}", flush=True)
     specs = [_crumpled(n, 5 + n, noise) for n in (3, 17, 24)]
     xp = make_params(bend_model=1, enable_self_contact=1, ground_height=-1.0, num_substeps=2,
@@ -33,15 +36,20 @@ def test_couples_match_plain(noise, cap, items):
                      repulsion_vf_items_per_face=items, repulsion_ee_items_per_face=items)
     a, ia = build_solver(specs, xp, seed=3)
     b, ib = build_solver(specs, xp, seed=3)
+    on_items = []
     for _ in range(2):
-        a.SubstepBatched()
+        n = a.time_repulsion(1)[1]                  # a batched substep, and what its lists hold
+        print("  ", n, flush=True)
+        on_items.append(n["item_path_instances"])
         for j in ib:
             b.SubstepPlain(j)
+    assert all(n == len(specs) for n in on_items) if listed else all(n < len(specs) for n in on_items)
     for s in (a, b):
-        try:
+        if lost:                                    # the first pairs were kept
+            with pytest.raises(XrtError, match="overflow"):
+                s.sync()
+        else:
             s.sync()
-        except XrtError as e:                       # capacity: the first pairs were kept
-            print("  ", e, flush=True)
     per_face = []
     for i, j, sp in zip(ia, ib, specs):
         for u, v in zip(a.GetState(i), b.GetState(j)):
@@ -50,6 +58,9 @@ def test_couples_match_plain(noise, cap, items):
         assert ca["pairs"] == cb["pairs"]
         per_face.append(ca["pairs"] / len(sp.tris))
     print("  pairs per face", per_face, flush=True)
+    if noise > 1:  # a face's pair with itself and two for each couple: some leaf has over 64
+        assert max(per_face) > 1 + 2 * 64
+    assert lost == (max(per_face) > cap)
 
 
 # an obstacle of 2^16 vertices (items listed by 16-bit vertex ids) and one of more (by edges)

@@ -21,8 +21,20 @@ def _spec(side, seed, slots=False):
     return scenes.ClothSpec(pos, tris, np.array([0], np.int32), 1e-7, 1e-4, x0, None, sl)
 
 
-def _run(specs, xp, batched, compliance=None, calls=(1, 2)):
+def _check_plan(s, specs, kind):
+    """the plan is there, and an instance of more than 1200 vertices is cut"""
+    patches = s.sweep_patches()[kind]
+    cut = sum(len(sp.pos) > 1200 for sp in specs)
+    assert patches >= len(specs) + cut and (cut or patches == len(specs)), patches
+
+
+def _run(specs, xp, batched, compliance=None, calls=(1, 2), patches=None):
     s, ids = build_solver(specs, xp, seed=3)
+    kind = "fem" if xp.constraint_model else "xpbd"
+    if patches is None:
+        _check_plan(s, specs, kind)
+    else:
+        assert s.sweep_patches()[kind] == patches
     if batched:
         s.set_tuning(1024, 0, 2 if compliance is not None else 1, 1)
     if compliance is not None:
@@ -85,15 +97,16 @@ def test_constraint_model_changed_after_the_start_equals_plain():
     for batched in (True, False):
         got = []
         for models in ((0, 1, 0), (1, 0)):
-            s, ids = build_solver([_spec(40, 1), _spec(27, 2)],
-                                  make_params(bend_model=1, num_iterations=3, num_substeps=2,
-                                              **{**FEM, "constraint_model": models[0]}), seed=2)
+            specs = [_spec(40, 1), _spec(27, 2)]
+            s, ids = build_solver(specs, make_params(bend_model=1, num_iterations=3, num_substeps=2,
+                                                     **{**FEM, "constraint_model": models[0]}), seed=2)
             if batched:
                 s.set_tuning(1024, 0, 1, 1)
             for m in models:
                 p = s.params
                 p.constraint_model = m
                 s.set_params(p)
+                _check_plan(s, specs, "fem" if m else "xpbd")
                 s.FramesBatched(1) if batched else s.FramesPlain(1)
             s.sync()
             got += [a for i in ids for a in s.GetState(i)]
@@ -102,13 +115,15 @@ def test_constraint_model_changed_after_the_start_equals_plain():
     _equal(*runs)
 
 
-def test_mesh_without_locality_equals_plain():
-    """Faces between random vertices: every patch would need nearly every vertex."""
-    print("case sweeps vs plain: a mesh without locality", flush=True)
+@pytest.mark.parametrize("n,faces,patches", [(3000, 2500, 3), (12000, 10000, 0)])
+def test_mesh_without_locality_equals_plain(n, faces, patches):
+    """Faces between random vertices: every patch needs nearly every vertex.  Where a workgroup can
+    hold those, a few patches each solve nearly all constraints; else the colors run as launches
+    of their own."""
+    print(f"case sweeps vs plain: a mesh without locality, {n} vertices", flush=True)
     rng = np.random.RandomState(1)
-    n = 3000
-    tris = np.array([rng.choice(n, 3, replace=False) for _ in range(2500)], np.int32)
+    tris = np.array([rng.choice(n, 3, replace=False) for _ in range(faces)], np.int32)
     pos = rng.rand(n, 3)
     spec = scenes.ClothSpec(pos, tris, np.zeros(0, np.int32), 1e-4, 1e-2, pos.astype(np.float32))
     xp = make_params(bend_model=1, num_iterations=2, num_substeps=2, ground_height=-5.0)
-    _equal(_run([spec], xp, True), _run([spec], xp, False))
+    _equal(_run([spec], xp, True, patches=patches), _run([spec], xp, False, patches=patches))

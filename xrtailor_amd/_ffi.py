@@ -100,6 +100,7 @@ SIGNATURES = {
     "xrt_get_params": [_P, C.POINTER(XrtParams)],
     "xrt_sync": [_P],
     "xrt_device_info": [_P, C.POINTER(C.c_int64)],
+    "xrt_sweep_patches": [_P, _IP],
     "xrt_build_edges": [_IP, _I, _IP, _I, _IP],
     "xrt_build_bends": [_IP, _I, _IP, _I, _IP, _I, _IP],
     "xrt_color_constraints": [_IP, _I, _I, _I, C.c_uint64, _I, _IP, _IP],

@@ -593,6 +593,13 @@ int xrt_device_info(xrt_ctx* ctx, int64_t info[4]) {
   return XRT_OK;
 }
 
+int xrt_sweep_patches(xrt_ctx* ctx, int32_t patches[3]) {
+  XRT_REQUIRE(ctx && ctx->started && patches, XRT_ERR_INVALID_ARG, "null argument or not started");
+  const PatchPlanDev* plans[3] = {&ctx->patches.xpbd, &ctx->patches.fem, &ctx->patches.adj};
+  for (int k = 0; k < 3; ++k) patches[k] = plans[k]->ready ? plans[k]->n : 0;
+  return XRT_OK;
+}
+
 int xrt_build_edges(const int32_t* tris, int32_t nt, int32_t* edges_out, int32_t max_edges,
                     int32_t* ne_out) {
   XRT_REQUIRE(tris && nt >= 0 && ne_out, XRT_ERR_INVALID_ARG, "null argument");

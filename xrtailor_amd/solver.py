@@ -561,6 +561,12 @@ class ClothSolver:
                            0)
         check(self.lib.xrt_set_tuning(self.ctx, C.byref(t)))
 
+    def sweep_patches(self) -> dict:
+        """Patches of the constraint sweeps' plans; 0: no plan, one launch per color."""
+        p = np.zeros(3, np.int32)
+        check(self.lib.xrt_sweep_patches(self.ctx, iptr(p)))
+        return dict(xpbd=int(p[0]), fem=int(p[1]), adjoint=int(p[2]))
+
     def time_batched_substep(self, n: int) -> float:
         ms = C.c_float()
         check(self.lib.xrt_time_batched_substep(self.ctx, n, C.byref(ms)))
