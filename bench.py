@@ -13,11 +13,12 @@ value        batched vertex-substeps/s (one hipGraph per frame; every contact ph
 plain_value  the same workload one instance at a time through per-instance launches
 roofline     dominant kernel, per-launch device time from HIP events on the solver stream:
              with contacts the EE repulsion item kernel, algorithmic bytes per launch
-             = 8 (EE items) + 16 N + 8 E (items, positions, edges read once); without
-             contacts the persistent substep kernel (or the wide substep's launches
-             together), sum_i (64 N_i + 16 E_i + 24 B_i + 12 K_i); HBM peak 8 TB/s.  traffic: HBM bytes per launch from the committed
-             rocprofv3 FETCH_SIZE / WRITE_SIZE summary of that kernel (profiles/traffic.json),
-             null when absent
+             = 8 (EE items) + 16 N (each item's four vertex ids and the positions read
+             once; + 8 E where a mesh has more than 65,536 vertices and its items name edges);
+             without contacts the persistent substep kernel (or the wide substep's launches
+             together), sum_i (64 N_i + 16 E_i + 24 B_i + 12 K_i); HBM peak 8 TB/s.
+             traffic: HBM bytes per launch from the committed rocprofv3 FETCH_SIZE /
+             WRITE_SIZE summary of that kernel (profiles/traffic.json), null when absent
 cpu_baseline the serial FP64 oracle on one core, one substep per instance over a bounded
              sample; the same leg reports the single-substep relative error of the GPU's
              batched substep against it (parity at the measured configuration)
@@ -32,11 +33,10 @@ cpu_baseline the serial FP64 oracle on one core, one substep per instance over a
                      quality mode's FEM constraints (Green strain over faces with moduli
                      1e3, 1e3, 4e2 and Poisson ratios 0.3, isometric bending stiffness 1e-2
                      over hinges) in place of the XPBD stretch and bend; roofline kernel
-                     WideStrainKernel, algorithmic bytes
-                     per launch 128 per face of the color (32 B element, three float4
-                     vertices read and written), the isometric bending launches beside it
-                     at 172 B per hinge; with --no-contacts the persistent kernel, 64 N +
-                     32 F + 44 hinges + 12 K per launch)
+                     the EE repulsion kernel, as for the batched workload; with
+                     --no-contacts the substep, 64 N + 32 F + 44 hinges + 12 K.  `fem` times
+                     the launches of one color each, which a frame runs only for meshes
+                     without a sweep plan)
                     (garment: 64 tube garments on capsule-chain bodies skinned on the GPU
                      every frame (LBS from joint transforms), bindings at the top ring and
                      waist, LRA, body contact; a step is the skinning plus one frame, timed
@@ -509,44 +509,43 @@ def main() -> int:
         # bracketed by unrecorded frames just before and after (the cost per frame changes
         # as the simulation advances)
         solver.RecordFrames(1, normals=True)
-        before = solver.time_frames(True, a.steps)
+        ms0 = solver.time_frames(True, a.steps)
         t1 = time.perf_counter()
         solver.RecordFrames(a.steps, normals=True)
         rms = (time.perf_counter() - t1) * 1e3
-        after = solver.time_frames(True, a.steps)
-        base = 0.5 * (before + after)
-        record = {"ms_per_frame": rms / a.steps, "frame_ms_before": before / a.steps,
-                  "frame_ms_after": after / a.steps, "overhead": rms / base - 1.0,
+        ms1 = solver.time_frames(True, a.steps)
+        base = 0.5 * (ms0 + ms1)
+        record = {"ms_per_frame": rms / a.steps, "frame_ms_before": ms0 / a.steps,
+                  "frame_ms_after": ms1 / a.steps, "overhead": rms / base - 1.0,
                   "bytes_per_frame": 24 * n_verts,
                   "d2h_gbs": 24 * n_verts * a.steps / (rms * 1e-3) / 1e9}
-        print(f"[bench] recorded frames {rms / a.steps:.1f} ms/frame vs {before / a.steps:.1f} "
-              f"before and {after / a.steps:.1f} after", file=sys.stderr, flush=True)
+        print(f"[bench] recorded frames {rms / a.steps:.1f} ms/frame vs {ms0 / a.steps:.1f} "
+              f"before and {ms1 / a.steps:.1f} after", file=sys.stderr, flush=True)
 
     # dominant kernel: per-launch device time from HIP events around each launch
     rep_counts, particle, binding, fem = None, None, None, None
     if quality:
-        kernel = "WideStrainKernel"
+        # one color of every instance per launch, averaged over the colors: a face's element
+        # (32 B) read, three vertices read and written (96 B); a hinge's indices (16 B), weights
+        # K (16 B), coeff (4 B), multiplier read and written (8 B), four vertices read and
+        # written (128 B)
         strain_ms, iso_ms = solver.time_fem(2 * params.num_iterations)
         faces = sum(solver.counts(i).nt for i in insts)
         hinges = sum(solver.counts(i).n_bends for i in insts)
         f_launch = max(solver.fem(i)["n_colors"] for i in insts)
         b_launch = max(solver.counts(i).bend_colors for i in insts)
-        kern_ms = strain_ms
-        # one face color of every instance per launch: element (32 B) read, three vertices
-        # read and written (96 B), averaged over the colors
-        bytes_kern = 128 * faces / f_launch
-        # hinge: indices (16 B), weights K (16 B), coeff (4 B), multiplier read and written
-        # (8 B), four vertices read and written (128 B)
-        fem = {"strain_ms": strain_ms, "strain_launches_per_pass": f_launch, "faces": faces,
+        fem = {"sweep_patches": solver.sweep_patches()["fem"],
+               "strain_ms": strain_ms, "strain_launches_per_pass": f_launch, "faces": faces,
+               "strain_gbs": 128 * faces / f_launch / (strain_ms * 1e-3) / 1e9,
                "iso_bend_ms": iso_ms, "iso_bend_launches_per_pass": b_launch, "hinges": hinges,
                "iso_bend_gbs": 172 * hinges / b_launch / (iso_ms * 1e-3) / 1e9}
-        if not contacts:
-            # the frame is the persistent kernel: state read + written (64 B per vertex),
-            # strain elements 32 B, isometric data 44 B per hinge, LRA 12 B, read once
-            kernel = substep_kernel_name(solver)
-            kern_ms = solver.time_batched_substep(max(10, a.steps))
-            lra = sum(solver.counts(i).lra_constraints for i in insts)
-            bytes_kern = 64 * n_verts + 32 * faces + 44 * hinges + 12 * lra
+    if quality and not contacts:
+        # state read + written (64 B per vertex), strain elements 32 B, isometric data 44 B per
+        # hinge, LRA 12 B, read once
+        kernel = substep_kernel_name(solver)
+        kern_ms = solver.time_batched_substep(max(10, a.steps))
+        lra = sum(solver.counts(i).lra_constraints for i in insts)
+        bytes_kern = 64 * n_verts + 32 * faces + 44 * hinges + 12 * lra
     elif a.workload == "garment":
         kernel = "LbsKernel"
         kern_ms, bind_ms = solver.time_binding(20)
@@ -572,8 +571,9 @@ def main() -> int:
     elif contacts:
         kernel = "MultiRepItemKernel<1>"
         kern_ms, rep_counts = solver.time_repulsion(params.num_substeps)  # a whole frame
-        n_edges = sum(solver.counts(i).n_edges for i in insts)
-        bytes_kern = 8 * rep_counts["ee_items"] + 16 * n_verts + 8 * n_edges
+        by_edges = [solver.counts(i).n_edges for i, sp in zip(insts, specs)
+                    if max(len(sp.pos), len(sp.obstacle[0]) if sp.obstacle else 0) > 65536]
+        bytes_kern = 8 * rep_counts["ee_items"] + 16 * n_verts + 8 * sum(by_edges)
     else:
         kernel = substep_kernel_name(solver)
         kern_ms = solver.time_batched_substep(max(10, a.steps))
