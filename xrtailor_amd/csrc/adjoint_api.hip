@@ -274,7 +274,7 @@ int WideSubstep(xrt_ctx* c, const StepConsts& k, const BendMode& bm, AdjointData
   for (int i = 0; i < n_inst; ++i) obs_contact = obs_contact || ObsContact(c, i);
   // the vertex-face solves end the sweep when every patch has a CU (one launch of 4.5 us and its
   // gap less an iteration, 1.6 us more sweep); with more patches than CUs their loads, at a few
-  // waves a CU, cost more than the launch (256 cloths: 344 us against 295 + 18)
+  // waves a CU, cost more than the launch (256 cloths, half-size workgroups: 344 us against 295 + 18)
   const bool sweep_vf =
       sweep && obs_contact && c->total_slots == 0 && PatchPlanOf(c).n <= c->cu_count;
   int rc;

@@ -889,7 +889,9 @@ __global__ __launch_bounds__(1024) void MultiObsMergeTopKernel(const InstContact
 // the first `edge_grid` blocks, then each vertex's point query, then its segment query
 // (vert_grid blocks each).  A query is a chain of dependent node loads (85 us for the edges of 8
 // cloths, 55 us for both of the vertices, with most of the chip idle), so the three run side by
-// side in one launch: together as long as the edges alone.
+// side in one launch: together as long as the edges alone.  Where the chip is full nothing is lost:
+// 256 cloths take 670 us against 457 + 207 in two launches (edges; both queries of a vertex in one
+// thread), 32 cloths 91 against 89 + 62.
 __global__ __launch_bounds__(kBlock) void MultiGenerateKernel(const InstContactDev* ic,
                                                               const int32_t* off_e,
                                                               const int32_t* off_v, int n,
@@ -1414,11 +1416,13 @@ __global__ __launch_bounds__(kBlock) void MultiAddTotalsKernel(const InstContact
 // MultiRepPairsKernel.  A wave takes 64 items per step; the few that are left open are queued
 // in LDS and evaluated 64 at a time (and at the end), so that the long evaluation does not run
 // in every step for one or two lanes.  The sums are fixed point: the order changes nothing.
-// Bound by the L1 lookups of the gathers (33 a load instruction, one a cycle: busy for 83 % of the
-// launch), so an item comes as the 16-bit ids of its vertices where the meshes are small enough:
-// four gathers, without the edges' or the face's.  63 M EE and 31 M VF items of 256 cloths: 709 ->
-// 426 and 228 -> 173 us (with the sharper EeReject and the longer blocks that MultiContactSetup
-// chooses).  Six waves a SIMD for EE, eight for VF: five 473 / 183, six 425 / 183, eight 437 / 173.
+// With six gathers an item it was bound by their L1 lookups (33 a load instruction, one a cycle:
+// busy for 83 % of the launch), so an item comes as the 16-bit ids of its vertices where the meshes
+// are small enough: four gathers, without the edges' or the face's.  63 M EE and 31 M VF items of 256
+// landing cloths: 709 -> 426 and 228 -> 173 us (with the sharper EeReject and the longer blocks that
+// MultiContactSetup chooses).  On settled cloths (77 M EE items, 620 us) lookups take 62 % of the
+// launch now and the vector ALUs 66 %.  Six waves a SIMD for EE, eight for VF: five 473 / 183, six
+// 425 / 183, eight 437 / 173.
 template <int is_ee>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(is_ee ? 6 : 8))) void
 MultiRepItemKernel(const InstContactDev* ic, const int32_t* off, int n,
