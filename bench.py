@@ -91,9 +91,8 @@ def measured_traffic(kernel: str, workload: str, algorithmic: float):
     for r in rec.get("kernels", []):
         if r.get("kernel") == kernel and r.get("workload") == workload:
             alg = r.get("algorithmic_bytes_per_launch")
-            if not alg or abs(alg - algorithmic) > 0.02 * algorithmic:
-                return None
-            return r.get("bytes_per_launch")
+            if alg and abs(alg - algorithmic) <= 0.02 * algorithmic:
+                return r.get("bytes_per_launch")
     return None
 
 
